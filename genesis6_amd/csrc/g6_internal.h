@@ -113,6 +113,7 @@ struct MdBuf {
   int cell_cap;
   int *nbr_j, *nbr_code, *nbr_cnt;
   int maxnb;
+  int scan;  // rows from a scan of every molecule instead of the cell lists
   double *frc;        // [6][n] force and torque (lab) of the last k_md_main
   double *blockpart;  // [2][nblk][16] k_md_main block partials, by parity
   double *blockek;    // [k_md_pre waves][kEkLen] kinetic partials
@@ -349,9 +350,11 @@ struct CloseArgs {
 // a row is rebuilt, then the compacted interacting entries (index and the
 // COM separation in the pair precision), then the lane partials of the
 // energy and virial.
+// words of the row sort's bit window (g6_md.hip)
+constexpr int kRowWords = 128;
 inline int main_region_bytes(int maxnb, int rsize) {
   auto up16 = [](int x) { return (x + 15) / 16 * 16; };
-  const int sort = 8 * maxnb;
+  const int sort = 8 * maxnb + 8 * kRowWords;
   const int comp = up16(4 * maxnb) + 3 * up16(rsize * maxnb);
   const int acc = 10 * 64 * 8;
   const int mx = sort > comp ? sort : comp;

@@ -344,27 +344,29 @@ __device__ __forceinline__ void md_pre_body(const ModelTable &mt, const Geom &g,
       rec[0] = S[0];
       rec[1] = S[1];
       rec[2] = S[2];
-      int jc[3], nd[3];
-      grid_nd<BOX>(g, nd);
-#pragma unroll
-      for (int a = 0; a < 3; a++) {
-        double d = S[a];
-        const double o = round(d * bx.invL[a]) * bx.L[a];
-        d = d - o;
-        int j = (int)round(d * bx.cellinv[a]);
-        if (j < 0) j += nd[a];
-        j = ((j % nd[a]) + nd[a]) % nd[a];
-        jc[a] = j;
+      if (!b.scan) {
+        int jc[3], nd[3];
+        grid_nd<BOX>(g, nd);
+  #pragma unroll
+        for (int a = 0; a < 3; a++) {
+          double d = S[a];
+          const double o = round(d * bx.invL[a]) * bx.L[a];
+          d = d - o;
+          int j = (int)round(d * bx.cellinv[a]);
+          if (j < 0) j += nd[a];
+          j = ((j % nd[a]) + nd[a]) % nd[a];
+          jc[a] = j;
+        }
+        const int c = (jc[2] * nd[1] + jc[1]) * nd[0] + jc[0];
+        b.cell[i] = c;
+        // slot 0 of a cell row is its count; residents follow
+        int *cr = b.cellres + ((size_t)parity * g.ncell + c) * b.cell_cap;
+        const int slot = atomicAdd(cr, 1) + 1;
+        if (slot < b.cell_cap)
+          cr[slot] = i;
+        else
+          raise_flag(b.flags, 3);  // cell capacity exceeded
       }
-      const int c = (jc[2] * nd[1] + jc[1]) * nd[0] + jc[0];
-      b.cell[i] = c;
-      // slot 0 of a cell row is its count; residents follow
-      int *cr = b.cellres + ((size_t)parity * g.ncell + c) * b.cell_cap;
-      const int slot = atomicAdd(cr, 1) + 1;
-      if (slot < b.cell_cap)
-        cr[slot] = i;
-      else
-        raise_flag(b.flags, 3);  // cell capacity exceeded
       if (b.half_skin2 > 0.0) {
         // a pair of the rows moves by at most twice the largest displacement
         // plus |L - L_ref| (image shifts of one box per axis)
@@ -522,23 +524,87 @@ __device__ inline double frac_in_cell(const BoxNow &bx, double x, int a) {
   return t - round(t);
 }
 
-// neighbour-row build of molecule i into nbr[i*maxnb ...], sorted by j so
-// that the force sums do not depend on the order in which the binning
-// atomics filled the cells; returns the row length (also stored).
+// The FP64 minimum-image test of Interaction_Compress2 at rc + skin for one
+// candidate: whether j is in i's row, and its image shift code.
+__device__ inline bool row_test(const BoxNow &bx, const MdBuf &b, double rr, double d0, double d1,
+                                double d2, int &code) {
+  const double k0 = round(d0 * bx.invL[0]), k1 = round(d1 * bx.invL[1]),
+               k2 = round(d2 * bx.invL[2]);
+  d0 = d0 - k0 * bx.L[0];
+  d1 = d1 - k1 * bx.L[1];
+  d2 = d2 - k2 * bx.L[2];
+  const double dd = d0 * d0 + d1 * d1 + d2 * d2;
+  const bool pass = dd < rr;
+  code = ((int)k0 + 512) | (((int)k1 + 512) << 10) | (((int)k2 + 512) << 20);
+  if (pass && (fabs(k0) > 511.0 || fabs(k1) > 511.0 || fabs(k2) > 511.0)) raise_flag(b.flags, 2);
+  return pass;
+}
+
+// Row of molecule i from a scan of every molecule in index order: the row
+// comes out sorted, with no cell lists.  Four candidates per lane are loaded
+// together (the COM components are read from the arrays the predictor wrote,
+// which are contiguous in j), so the cost is n / 64 tests per lane and no
+// latency of cell counts, search and sort.  Taken up to kScanMax molecules.
 template <int BOX>
-__device__ inline int build_row(const Geom &g, const MdBuf &b, int parity, int i, int lane,
-                                int (&s_beg)[128], int (&s_pre)[132], int *s_j, int *s_c) {
-  constexpr bool NPT = BOX == kBoxBaro;
+__device__ inline int scan_row(const Geom &g, const MdBuf &b, int i, int lane, double xi, double yi,
+                               double zi, int *nj, int *nc) {
+  const BoxNow bx = box_now<BOX>(g, b);
+  const int n = g.n, cap = b.maxnb;
+  const unsigned long long lt = (1ull << lane) - 1ull;
+  int base = 0;
+  for (int j0 = 0; j0 < n; j0 += 256) {
+    double x[4], y[4], z[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const int j = min(j0 + 64 * u + lane, n - 1);
+      x[u] = b.com[j];
+      y[u] = b.com[n + j];
+      z[u] = b.com[2 * n + j];
+    }
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const int j = j0 + 64 * u + lane;
+      int code = 0;
+      const bool pass =
+          j < n && j != i && row_test(bx, b, g.rr, xi - x[u], yi - y[u], zi - z[u], code);
+      const unsigned long long mask = __ballot(pass);
+      const int pos = base + __popcll(mask & lt);
+      if (pass) {
+        if (pos < cap) {
+          nj[pos] = j;
+          nc[pos] = code;
+        } else {
+          raise_flag(b.flags, 4);  // neighbour-row capacity exceeded
+        }
+      }
+      base += __popcll(mask);
+    }
+  }
+  return min(base, cap);
+}
+
+// Row of molecule i from the cell lists, sorted by j so that the force sums
+// do not depend on the order in which the binning atomics filled the cells.
+// The sort places every entry at the number of smaller j in the row: a bit
+// per molecule index in LDS (a window of 32 * kRowWords indices at a time),
+// the words' running counts, and the bits below j in its word.  (Counting the
+// smaller entries of the row per entry was 3 passes of 176 LDS reads at 4096
+// molecules, skin 1.8 A, twice the instructions of a step without a build.)
+template <int BOX>
+__device__ inline int cell_row(const Geom &g, const MdBuf &b, int parity, int i, int lane,
+                               double xi, double yi, double zi, int (&s_beg)[128],
+                               int (&s_pre)[132], int *s_j, int *nj, int *nc) {
   const BoxNow bx = box_now<BOX>(g, b);
   const int n = g.n;
+  int *s_c = s_j + b.maxnb;
+  unsigned *s_bit = reinterpret_cast<unsigned *>(s_c + b.maxnb);
+  int *s_cnt = reinterpret_cast<int *>(s_bit + kRowWords);
   int nd[3];
   grid_nd<BOX>(g, nd);
   const int nx = nd[0], ny = nd[1], nz = nd[2];
   const int c = b.cell[i];
   const int cx = c % nx, cy = (c / nx) % ny, cz = c / (nx * ny);
   const Stencil st = stencil_of(nd);
-  const double *reci = b.rec + (size_t)i * b.rs;
-  const double xi = reci[0], yi = reci[1], zi = reci[2];
   const double ux = frac_in_cell(bx, xi, 0), uy = frac_in_cell(bx, yi, 1),
                uz = frac_in_cell(bx, zi, 2);
   const int *res = b.cellres + (size_t)parity * g.ncell * b.cell_cap;
@@ -592,16 +658,7 @@ __device__ inline int build_row(const Geom &g, const MdBuf &b, int parity, int i
       j = res[s_beg[lo] + (t - s_pre[lo])];
       if (j != i) {
         const double *recj = b.rec + (size_t)j * b.rs;
-        double d0 = xi - recj[0], d1 = yi - recj[1], d2 = zi - recj[2];
-        const double k0 = round(d0 * bx.invL[0]), k1 = round(d1 * bx.invL[1]),
-                     k2 = round(d2 * bx.invL[2]);
-        d0 = d0 - k0 * bx.L[0];
-        d1 = d1 - k1 * bx.L[1];
-        d2 = d2 - k2 * bx.L[2];
-        const double dd = d0 * d0 + d1 * d1 + d2 * d2;
-        pass = dd < g.rr;
-        code = ((int)k0 + 512) | (((int)k1 + 512) << 10) | (((int)k2 + 512) << 20);
-        if (pass && (fabs(k0) > 511.0 || fabs(k1) > 511.0 || fabs(k2) > 511.0)) raise_flag(b.flags, 2);
+        pass = row_test(bx, b, g.rr, xi - recj[0], yi - recj[1], zi - recj[2], code);
       }
     }
     const unsigned long long mask = __ballot(pass);
@@ -618,16 +675,66 @@ __device__ inline int build_row(const Geom &g, const MdBuf &b, int parity, int i
   }
   wsync();
   const int m = min(base, cap);
-  // rank sort by j (each j occurs once in a row)
-  int *nj = b.nbr_j + (size_t)i * cap;
-  int *nc = b.nbr_code + (size_t)i * cap;
-  for (int t = lane; t < m; t += 64) {
-    const int key = s_j[t];
-    int rank = 0;
-    for (int u = 0; u < m; u++) rank += s_j[u] < key;
-    nj[rank] = key;
-    nc[rank] = s_c[t];
+  // windows of the index range: the bits of the entries, the running counts
+  // of the words (two words per lane of the wave), the entries' places
+  int below = 0;
+  for (int w0 = 0; w0 < n; w0 += 32 * kRowWords) {
+#pragma unroll
+    for (int u = 0; u < kRowWords / 64; u++) s_bit[64 * u + lane] = 0u;
+    wsync();
+    for (int t = lane; t < m; t += 64) {
+      const unsigned q = (unsigned)(s_j[t] - w0);
+      if (q < 32u * kRowWords) atomicOr(&s_bit[q >> 5], 1u << (q & 31));
+    }
+    wsync();
+    int cnt[kRowWords / 64], sum = 0;
+#pragma unroll
+    for (int u = 0; u < kRowWords / 64; u++) {
+      cnt[u] = __popc(s_bit[lane * (kRowWords / 64) + u]);
+      sum += cnt[u];
+    }
+    int inc = sum;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int v = __shfl_up(inc, d, 64);
+      if (lane >= d) inc += v;
+    }
+    int run = below + inc - sum;
+#pragma unroll
+    for (int u = 0; u < kRowWords / 64; u++) {
+      s_cnt[lane * (kRowWords / 64) + u] = run;
+      run += cnt[u];
+    }
+    below += __shfl(inc, 63, 64);
+    wsync();
+    for (int t = lane; t < m; t += 64) {
+      const int key = s_j[t];
+      const unsigned q = (unsigned)(key - w0);
+      if (q < 32u * kRowWords) {
+        const int rank = s_cnt[q >> 5] + __popc(s_bit[q >> 5] & ((1u << (q & 31)) - 1u));
+        nj[rank] = key;
+        nc[rank] = s_c[t];
+      }
+    }
+    wsync();
   }
+  return m;
+}
+
+// neighbour-row build of molecule i into nbr[i*maxnb ...], in the order of
+// j; returns the row length (also stored).
+template <int BOX>
+__device__ inline int build_row(const Geom &g, const MdBuf &b, int parity, int i, int lane,
+                                int (&s_beg)[128], int (&s_pre)[132], int *s_sort) {
+  constexpr bool NPT = BOX == kBoxBaro;
+  const int n = g.n;
+  const double *reci = b.rec + (size_t)i * b.rs;
+  const double xi = reci[0], yi = reci[1], zi = reci[2];
+  int *nj = b.nbr_j + (size_t)i * b.maxnb;
+  int *nc = b.nbr_code + (size_t)i * b.maxnb;
+  const int m = b.scan ? scan_row<BOX>(g, b, i, lane, xi, yi, zi, nj, nc)
+                       : cell_row<BOX>(g, b, parity, i, lane, xi, yi, zi, s_beg, s_pre, s_sort, nj,
+                                       nc);
   wsync();  // the force loop reads entries other lanes wrote
   if (lane == 0) {
     b.nbr_cnt[i] = m;
@@ -635,6 +742,7 @@ __device__ inline int build_row(const Geom &g, const MdBuf &b, int parity, int i
     b.com_ref[n + i] = yi;
     b.com_ref[2 * n + i] = zi;
     if (NPT && i == 0) {  // the box the rows were built in
+      const BoxNow bx = box_now<BOX>(g, b);
       b.box[9] = bx.L[0];
       b.box[10] = bx.L[1];
       b.box[11] = bx.L[2];
@@ -671,8 +779,8 @@ __device__ __forceinline__ void md_main_body(const ModelTable &mt, const Geom &g
     int jj[4], cc[4];
     int m;
     if (b.flags[2 + parity]) {
-      int *sj = reinterpret_cast<int *>(reg);
-      m = build_row<BOX>(g, b, parity, i, lane, s_beg[wid], s_pre[wid], sj, sj + cap);
+      m = build_row<BOX>(g, b, parity, i, lane, s_beg[wid], s_pre[wid],
+                         reinterpret_cast<int *>(reg));
       nlist = m;
     } else {
       m = b.nbr_cnt[i];
