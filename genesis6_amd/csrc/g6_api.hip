@@ -409,6 +409,8 @@ static int env_int(const char *name, int dflt) {
   return e ? atoi(e) : dflt;
 }
 
+int step_max(int prec) { return env_int("G6_STEP_MAX", prec == G6_FP32 ? kStepMaxF : kStepMaxD); }
+
 // Rows are built from a scan of every molecule up to kScanMax molecules, from
 // the cell lists beyond.  Measured per step, cells against scan, TIP4P, FP64
 // rows rebuilt every step: 216 molecules 19.6 / 13.9 us, 1000 22.8 / 18.1,
@@ -438,6 +440,7 @@ static void set_row_grid(System &s) {
   // line
   s.md.scan = s.n <= env_int("G6_SCAN_MAX", kScanMax) && !(cc > 1);
   s.nblk_md = (s.n + 3) / 4;
+  s.one_kernel = s.n <= step_max(s.prec);
   s.md.part = nullptr;
   s.tiles = false;
 }
@@ -541,13 +544,14 @@ static int alloc_all(System &s) {
   auto A = [](void **p, size_t b) { return hipMalloc(p, b > 0 ? b : 8); };
 #define AL(ptr, bytes) G6_CHECK(A((void **)&(ptr), (bytes)))
   MdBuf &m = s.md;
-  AL(m.com, sizeof(double) * 3 * n);
-  AL(m.dx, sizeof(double) * 15 * n);
-  AL(m.w, sizeof(double) * 15 * n);
-  AL(m.quat, sizeof(double) * 20 * n);
+  AL(m.com, sizeof(double) * kStateRows * n);
+  m.dx = m.com + 3 * (size_t)n;
+  m.w = m.com + kRowW * (size_t)n;
+  m.quat = m.com + kRowQ * (size_t)n;
+  m.com_ref = m.com + kRowRef * (size_t)n;
   AL(m.tmat, sizeof(double) * 9 * n);
-  AL(m.rec, sizeof(double) * (size_t)m.rs * n);
-  AL(m.com_ref, sizeof(double) * 3 * n);
+  AL(m.rec, sizeof(double) * 2 * (size_t)m.rs * n);
+  AL(m.comp, sizeof(double) * 6 * n);
   AL(m.cell, sizeof(int) * n);
   // cell lists sized for the row grid and, when the system qualifies, the tile grid
   size_t ncap = (size_t)ncm * m.cell_cap;
@@ -555,7 +559,7 @@ static int alloc_all(System &s) {
     const size_t nt = (size_t)s.tile_ndiv * s.tile_ndiv * s.tile_ndiv * s.tile_cap;
     if (nt > ncap) ncap = nt;
   }
-  AL(m.cellres, sizeof(int) * 2 * ncap);
+  AL(m.cellres, sizeof(int) * 3 * ncap);
   AL(m.nbr_j, sizeof(int) * (size_t)n * m.maxnb);
   AL(m.nbr_code, sizeof(int) * (size_t)n * m.maxnb);
   AL(m.nbr_cnt, sizeof(int) * n);
@@ -567,9 +571,10 @@ static int alloc_all(System &s) {
     }
     AL(m.blockpart, sizeof(double) * 2 * kBP * nb);
   }
-  AL(m.blockek, sizeof(double) * kEkLen * (size_t)pre_waves(n));
+  AL(m.stepek, sizeof(double) * 2 * kEkLen * (size_t)((n + 3) / 4));
+  AL(m.stepkin, sizeof(double) * 2 * (size_t)((n + 3) / 4));
   AL(m.frc, sizeof(double) * 6 * n);
-  AL(m.nose, sizeof(double) * 9);
+  AL(m.nose, sizeof(double) * 18);
   AL(m.thermo, sizeof(double) * G6_THERMO_LEN);
   AL(m.flags, sizeof(int) * 8);
   s.nose = m.nose;
@@ -590,13 +595,9 @@ static int alloc_all(System &s) {
   AL(s.com_ref, sizeof(double) * 3 * n);
   AL(s.lflags, sizeof(int) * 8);
 #undef AL
-  G6_CHECK(hipMemset(m.com, 0, sizeof(double) * 3 * n));
-  G6_CHECK(hipMemset(m.dx, 0, sizeof(double) * 15 * n));
-  G6_CHECK(hipMemset(m.w, 0, sizeof(double) * 15 * n));
-  G6_CHECK(hipMemset(m.quat, 0, sizeof(double) * 20 * n));
+  G6_CHECK(hipMemset(m.com, 0, sizeof(double) * kStateRows * n));
   G6_CHECK(hipMemset(m.nbr_cnt, 0, sizeof(int) * n));
-  G6_CHECK(hipMemset(m.com_ref, 0, sizeof(double) * 3 * n));
-  G6_CHECK(hipMemset(m.nose, 0, sizeof(double) * 9));
+  G6_CHECK(hipMemset(m.nose, 0, sizeof(double) * 18));
   G6_CHECK(hipMemset(m.thermo, 0, sizeof(double) * G6_THERMO_LEN));
   return 0;
 }
@@ -620,9 +621,9 @@ static int tile_alloc(System &s) {
 
 // neighbour rows and cell lists ready for a fresh first step
 static int reset_step_state(System &s) {
-  int fl[8] = {0, 0, 1, 1, 0, 0, 0, 0};
+  int fl[8] = {0, 0, 1, 1, 1, 0, 0, 0};
   G6_CHECK(hipMemcpy(s.md.flags, fl, sizeof(fl), hipMemcpyHostToDevice));
-  G6_CHECK(hipMemset(s.md.cellres, 0, sizeof(int) * 2 * (size_t)s.geo_md.ncell * s.md.cell_cap));
+  G6_CHECK(hipMemset(s.md.cellres, 0, sizeof(int) * 3 * (size_t)s.geo_md.ncell * s.md.cell_cap));
   return 0;
 }
 
@@ -670,9 +671,9 @@ int use_row_grid(System &s) {
 
 static void free_all(System &s) {
   const MdBuf &m = s.md;
-  void *ps[] = {m.com, m.dx, m.w, m.quat, m.tmat, m.rec, m.com_ref,
+  void *ps[] = {m.com, m.tmat, m.rec, m.comp, m.stepek, m.stepkin,
                 m.cell, m.cellres, m.nbr_j, m.nbr_code, m.nbr_cnt, m.blockpart,
-                m.blockek, m.frc, m.nose, m.thermo, m.flags, s.cell, s.cell_count, s.cell_start,
+                m.frc, m.nose, m.thermo, m.flags, s.cell, s.cell_count, s.cell_start,
                 s.cell_fill, s.sorted_tmp, s.sorted, s.cnt, s.off, s.pi, s.pj, s.scode,
                 s.com_ref, s.lflags, m.box, m.anders, s.tile_part, m.nb_id, m.nb_base,
                 m.trow, m.trow_cnt, m.tcnt, s.snap, s.seam};
@@ -684,34 +685,46 @@ static void free_all(System &s) {
   if (s.stream) (void)hipStreamDestroy(s.stream);
 }
 
-// k steps: predict, forces; (correct + predict, forces) x (k-1); correct.
-// Each call is self-contained, so a captured graph of k steps can be replayed.
-// With the Andersen barostat the box of step t follows from the pressure of
-// step t-1, which needs every molecule's corrector: correct, close (thermo,
-// Nose and Andersen correct and predict, the new box), predict and bin in
-// that box, forces; four kernels per step.
+// k steps.  Each call is self-contained (it starts with the predictors and
+// ends with the correctors), so a captured graph of k steps can be replayed.
+//   Up to step_max molecules on the rows: the predictors, then one kernel per
+//   step (forces, correctors and the next predictors; md_step_body).
+//   Beyond, and on the tiles: predict, forces; (correct + predict, forces) x
+//   (k-1); correct.
+//   Andersen barostat: the box of step t follows from the pressure of step
+//   t-1, which needs every molecule's corrector: correct, close (thermo, Nose
+//   and Andersen correct and predict, the new box), predict and bin in that
+//   box, forces; four kernels per step.
 static void launch_steps(System &s, int k) {
+  if (k < 1) return;
   if (s.andersen) {
     for (int q = 0; q < k; q++) {
       const int p = q & 1;
       if (q > 0) md_launch_pre(s, true, false, false, 0);
-      // clears the cells and rebuild flag of parity p before they are filled
-      md_launch_close(s, (q > 0 ? 1 : 0) | 2 | 4, 1 - p, 1 - p);
+      // clears the cells and rebuild flag of list p before they are filled
+      md_launch_close(s, (q > 0 ? 1 : 0) | 2, 1 << p, 1 - p);
       md_launch_pre(s, false, true, true, p);
       md_launch_main(s, nullptr, p, 0);
     }
     md_launch_pre(s, true, false, false, 0);
-    md_launch_close(s, 1 | 8, 0, (k - 1) & 1);
+    md_launch_close(s, 1, 7, (k - 1) & 1);
     return;
   }
-  for (int q = 0; q < k; q++) {
-    const int p = q & 1;
-    md_launch_pre(s, q > 0, true, true, p);
-    if (q == 0) md_launch_close(s, 2 | 4, p, 1 - p);
-    md_launch_main(s, nullptr, p, q > 0 ? (1 | 2 | 4) : 0);
+  if (s.tiles || !s.one_kernel) {
+    for (int q = 0; q < k; q++) {
+      const int p = q & 1;
+      md_launch_pre(s, q > 0, true, true, p);
+      if (q == 0) md_launch_close(s, 2, 1 << (1 - p), 1 - p);
+      md_launch_main(s, nullptr, p, q > 0 ? (1 | 2) : 0);
+    }
+    md_launch_pre(s, true, false, false, 0);
+    md_launch_close(s, 1, 7, (k - 1) & 1);
+    return;
   }
-  md_launch_pre(s, true, false, false, 0);
-  md_launch_close(s, 1 | 8, 0, (k - 1) & 1);
+  md_launch_pre(s, false, true, true, 0, (k - 1) & 1);
+  md_launch_step_close(s, 2, k);
+  for (int q = 0; q < k; q++) md_launch_step(s, q, k);
+  md_launch_step_close(s, 1, k);
 }
 
 void drop_graphs(System &s) {
@@ -1006,8 +1019,7 @@ static int snap_state(System &s, bool restore) {
   struct Part {
     double *d;
     size_t len;
-  } parts[] = {{s.md.com, 3 * n}, {s.md.dx, 15 * n}, {s.md.w, 15 * n},   {s.md.quat, 20 * n},
-               {s.md.nose, 9},    {s.md.box, 8},      {s.md.anders, 8}};
+  } parts[] = {{s.md.com, kRowRef * n}, {s.md.nose, 9}, {s.md.box, 8}, {s.md.anders, 8}};
   double *p = s.snap;
   for (const Part &q : parts) {
     if (!q.d) continue;
@@ -1104,16 +1116,24 @@ int g6_step_timed(g6_handle h, int nsteps, double *t) {
   if (!s || nsteps < 1 || !t || s->andersen) return G6_EARG;
   double acc[5] = {0, 0, 0, 0, 0};
   for (int k = 0; k < nsteps; k++) {
-    // one step: predict, forces, correct (the corrector and the next
-    // predictor share a kernel in g6_step; here they are timed apart)
+    // one step: predict, forces, correct.  Where a step is one kernel the
+    // corrector runs in the force kernel; elsewhere the corrector and the
+    // next predictor, which share a kernel in g6_step, are timed apart
     G6_CHECK(hipEventRecord(s->ev[0], s->stream));
     md_launch_pre(*s, false, true, true, 0);
-    md_launch_close(*s, 2 | 4, 0, 1);
+    const bool two = s->tiles || !s->one_kernel;
+    if (two) md_launch_close(*s, 2, 2, 1);
+    else md_launch_step_close(*s, 2, 1);
     G6_CHECK(hipEventRecord(s->ev[1], s->stream));
-    md_launch_main(*s, nullptr, 0, 0);
+    if (two) md_launch_main(*s, nullptr, 0, 0);
+    else md_launch_step(*s, 0, 1);
     G6_CHECK(hipEventRecord(s->ev[2], s->stream));
-    md_launch_pre(*s, true, false, false, 0);
-    md_launch_close(*s, 1 | 8, 0, 0);
+    if (two) {
+      md_launch_pre(*s, true, false, false, 0);
+      md_launch_close(*s, 1, 7, 0);
+    } else {
+      md_launch_step_close(*s, 1, 1);
+    }
     G6_CHECK(hipEventRecord(s->ev[3], s->stream));
     G6_CHECK(hipEventSynchronize(s->ev[3]));
     float a, b, c, e;
@@ -1121,7 +1141,7 @@ int g6_step_timed(g6_handle h, int nsteps, double *t) {
     G6_CHECK(hipEventElapsedTime(&b, s->ev[1], s->ev[2]));
     G6_CHECK(hipEventElapsedTime(&c, s->ev[2], s->ev[3]));
     G6_CHECK(hipEventElapsedTime(&e, s->ev[0], s->ev[3]));
-    acc[0] += b;   // force kernel (rows rebuilt in it when due)
+    acc[0] += b;   // force kernel (rows rebuilt in it when due, the rows' corrector)
     acc[1] += 0;   // no separate list build
     acc[2] += a + c;
     acc[3] += e;
@@ -1193,7 +1213,7 @@ static int eval_forces_into(System *s, double *out, double *force, double *torqu
     md_launch_flag(*s, 2, 1);  // rebuild the rows of parity 0
     md_launch_pre(*s, false, false, true, 0);
     md_launch_main(*s, out, 0, 0);
-    md_launch_close(*s, 16 | 8, 0, 0);
+    md_launch_close(*s, 16, 7, 0);
     G6_CHECK(hipGetLastError());
     G6_CHECK(hipMemcpyAsync(force, out, sizeof(double) * 3 * n, hipMemcpyDeviceToHost, s->stream));
     G6_CHECK(hipMemcpyAsync(torque, out + 3 * n, sizeof(double) * 3 * n, hipMemcpyDeviceToHost,
@@ -1321,7 +1341,7 @@ int g6_set_andersen(g6_handle h, int mode, double pex, double mass, const double
     G6_CHECK(hipMemcpy(s->md.anders, an, sizeof(an), hipMemcpyHostToDevice));
     s->andersen_mode = mode;
     // rows of the new box
-    int one[2] = {1, 1};
+    int one[3] = {1, 1, 1};
     G6_CHECK(hipMemcpy(s->md.flags + 2, one, sizeof(one), hipMemcpyHostToDevice));
   }
   drop_graphs(*s);  // the captured launches embed the step sequence

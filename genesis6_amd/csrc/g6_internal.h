@@ -103,22 +103,35 @@ struct Geom {
 // site, as floats from [4] (FP32 mode, 128 B) or doubles from [4] (FP64).
 constexpr int kRecF = 16, kRecD = 24;
 
+// Rows of the state block [kStateRows][n]: com 0..2, dx 3..17, w, quat, com_ref
+constexpr int kRowW = 18, kRowQ = 33, kRowRef = 53, kStateRows = 56;
+
 // Device pointers and sizes of the MD path, passed to kernels by value.
 struct MdBuf {
+  // com is the state block's first row; dx, w, quat and com_ref (the COMs at
+  // the last row build) are rows of it
   double *com, *dx, *w, *quat, *tmat, *com_ref;
-  double *rec;  // [n][rs] records
+  // records [2][n][rs] and the predicted COMs by component [2][3][n] (scanned
+  // rows): a step kernel reads one half and writes the next step's into the
+  // other; every other kernel uses the first half
+  double *rec, *comp;
   int rs;
   int *cell;     // [n] MD-grid cell of each molecule
-  int *cellres;  // [2][ncell][cell_cap]: slot 0 the count, residents from slot 1
+  // [3][ncell][cell_cap]: entry 0 the count, residents from entry 1.  A step
+  // kernel reads one of the three lists, fills the next and clears the third
+  int *cellres;
   int cell_cap;
   int *nbr_j, *nbr_code, *nbr_cnt;
   int maxnb;
   int scan;  // rows from a scan of every molecule instead of the cell lists
   double *frc;        // [6][n] force and torque (lab) of the last k_md_main
   double *blockpart;  // [2][nblk][16] k_md_main block partials, by parity
-  double *blockek;    // [k_md_pre waves][kEkLen] kinetic partials
-  double *nose, *thermo;
-  int *flags;  // [0] error code, [2 + parity] rebuild rows this step
+  // kinetic partials [2][groups][kEkLen] and kinetic energies [2][groups] of
+  // the groups of four molecules: the step kernel's by parity, k_md_pre's in
+  // the first halves
+  double *stepek, *stepkin;
+  double *nose, *thermo;  // nose[2][9]: by parity inside a call, [0] between
+  int *flags;  // [0] error code, [2 + list] rebuild rows this step
   double half_skin2;
   // Andersen constant-pressure MD (both nullptr for a fixed box).  box
   // (kBoxLen doubles): [0..2] the current edges, [3..5] their inverses,
@@ -284,6 +297,7 @@ struct System {
   int *flags = nullptr;   // = md.flags
   int *lflags = nullptr;  // g6_pairlist: [0] error code, [1] build gate
   int nblk_md = 0;
+  bool one_kernel = false;  // steps on the rows run as one kernel each
   PairK<float> pkf{};
   PairK<double> pkd{};
   hipStream_t stream = nullptr;
@@ -343,8 +357,13 @@ PairK<R> make_pair_k(const ModelTable &mt, const Geom &g) {
 // Arguments of the step-close work (k_md_close, or block 0 of k_md_main).
 struct CloseArgs {
   int mode, nose_active, nblk_pre, nblk_main;
-  const double *bpart;  // pair partials of the k_md_main being closed
+  const double *bpart;  // pair partials of the force kernel being closed
   double dt;
+  // kinetic partials [nblk_pre][kEkLen] and kinetic energies [nblk_pre]
+  const double *ek, *kin;
+  const double *nose_in;  // thermostat state read and written
+  double *nose_out;
+  int clear;  // cell lists and rebuild flags to clear, one bit each
 };
 // Bytes of the per-wave LDS region of k_md_main: the row sort buffers while
 // a row is rebuilt, then the compacted interacting entries (index and the
@@ -354,7 +373,7 @@ struct CloseArgs {
 constexpr int kRowWords = 128;
 inline int main_region_bytes(int maxnb, int rsize) {
   auto up16 = [](int x) { return (x + 15) / 16 * 16; };
-  const int sort = 8 * maxnb + 8 * kRowWords;
+  const int sort = 8 * maxnb + 8 * kRowWords + 4 * (128 + 132);  // entries, window, stencil
   const int comp = up16(4 * maxnb) + 3 * up16(rsize * maxnb);
   const int acc = 10 * 64 * 8;
   const int mx = sort > comp ? sort : comp;
@@ -363,23 +382,41 @@ inline int main_region_bytes(int maxnb, int rsize) {
 // doubles per block partial of k_md_main: the energy and the pair virial
 // [0..9] (each a compensated block sum, rounded once), pair counts [10..11]
 constexpr int kBP = 16;
-// kinetic partials per k_md_pre wave: sum |dx(1)|^2, sum w_x^2, w_y^2, w_z^2,
+// kinetic partials per group of four molecules: sum |dx(1)|^2, sum w_x^2, w_y^2, w_z^2,
 // and the upper triangle xx xy xz yy yz zz of sum dx(1) dx(1)^T
 constexpr int kEkLen = 10;
-// reduction slots of the step close per wave: 12 pair quantities and kEkLen
-// kinetic ones
-constexpr int kRed = 12 + kEkLen;
-// waves of k_md_pre (64 molecules per block of four waves); each writes
-// one kinetic partial
-inline int pre_waves(int n) { return (n + 63) / 64 * 4; }
-void md_launch_pre(System &s, bool correct, bool predict, bool sites, int parity);
+// reduction slots of the step close per wave: 12 pair quantities, kEkLen
+// kinetic ones and the kinetic energy
+constexpr int kRed = 12 + kEkLen + 1;
+// blocks of k_md_pre (64 molecules each)
+inline int pre_blocks(int n) { return (n + 63) / 64; }
+// k_md_pre into cell list `list` and record half `half`
+void md_launch_pre(System &s, bool correct, bool predict, bool sites, int list, int half = 0);
 // flags[k] = v, stream-ordered
 void md_launch_flag(System &s, int k, int v);
-// close of the step whose k_md_main wrote the partials of src_parity
-void md_launch_close(System &s, int mode, int parity, int src_parity);
-// k_md_main of this parity; close_mode != 0 closes the previous step
-// (partials of parity 1 - parity) in block 0
+// close of the step whose force kernel wrote the pair partials of src_parity;
+// clear: cell lists and rebuild flags to clear (bits)
+void md_launch_close(System &s, int mode, int clear, int src_parity);
+// k_md_main on cell list / rebuild flag `parity`, partials of this parity;
+// close_mode != 0 closes the previous step (partials of parity 1 - parity) in
+// block 0 and clears the other list
 void md_launch_main(System &s, double *out, int parity, int close_mode);
+// One kernel per step (md_step_body): step q of a call of k steps, and the
+// closes of the thermostat state before the first step (mode 2) and after the
+// last (mode 1).
+void md_launch_step(System &s, int q, int k);
+void md_launch_step_close(System &s, int mode, int k);
+// One kernel per step up to this many molecules of a launch, predictor and
+// force kernels beyond: with four molecules per block the corrector keeps 16
+// of 64 lanes, about a quarter more instructions per molecule than the
+// predictor kernel's 64 molecules per block, which a launch that fills the
+// chip several times over pays and a shorter one hides.  Measured per step,
+// two kernels / one, TIP4P: FP32 1000 molecules 12.1 / 8.6 us, 4096 21.3 /
+// 18.2, 5600 26.1 / 23.4 (ST2 29.3 / 28.8, 8289 38.8 / 40.9); FP64 216 with
+// rows rebuilt every step 14.1 / 10.4, 4096 25.7 / 25.2, 5600 32.1 / 33.5; 64
+// ladder systems of 61,440 molecules 144 / 158.
+constexpr int kStepMaxF = 6144, kStepMaxD = 4608;
+int step_max(int prec);  // the line, or G6_STEP_MAX
 // the cell-tile force kernel (g6_tile.hip) and the reduction of its partials
 // into force and body torque (out[6][n])
 void md_launch_tile(System &s, int parity, const CloseArgs &ca);
@@ -420,6 +457,7 @@ struct Ladder {
   MdRep *reps = nullptr;                         // [nsys], device
   int2 *map_pre = nullptr, *map_main = nullptr;  // [grid], device
   int grid_pre = 0, grid_main = 0, reg_bytes = 0;
+  bool one_kernel = false;
   double *th_dev = nullptr;  // [nsys][G6_THERMO_LEN] gathered thermo records
   int *fl_dev = nullptr;     // [nsys] gathered error codes
   double *th_host = nullptr; // pinned copies of the two
@@ -429,9 +467,10 @@ struct Ladder {
   int graph_steps = 0;
   int map_mode = G6_LADDER_MAP_FLAT;
 };
-void md_launch_pre_lad(Ladder &l, bool correct, bool predict, bool sites, int parity);
-void md_launch_close_lad(Ladder &l, int mode, int parity, int src_parity);
+void md_launch_pre_lad(Ladder &l, bool correct, bool predict, int list, int half);
+void md_launch_close_lad(Ladder &l, int mode, int k);
 void md_launch_main_lad(Ladder &l, int parity, int close_mode);
+void md_launch_step_lad(Ladder &l, int q, int k);
 void md_launch_gather_lad(Ladder &l);  // thermo records and error codes
 // Set a system's thermostat to temp after a replica exchange
 // (Mixture.F90:1630-1653): velocities scaled by sqrt(temp / old temp),

@@ -70,14 +70,22 @@ static int set_temperature_from(System &s, double temp, double old_temp) {
 
 // k steps of every system, the launch sequence of g6_step's launch_steps
 static void launch_steps_lad(Ladder &l, int k) {
+  if (k < 1) return;
+  if (l.one_kernel) {
+    md_launch_pre_lad(l, false, true, 0, (k - 1) & 1);
+    md_launch_close_lad(l, 2, k);
+    for (int q = 0; q < k; q++) md_launch_step_lad(l, q, k);
+    md_launch_close_lad(l, 1, k);
+    return;
+  }
   for (int q = 0; q < k; q++) {
     const int p = q & 1;
-    md_launch_pre_lad(l, q > 0, true, true, p);
-    if (q == 0) md_launch_close_lad(l, 2 | 4, p, 1 - p);
-    md_launch_main_lad(l, p, q > 0 ? (1 | 2 | 4) : 0);
+    md_launch_pre_lad(l, q > 0, true, p, 0);
+    if (q == 0) md_launch_close_lad(l, 2, k);
+    md_launch_main_lad(l, p, q > 0 ? (1 | 2) : 0);
   }
-  md_launch_pre_lad(l, true, false, false, 0);
-  md_launch_close_lad(l, 1 | 8, 0, (k - 1) & 1);
+  md_launch_pre_lad(l, true, false, 0, 0);
+  md_launch_close_lad(l, 1, k);
 }
 
 // Block maps: systems go to the XCD lane with the fewest molecules so far
@@ -162,9 +170,12 @@ static void build_map_flat(const std::vector<int> &nblk, int first, std::vector<
 static int ladder_maps(Ladder &l) {
   const size_t ns = l.sys.size();
   std::vector<int> order(ns), lane_of(ns), np(ns), nm(ns);
+  long long total = 0;
+  for (const System *s : l.sys) total += s->n;
+  l.one_kernel = total <= step_max(l.prec);
   for (size_t r = 0; r < ns; r++) {
     order[r] = (int)r;
-    np[r] = pre_waves(l.sys[r]->n) / 4;
+    np[r] = pre_blocks(l.sys[r]->n);
     nm[r] = l.sys[r]->nblk_md;
   }
   std::vector<int2> mp, mm;

@@ -1,4 +1,5 @@
-// The MD step (the path g6_step runs), two kernels per step:
+// The MD step (the path g6_step runs), one kernel per step for systems of up
+// to a few thousand molecules (k_md_step) and two beyond:
 //
 //   k_md_pre   64 molecules per block, one Gear role per wave, state held
 //              in registers: rigid_correct with the forces of the previous
@@ -15,10 +16,10 @@
 //              k_md_close).  Pair partials alternate between two parities.
 //   k_md_main  one wavefront per molecule i:
 //              (1) if a rebuild is due, i's own neighbour row: every j != i
-//                  of the cells whose box lies within rc + skin of i (a 5^3
-//                  stencil of cells of edge >= (rc+skin)/2) that passes the
-//                  reference's FP64 minimum-image test dd < (rc+skin)^2,
-//                  sorted by j;
+//                  (small systems), or every j != i of the cells whose box
+//                  lies within rc + skin of i (a 5^3 stencil of cells of edge
+//                  >= (rc+skin)/2), that passes the reference's FP64
+//                  minimum-image test dd < (rc+skin)^2, sorted by j;
 //              (2) the pair forces of i with every listed j whose FP64 COM
 //                  distance passes dd < rc^2 - the reference's
 //                  Interaction_Compress2 test, so the interacting set is the
@@ -26,16 +27,20 @@
 //              (3) wave reduction of i's force and lab torque (the work of
 //                  rigid_collectforce), stored for the corrector;
 //              (4) block partials of energy and virial.
-// A step is k_md_pre(correct previous, predict) + k_md_main, whose block 0
-// first does the close work of the previous step (k_md_close runs on its own
-// only around the first and last step of a run); a run of steps ends with a
-// correct-only k_md_pre + k_md_close, so every
-// g6_step call leaves the state of the reference's loop end (after
-// Nose_Correct, Mixture.F90:2282).  Cell lists and rebuild flags alternate
-// between two parities so that no kernel needs a grid-wide barrier.
+//   k_md_step  k_md_main's work and, for the block's four molecules, the
+//              corrector and the next step's k_md_pre.
+// A step is k_md_step, or k_md_pre(correct previous, predict) + k_md_main;
+// block 0 of the pair kernel first does the close work of the previous step
+// (k_md_close runs on its own only around the first and last step of a run).
+// A run of steps ends with the correctors and k_md_close, so every g6_step
+// call leaves the state of the reference's loop end (after Nose_Correct,
+// Mixture.F90:2282).  Cell lists, rebuild flags and partials alternate so that
+// no kernel needs a grid-wide barrier; both forms give the same bits.
 // Each unordered pair is evaluated in both rows, so no molecule's force
 // needs an atomic, rows are sorted and every reduction runs in a fixed
 // order: results are deterministic.  Energies and the virial are halved.
+#include <type_traits>
+
 #include "g6_md_common.h"
 
 // Everything written in this file is FP64 bookkeeping in the reference's
@@ -58,6 +63,25 @@ __device__ inline void part_sum(const MdBuf &b, int i, double (&f)[3]) {
     for (int a = 0; a < 3; a++) f[a] += (double)p[q * 6 + a];
 }
 
+// value of lane l of the quad
+template <int L>
+__device__ inline double quad_d(double v) {
+  return dpp_d<L * 0x55>(v);
+}
+// sum over the quad in a fixed order, in every lane
+__device__ inline double quad_sum_d(double v) {
+  v += dpp_d<0xB1>(v);
+  v += dpp_d<0x4E>(v);
+  return v;
+}
+
+// kinetic energy of four molecules from their sums of |dx(1)|^2 and w^2
+__device__ inline double kin_energy(const ModelTable &mt, double dt, double et, double ex,
+                                    double ey, double ez) {
+  return et * mt.mass * 0.5 * (1.0 / (dt * dt)) +
+         (ex * mt.Ixx + ey * mt.Iyy + ez * mt.Izz) * 0.5;
+}
+
 // ---- kernel A --------------------------------------------------------------
 // A block updates 64 molecules (one per lane) with one role per wave:
 //   wave 0  translation: com, dx[5][3]; record COM, binning, skin test
@@ -72,19 +96,23 @@ __device__ inline void part_sum(const MdBuf &b, int i, double (&f)[3]) {
 template <int BOX>
 __device__ __forceinline__ void md_pre_body(const ModelTable &mt, const Geom &g, const MdBuf &b,
                                             double dt, int nose_active, int do_correct,
-                                            int do_predict, int do_sites, int parity, int blk) {
+                                            int do_predict, int do_sites, int list, int half,
+                                            int blk) {
   constexpr bool NPT = BOX == kBoxBaro;
   __shared__ double s_w0[3][64], s_W[12][64];
   __shared__ double s_q0[4][64], s_p[4][64], s_r[4][64], s_s[4][64], s_qn[4][64];
+  __shared__ double s_ew[3][16];
   const int n = g.n;
   const int role = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   const int i = blk * 64 + lane;
   const bool ok = i < n;
   const bool q2 = role == 2;  // wave 2: components a, b; wave 3: c, d
-  double ek[kEkLen];  // Ek terms and the kinetic tensor
-#pragma unroll
-  for (int q = 0; q < kEkLen; q++) ek[q] = 0.0;
+  // kinetic partials of the group of four molecules of lanes 4 l .. 4 l + 3
+  const int grp = blk * 16 + (lane >> 2);
+  const bool grp_ok = (lane & 3) == 0 && grp * 4 < n;
+  double *ek = b.stepek + (size_t)grp * kEkLen;
+  double et = 0.0;
   double S[20];  // wave 0: com, dx; wave 1: w; waves 2-3: q (all four)
 #pragma unroll
   for (int k = 0; k < 20; k++) S[k] = 0.0;
@@ -157,15 +185,20 @@ __device__ __forceinline__ void md_pre_body(const ModelTable &mt, const Geom &g,
           S[12 + a] = S[12 + a] + kG5_4 * d;
           S[15 + a] = S[15 + a] + kG5_5 * d;
         }
-        ek[0] = S[3] * S[3] + S[4] * S[4] + S[5] * S[5];
-        // Rigid_PressureTensor sums (RigidModule.F90:600-619), upper triangle
-        ek[4] = S[3] * S[3];
-        ek[5] = S[3] * S[4];
-        ek[6] = S[3] * S[5];
-        ek[7] = S[4] * S[4];
-        ek[8] = S[4] * S[5];
-        ek[9] = S[5] * S[5];
       }
+      // Rigid_Ek and Rigid_PressureTensor sums (RigidModule.F90:576-619),
+      // upper triangle
+      const double v[3] = {ok ? S[3] : 0.0, ok ? S[4] : 0.0, ok ? S[5] : 0.0};
+      et = quad_sum_d(v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
+      if (grp_ok) ek[0] = et;
+      int q = 4;
+#pragma unroll
+      for (int l = 0; l < 3; l++)
+#pragma unroll
+        for (int h = l; h < 3; h++, q++) {
+          const double e = quad_sum_d(v[l] * v[h]);
+          if (grp_ok) ek[q] = e;
+        }
     } else if (role == 1) {
       if (ok) {
         // rigid_collectforce's body-frame torque (RigidModule.F90:301-306)
@@ -187,9 +220,12 @@ __device__ __forceinline__ void md_pre_body(const ModelTable &mt, const Geom &g,
           S[9 + a] = S[9 + a] + kG4_3 * d;
           S[12 + a] = S[12 + a] + kG4_4 * d;
         }
-        ek[1] = S[0] * S[0];
-        ek[2] = S[1] * S[1];
-        ek[3] = S[2] * S[2];
+      }
+#pragma unroll
+      for (int c = 0; c < 3; c++) {
+        const double w0 = ok ? S[c] : 0.0, e = quad_sum_d(w0 * w0);
+        if (grp_ok) ek[1 + c] = e;
+        if ((lane & 3) == 0) s_ew[c][lane >> 2] = e;
       }
 #pragma unroll
       for (int k = 0; k < 12; k++) s_W[k][lane] = S[k];
@@ -216,6 +252,9 @@ __device__ __forceinline__ void md_pre_body(const ModelTable &mt, const Geom &g,
       }
     }
     __syncthreads();
+    if (role == 0 && grp_ok)
+      b.stepkin[grp] = kin_energy(mt, dt, et, s_ew[0][lane >> 2], s_ew[1][lane >> 2],
+                                  s_ew[2][lane >> 2]);
     // quaternion derivatives from the corrected w: own components, then
     // the partner's through LDS
     double w1x = 0, w1y = 0, w1z = 0, w2x = 0, w2y = 0, w2z = 0, w3x = 0, w3y = 0, w3z = 0,
@@ -340,10 +379,12 @@ __device__ __forceinline__ void md_pre_body(const ModelTable &mt, const Geom &g,
   }
   if (do_sites && ok) {
     if (role == 0) {
-      double *rec = b.rec + (size_t)i * b.rs;
-      rec[0] = S[0];
-      rec[1] = S[1];
-      rec[2] = S[2];
+      double *rec = b.rec + ((size_t)half * n + i) * b.rs;
+#pragma unroll
+      for (int a = 0; a < 3; a++) {
+        rec[a] = S[a];
+        if (b.scan) b.comp[(3 * half + a) * n + i] = S[a];
+      }
       if (!b.scan) {
         int jc[3], nd[3];
         grid_nd<BOX>(g, nd);
@@ -360,7 +401,7 @@ __device__ __forceinline__ void md_pre_body(const ModelTable &mt, const Geom &g,
         const int c = (jc[2] * nd[1] + jc[1]) * nd[0] + jc[0];
         b.cell[i] = c;
         // slot 0 of a cell row is its count; residents follow
-        int *cr = b.cellres + ((size_t)parity * g.ncell + c) * b.cell_cap;
+        int *cr = b.cellres + ((size_t)list * g.ncell + c) * b.cell_cap;
         const int slot = atomicAdd(cr, 1) + 1;
         if (slot < b.cell_cap)
           cr[slot] = i;
@@ -377,9 +418,9 @@ __device__ __forceinline__ void md_pre_body(const ModelTable &mt, const Geom &g,
           h2 = h > 0.0 ? h * h : -1.0;
         }
         const double e0 = S[0] - cref[0], e1 = S[1] - cref[1], e2 = S[2] - cref[2];
-        if (e0 * e0 + e1 * e1 + e2 * e2 > h2) b.flags[2 + parity] = 1;
+        if (e0 * e0 + e1 * e1 + e2 * e2 > h2) b.flags[2 + list] = 1;
       } else if (i == 0) {
-        b.flags[2 + parity] = 1;  // no skin: the reference rebuilds every step
+        b.flags[2 + list] = 1;  // no skin: the reference rebuilds every step
       }
       if (NPT && i == 0 &&
           (bx.L[0] < b.box[12] * b.box[15] || bx.L[1] < b.box[13] * b.box[15] ||
@@ -404,10 +445,10 @@ __device__ __forceinline__ void md_pre_body(const ModelTable &mt, const Geom &g,
 #pragma unroll
         for (int a = 5; a < 9; a++) b.tmat[a * n + i] = t[a];
       }
-      double *rec = b.rec + (size_t)i * b.rs;
+      double *rec = b.rec + ((size_t)half * n + i) * b.rs;
       float *recf = reinterpret_cast<float *>(rec + 4);
-      const int nq = mt.nsite - 1, half = (nq + 1) / 2;
-      const int s0 = q2 ? 0 : half, s1 = q2 ? half : nq;
+      const int nq = mt.nsite - 1, mid = (nq + 1) / 2;
+      const int s0 = q2 ? 0 : mid, s1 = q2 ? mid : nq;
       for (int s = s0; s < s1; s++) {
         const double r0 = t[0] * mt.bx[s] + t[1] * mt.by[s] + t[2] * mt.bz[s];
         const double r1 = t[3] * mt.bx[s] + t[4] * mt.by[s] + t[5] * mt.bz[s];
@@ -424,65 +465,35 @@ __device__ __forceinline__ void md_pre_body(const ModelTable &mt, const Geom &g,
       }
     }
   }
-  // kinetic partials of this wave, reduced by the step close
-  // each wave reduces the partials its role produced (the rest are zero)
-  if (do_correct && role == 0) {
-    ek[0] = wsum63(ek[0]);
-#pragma unroll
-    for (int q = 4; q < kEkLen; q++) ek[q] = wsum63(ek[q]);
-  } else if (do_correct && role == 1) {
-#pragma unroll
-    for (int q = 1; q < 4; q++) ek[q] = wsum63(ek[q]);
-  }
-  if (lane == 63) {
-    const size_t wv = (size_t)blk * 4 + role;
-#pragma unroll
-    for (int q = 0; q < kEkLen; q++) b.blockek[wv * kEkLen + q] = ek[q];
-  }
 }
 
 template <int BOX>
 __global__ __launch_bounds__(256) void k_md_pre(ModelTable mt, Geom g, MdBuf b, double dt,
                                                 int nose_active, int do_correct, int do_predict,
-                                                int do_sites, int parity) {
-  md_pre_body<BOX>(mt, g, b, dt, nose_active, do_correct, do_predict, do_sites, parity,
+                                                int do_sites, int list, int half) {
+  md_pre_body<BOX>(mt, g, b, dt, nose_active, do_correct, do_predict, do_sites, list, half,
                    blockIdx.x);
 }
 
 // Ladder form: one launch over the blocks of every system of a ladder;
-// map[blockIdx.x] names the system and its block (system < 0: an idle
-// block that pads the XCD interleave).
+// map[blockIdx.x] names the system and its block (system < 0: an idle block
+// that pads the XCD interleave).
 __global__ __launch_bounds__(256) void k_md_pre_lad(ModelTable mt, const MdRep *__restrict__ reps,
                                                     const int2 *__restrict__ map, int do_correct,
-                                                    int do_predict, int do_sites, int parity) {
+                                                    int do_predict, int list, int half) {
   const int2 m = map[blockIdx.x];
   if (m.x < 0) return;
   const Geom g = reps[m.x].g;
   const MdBuf b = reps[m.x].b;
   md_pre_body<kBoxCube>(mt, g, b, reps[m.x].dt, reps[m.x].nose_active, do_correct, do_predict,
-                     do_sites,
-              parity, m.y);
+                        do_predict, list, half, m.y);
 }
 
 template <bool NPT>
-__global__ __launch_bounds__(256) void k_md_close(ModelTable mt, MdBuf b, int n, double dt,
-                                                  int nblk_pre, const double *bpart,
-                                                  int nblk_main, int ncell, int nose_active,
-                                                  int mode, int parity, double box_vol) {
+__global__ __launch_bounds__(256) void k_md_close(ModelTable mt, MdBuf b, int n, int ncell,
+                                                  double box_vol, CloseArgs ca) {
   __shared__ double s_red[4][kRed];
-  close_body<NPT>(mt, b, n, dt, nblk_pre, bpart, nblk_main, ncell, nose_active, mode, parity,
-                  box_vol, s_red);
-}
-
-// Ladder form: block r closes system r.
-__global__ __launch_bounds__(256) void k_md_close_lad(ModelTable mt, const MdRep *__restrict__ reps,
-                                                      int mode, int parity, int src_parity) {
-  __shared__ double s_red[4][kRed];
-  const MdRep &r = reps[blockIdx.x];
-  const MdBuf b = r.b;
-  const int n = r.g.n, nm = r.nblk_main;
-  close_body<false>(mt, b, n, r.dt, (n + 63) / 64 * 4, b.blockpart + (size_t)src_parity * nm * kBP, nm,
-             r.g.ncell, r.nose_active, mode, parity, box_volume(r.g.L), s_red);
+  close_body<NPT, 8>(mt, b, n, ncell, box_vol, ca, s_red);
 }
 
 // ---- kernel B --------------------------------------------------------------
@@ -546,8 +557,8 @@ __device__ inline bool row_test(const BoxNow &bx, const MdBuf &b, double rr, dou
 // which are contiguous in j), so the cost is n / 64 tests per lane and no
 // latency of cell counts, search and sort.  Taken up to kScanMax molecules.
 template <int BOX>
-__device__ inline int scan_row(const Geom &g, const MdBuf &b, int i, int lane, double xi, double yi,
-                               double zi, int *nj, int *nc) {
+__device__ inline int scan_row(const Geom &g, const MdBuf &b, const double *com, int i, int lane,
+                               double xi, double yi, double zi, int *nj, int *nc) {
   const BoxNow bx = box_now<BOX>(g, b);
   const int n = g.n, cap = b.maxnb;
   const unsigned long long lt = (1ull << lane) - 1ull;
@@ -557,9 +568,9 @@ __device__ inline int scan_row(const Geom &g, const MdBuf &b, int i, int lane, d
 #pragma unroll
     for (int u = 0; u < 4; u++) {
       const int j = min(j0 + 64 * u + lane, n - 1);
-      x[u] = b.com[j];
-      y[u] = b.com[n + j];
-      z[u] = b.com[2 * n + j];
+      x[u] = com[j];
+      y[u] = com[n + j];
+      z[u] = com[2 * n + j];
     }
 #pragma unroll
     for (int u = 0; u < 4; u++) {
@@ -591,14 +602,15 @@ __device__ inline int scan_row(const Geom &g, const MdBuf &b, int i, int lane, d
 // smaller entries of the row per entry was 3 passes of 176 LDS reads at 4096
 // molecules, skin 1.8 A, twice the instructions of a step without a build.)
 template <int BOX>
-__device__ inline int cell_row(const Geom &g, const MdBuf &b, int parity, int i, int lane,
-                               double xi, double yi, double zi, int (&s_beg)[128],
-                               int (&s_pre)[132], int *s_j, int *nj, int *nc) {
+__device__ inline int cell_row(const Geom &g, const MdBuf &b, const double *rec, int list, int i,
+                               int lane, double xi, double yi, double zi, int *s_j, int *nj,
+                               int *nc) {
   const BoxNow bx = box_now<BOX>(g, b);
   const int n = g.n;
   int *s_c = s_j + b.maxnb;
   unsigned *s_bit = reinterpret_cast<unsigned *>(s_c + b.maxnb);
   int *s_cnt = reinterpret_cast<int *>(s_bit + kRowWords);
+  int *s_beg = s_cnt + kRowWords, *s_pre = s_beg + 128;
   int nd[3];
   grid_nd<BOX>(g, nd);
   const int nx = nd[0], ny = nd[1], nz = nd[2];
@@ -607,7 +619,7 @@ __device__ inline int cell_row(const Geom &g, const MdBuf &b, int parity, int i,
   const Stencil st = stencil_of(nd);
   const double ux = frac_in_cell(bx, xi, 0), uy = frac_in_cell(bx, yi, 1),
                uz = frac_in_cell(bx, zi, 2);
-  const int *res = b.cellres + (size_t)parity * g.ncell * b.cell_cap;
+  const int *res = b.cellres + (size_t)list * g.ncell * b.cell_cap;
   int carry = 0;
   for (int e0 = 0; e0 < st.nst; e0 += 64) {
     const int e = e0 + lane;
@@ -657,7 +669,7 @@ __device__ inline int cell_row(const Geom &g, const MdBuf &b, int parity, int i,
       }
       j = res[s_beg[lo] + (t - s_pre[lo])];
       if (j != i) {
-        const double *recj = b.rec + (size_t)j * b.rs;
+        const double *recj = rec + (size_t)j * b.rs;
         pass = row_test(bx, b, g.rr, xi - recj[0], yi - recj[1], zi - recj[2], code);
       }
     }
@@ -724,17 +736,18 @@ __device__ inline int cell_row(const Geom &g, const MdBuf &b, int parity, int i,
 // neighbour-row build of molecule i into nbr[i*maxnb ...], in the order of
 // j; returns the row length (also stored).
 template <int BOX>
-__device__ inline int build_row(const Geom &g, const MdBuf &b, int parity, int i, int lane,
-                                int (&s_beg)[128], int (&s_pre)[132], int *s_sort) {
+__device__ inline int build_row(const Geom &g, const MdBuf &b, int list, int half, int i, int lane,
+                                int *s_sort) {
   constexpr bool NPT = BOX == kBoxBaro;
   const int n = g.n;
-  const double *reci = b.rec + (size_t)i * b.rs;
+  const double *rec = b.rec + (size_t)half * n * b.rs;
+  const double *reci = rec + (size_t)i * b.rs;
   const double xi = reci[0], yi = reci[1], zi = reci[2];
   int *nj = b.nbr_j + (size_t)i * b.maxnb;
   int *nc = b.nbr_code + (size_t)i * b.maxnb;
-  const int m = b.scan ? scan_row<BOX>(g, b, i, lane, xi, yi, zi, nj, nc)
-                       : cell_row<BOX>(g, b, parity, i, lane, xi, yi, zi, s_beg, s_pre, s_sort, nj,
-                                       nc);
+  const int m = b.scan ? scan_row<BOX>(g, b, b.comp + (size_t)3 * half * n, i, lane, xi, yi, zi, nj,
+                                       nc)
+                       : cell_row<BOX>(g, b, rec, list, i, lane, xi, yi, zi, s_sort, nj, nc);
   wsync();  // the force loop reads entries other lanes wrote
   if (lane == 0) {
     b.nbr_cnt[i] = m;
@@ -751,145 +764,196 @@ __device__ inline int build_row(const Geom &g, const MdBuf &b, int parity, int i
   return m;
 }
 
+// The pair forces on molecule i by its wave: its row is rebuilt if a rebuild
+// is due, the row's pairs within rc are compacted into the wave's LDS region
+// `reg`, then evaluated.  The results are each lane's sums over its own pairs
+// (two or three in a liquid) in the pair precision.
+template <typename R>
+struct PairOut {
+  R F[3], T[3], e, v[9];
+  int npair, nlist;  // wave-uniform counts
+};
+template <int M, typename R, int BOX, class Mid>
+__device__ __forceinline__ void pair_phase(const Geom &g, const MdBuf &b, const PairK<R> &pk,
+                                           int rebuild, int list, int half, int i, int lane,
+                                           unsigned char *reg, PairOut<R> &o, Mid &&mid) {
+  using T = Traits<M>;
+  const int cap = b.maxnb;
+  const BoxNow bl = box_now<BOX>(g, b);
+  const double *rec = b.rec + (size_t)half * g.n * b.rs;
+  const int *nj = b.nbr_j + (size_t)i * cap;
+  const int *nc = b.nbr_code + (size_t)i * cap;
+  constexpr int kIdle = 512 | (512 << 10) | (512 << 20);  // zero shift
+  // the first round of row entries is fetched with the row length (or
+  // right after a rebuild)
+  int jj[4], cc[4];
+  int m;
+  if (rebuild) {
+    m = build_row<BOX>(g, b, list, half, i, lane, reinterpret_cast<int *>(reg));
+    o.nlist = m;
+  } else {
+    m = b.nbr_cnt[i];
+  }
+#pragma unroll
+  for (int u = 0; u < 4; u++) {
+    const int k = 64 * u + lane;
+    jj[u] = k < cap ? nj[k] : i;
+    cc[u] = k < cap ? nc[k] : kIdle;
+  }
+  // entries at or past the row length hold stale or never-written values:
+  // they are replaced before any of them forms an address
+#pragma unroll
+  for (int u = 0; u < 4; u++) {
+    if (64 * u + lane >= m) {
+      jj[u] = i;
+      cc[u] = kIdle;
+    }
+  }
+  const double *reci = rec + (size_t)i * b.rs;
+  const double xi = reci[0], yi = reci[1], zi = reci[2];
+  // pass 1: the reference's FP64 interaction test on every row entry; the
+  // entries that pass are compacted in row order into LDS
+  int *cj = reinterpret_cast<int *>(reg);
+  R *dv = reinterpret_cast<R *>(reg + (4 * cap + 15) / 16 * 16);
+  const int dstride = (int)(((size_t)cap * sizeof(R) + 15) / 16 * 16 / sizeof(R));
+  wsync();  // the sort buffers of build_row share this region
+  int np = 0;
+  // four entries per lane per round: the index loads, then the record
+  // loads, are in flight together
+  for (int k0 = 0; k0 < m; k0 += 256) {
+    if (k0 > 0) {
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        const int k = k0 + 64 * u + lane;
+        jj[u] = k < m ? nj[k] : i;
+        cc[u] = k < m ? nc[k] : kIdle;
+      }
+    }
+    double xj[4], yj[4], zj[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const double *recj = rec + (size_t)jj[u] * b.rs;
+      xj[u] = recj[0];
+      yj[u] = recj[1];
+      zj[u] = recj[2];
+    }
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const int code = cc[u];
+      const double ox = (double)((code & 1023) - 512) * bl.L[0];
+      const double oy = (double)(((code >> 10) & 1023) - 512) * bl.L[1];
+      const double oz = (double)(((code >> 20) & 1023) - 512) * bl.L[2];
+      const double d0 = (xi - xj[u]) - ox;
+      const double d1 = (yi - yj[u]) - oy;
+      const double d2 = (zi - zj[u]) - oz;
+      const bool pass = k0 + 64 * u + lane < m && d0 * d0 + d1 * d1 + d2 * d2 < g.rc2;
+      const unsigned long long mask = __ballot(pass);
+      if (pass) {
+        const int pos = np + __popcll(mask & ((1ull << lane) - 1ull));
+        cj[pos] = jj[u];
+        dv[pos] = R(d0);
+        dv[dstride + pos] = R(d1);
+        dv[2 * dstride + pos] = R(d2);
+      }
+      np += __popcll(mask);
+    }
+  }
+  o.npair = np;
+  mid();
+  wsync();
+  // pass 2: the interacting pairs, densely, two per lane per round
+  R ri[T::NS][3];
+  RecSites<M, R>::load(reci, ri);
+  R(&Fr)[3] = o.F;
+  R(&Tr)[3] = o.T;
+  R(&vr)[9] = o.v;
+  auto eval = [&](int j, R d0, R d1, R d2, const R (&rj)[T::NS][3]) {
+    R Fp[3], Tp[3];
+    const R e = pair_on_i<M, R>(pk, d0 * d0 + d1 * d1 + d2 * d2, d0, d1, d2, ri, rj, Fp, Tp);
+    Fr[0] += Fp[0]; Fr[1] += Fp[1]; Fr[2] += Fp[2];
+    Tr[0] += Tp[0]; Tr[1] += Tp[1]; Tr[2] += Tp[2];
+    o.e += e;
+    // pair virial d (x) F, fused multiply-adds
+    const R dd3[3] = {d0, d1, d2};
+#pragma unroll
+    for (int a = 0; a < 3; a++)
+#pragma unroll
+      for (int c = 0; c < 3; c++) vr[3 * a + c] = fma_r(dd3[a], Fp[c], vr[3 * a + c]);
+  };
+  for (int k0 = 0; k0 < np; k0 += 128) {
+    const int ka = k0 + lane, kb = k0 + 64 + lane;
+    const int ja = ka < np ? cj[ka] : i, jb = kb < np ? cj[kb] : i;
+    R ra[T::NS][3], rb[T::NS][3];
+    RecSites<M, R>::load(rec + (size_t)ja * b.rs, ra);
+    RecSites<M, R>::load(rec + (size_t)jb * b.rs, rb);
+    if (ka < np) eval(ja, dv[ka], dv[dstride + ka], dv[2 * dstride + ka], ra);
+    if (kb < np) eval(jb, dv[kb], dv[dstride + kb], dv[2 * dstride + kb], rb);
+  }
+}
+
+template <typename R>
+__device__ inline void pair_zero(PairOut<R> &o) {
+#pragma unroll
+  for (int a = 0; a < 3; a++) o.F[a] = o.T[a] = R(0);
+  o.e = R(0);
+#pragma unroll
+  for (int q = 0; q < 9; q++) o.v[q] = R(0);
+  o.npair = o.nlist = 0;
+}
+
+// each lane's energy and virial into its wave's LDS region [10][64], which
+// the compacted entries no longer need
+template <typename R>
+__device__ inline void park_sums(const PairOut<R> &o, unsigned char *reg, int lane,
+                                 double (&s_cnt)[2]) {
+  double *acc = reinterpret_cast<double *>(reg);
+  acc[lane] = (double)o.e;
+#pragma unroll
+  for (int q = 0; q < 9; q++) acc[(1 + q) * 64 + lane] = (double)o.v[q];
+  if (lane == 0) {
+    s_cnt[0] = (double)o.npair;
+    s_cnt[1] = (double)o.nlist;
+  }
+}
+// block partial of quantity q (energy, virial) from the parked lanes, in a
+// fixed order: thread (q, seg) sums lanes seg, seg+16, ... of the 256 (for
+// each u the 16 threads of a DPP row read 16 consecutive doubles: no bank
+// conflict), compensated (TwoSum over the 16 terms and the row), halved
+// (every pair is met from both sides)
+__device__ inline void block_sum(const unsigned char *s_dyn, int reg_bytes, int q, int seg,
+                                 double *out) {
+  double r = 0.0, rc = 0.0;
+#pragma unroll
+  for (int u = 0; u < 16; u++) {
+    const int L = seg + 16 * u;
+    two_sum_acc(r, rc,
+                reinterpret_cast<const double *>(s_dyn + (size_t)(L >> 6) * reg_bytes)[q * 64 + (L & 63)]);
+  }
+  rowsum16_dd(r, rc);
+  if (seg == 0) out[q] = 0.5 * (r + rc);
+}
+
 // blk is the block's index within its system and nblk the system's block
 // count (blockIdx.x and gridDim.x for one system).
 template <int M, typename R, int BOX>
-__device__ __forceinline__ void md_main_body(const ModelTable &mt, const Geom &g, const MdBuf &b,
-                                             const PairK<R> &pk, double *out, int parity,
-                                             const CloseArgs &ca, int reg_bytes, int blk,
+__device__ __forceinline__ void md_main_body(const Geom &g, const MdBuf &b, const PairK<R> &pk,
+                                             double *out, int parity, int reg_bytes, int blk,
                                              int nblk) {
-  using T = Traits<M>;
   extern __shared__ __align__(16) unsigned char s_dyn[];  // [4][reg_bytes]
-  __shared__ int s_beg[4][128], s_pre[4][132];
   __shared__ double s_cnt[4][2];
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int n = g.n;
   const int i = blk * 4 + wid;
-  const int cap = b.maxnb;
-  const BoxNow bl = box_now<BOX>(g, b);
   unsigned char *reg = s_dyn + (size_t)wid * reg_bytes;
-  double ep = 0, v[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-  int npair = 0, nlist = 0;  // wave-uniform counts
+  PairOut<R> o;
+  pair_zero(o);
   if (i < n) {
-    const int *nj = b.nbr_j + (size_t)i * cap;
-    const int *nc = b.nbr_code + (size_t)i * cap;
-    constexpr int kIdle = 512 | (512 << 10) | (512 << 20);  // zero shift
-    // the first round of row entries is fetched with the row length (or
-    // right after a rebuild)
-    int jj[4], cc[4];
-    int m;
-    if (b.flags[2 + parity]) {
-      m = build_row<BOX>(g, b, parity, i, lane, s_beg[wid], s_pre[wid],
-                         reinterpret_cast<int *>(reg));
-      nlist = m;
-    } else {
-      m = b.nbr_cnt[i];
-    }
-#pragma unroll
-    for (int u = 0; u < 4; u++) {
-      const int k = 64 * u + lane;
-      jj[u] = k < cap ? nj[k] : i;
-      cc[u] = k < cap ? nc[k] : kIdle;
-    }
-    // entries at or past the row length hold stale or never-written values:
-    // they are replaced before any of them forms an address
-#pragma unroll
-    for (int u = 0; u < 4; u++) {
-      if (64 * u + lane >= m) {
-        jj[u] = i;
-        cc[u] = kIdle;
-      }
-    }
-    const double *reci = b.rec + (size_t)i * b.rs;
-    const double xi = reci[0], yi = reci[1], zi = reci[2];
-    // pass 1: the reference's FP64 interaction test on every row entry; the
-    // entries that pass are compacted in row order into LDS
-    int *cj = reinterpret_cast<int *>(reg);
-    R *dv = reinterpret_cast<R *>(reg + (4 * cap + 15) / 16 * 16);
-    const int dstride = (int)(((size_t)cap * sizeof(R) + 15) / 16 * 16 / sizeof(R));
-    wsync();  // the sort buffers of build_row share this region
-    int np = 0;
-    // four entries per lane per round: the index loads, then the record
-    // loads, are in flight together
-    for (int k0 = 0; k0 < m; k0 += 256) {
-      if (k0 > 0) {
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-          const int k = k0 + 64 * u + lane;
-          jj[u] = k < m ? nj[k] : i;
-          cc[u] = k < m ? nc[k] : kIdle;
-        }
-      }
-      double xj[4], yj[4], zj[4];
-#pragma unroll
-      for (int u = 0; u < 4; u++) {
-        const double *recj = b.rec + (size_t)jj[u] * b.rs;
-        xj[u] = recj[0];
-        yj[u] = recj[1];
-        zj[u] = recj[2];
-      }
-#pragma unroll
-      for (int u = 0; u < 4; u++) {
-        const int code = cc[u];
-        const double ox = (double)((code & 1023) - 512) * bl.L[0];
-        const double oy = (double)(((code >> 10) & 1023) - 512) * bl.L[1];
-        const double oz = (double)(((code >> 20) & 1023) - 512) * bl.L[2];
-        const double d0 = (xi - xj[u]) - ox;
-        const double d1 = (yi - yj[u]) - oy;
-        const double d2 = (zi - zj[u]) - oz;
-        const bool pass = k0 + 64 * u + lane < m && d0 * d0 + d1 * d1 + d2 * d2 < g.rc2;
-        const unsigned long long mask = __ballot(pass);
-        if (pass) {
-          const int pos = np + __popcll(mask & ((1ull << lane) - 1ull));
-          cj[pos] = jj[u];
-          dv[pos] = R(d0);
-          dv[dstride + pos] = R(d1);
-          dv[2 * dstride + pos] = R(d2);
-        }
-        np += __popcll(mask);
-      }
-    }
-    npair = np;
-    wsync();
-    // pass 2: the interacting pairs, densely, two per lane per round
-    R ri[T::NS][3];
-    RecSites<M, R>::load(reci, ri);
-    // each lane's own pairs (two or three in a liquid) are summed in the pair
-    // precision; the lane totals then go to FP64 for the wave and block sums
-    R Fr[3] = {R(0), R(0), R(0)}, Tr[3] = {R(0), R(0), R(0)}, er = R(0);
-    R vr[9];
-#pragma unroll
-    for (int q = 0; q < 9; q++) vr[q] = R(0);
-    auto eval = [&](int j, R d0, R d1, R d2, const R (&rj)[T::NS][3]) {
-      R Fp[3], Tp[3];
-      const R e = pair_on_i<M, R>(pk, d0 * d0 + d1 * d1 + d2 * d2, d0, d1, d2, ri, rj, Fp, Tp);
-      Fr[0] += Fp[0]; Fr[1] += Fp[1]; Fr[2] += Fp[2];
-      Tr[0] += Tp[0]; Tr[1] += Tp[1]; Tr[2] += Tp[2];
-      er += e;
-      // pair virial d (x) F, fused multiply-adds
-      const R dd3[3] = {d0, d1, d2};
-#pragma unroll
-      for (int a = 0; a < 3; a++)
-#pragma unroll
-        for (int c = 0; c < 3; c++) vr[3 * a + c] = fma_r(dd3[a], Fp[c], vr[3 * a + c]);
-    };
-    for (int k0 = 0; k0 < np; k0 += 128) {
-      const int ka = k0 + lane, kb = k0 + 64 + lane;
-      const int ja = ka < np ? cj[ka] : i, jb = kb < np ? cj[kb] : i;
-      R ra[T::NS][3], rb[T::NS][3];
-      RecSites<M, R>::load(b.rec + (size_t)ja * b.rs, ra);
-      RecSites<M, R>::load(b.rec + (size_t)jb * b.rs, rb);
-      if (ka < np) eval(ja, dv[ka], dv[dstride + ka], dv[2 * dstride + ka], ra);
-      if (kb < np) eval(jb, dv[kb], dv[dstride + kb], dv[2 * dstride + kb], rb);
-    }
+    pair_phase<M, R, BOX>(g, b, pk, b.flags[2 + parity], parity, 0, i, lane, reg, o, [] {});
     double F[3], Ti[3];
-    ep = (double)er;
-#pragma unroll
-    for (int q = 0; q < 9; q++) v[q] = (double)vr[q];
 #pragma unroll
     for (int a = 0; a < 3; a++) {
-      F[a] = wsum63((double)Fr[a]);
-      Ti[a] = wsum63((double)Tr[a]);
+      F[a] = wsum63((double)o.F[a]);
+      Ti[a] = wsum63((double)o.T[a]);
     }
     if (lane == 63) {
       if (out) {
@@ -910,38 +974,16 @@ __device__ __forceinline__ void md_main_body(const ModelTable &mt, const Geom &g
         }
       }
     }
-    wsync();  // the compacted entries are dead; the region takes the partials
+    wsync();  // every lane has read the compacted entries
   }
-  // block partials in a fixed order: each wave's lane partials of energy
-  // and virial go to its LDS region, 16 lanes per row then sum 16 entries
-  // each, and the row sums are combined
-  double *acc = reinterpret_cast<double *>(reg);  // [10][64] of this wave
-  acc[lane] = ep;
-#pragma unroll
-  for (int q = 0; q < 9; q++) acc[(1 + q) * 64 + lane] = v[q];
-  if (lane == 0) {
-    s_cnt[wid][0] = (double)npair;
-    s_cnt[wid][1] = (double)nlist;
-  }
+  park_sums(o, reg, lane, s_cnt[wid]);
   __syncthreads();
+  double *part = b.blockpart + ((size_t)parity * nblk + blk) * kBP;
   if (threadIdx.x < 160) {
-    // thread (q, seg) sums lanes seg, seg+16, ... of the 256: for each u the
-    // 16 threads of a DPP row read 16 consecutive doubles (no bank conflict)
-    // (compensated: TwoSum over the 16 terms and the row)
-    const int q = threadIdx.x >> 4, seg = threadIdx.x & 15;
-    double r = 0.0, rc = 0.0;
-#pragma unroll
-    for (int u = 0; u < 16; u++) {
-      const int L = seg + 16 * u;
-      two_sum_acc(r, rc,
-                  reinterpret_cast<const double *>(s_dyn + (size_t)(L >> 6) * reg_bytes)[q * 64 + (L & 63)]);
-    }
-    rowsum16_dd(r, rc);
-    if (seg == 0) b.blockpart[((size_t)parity * nblk + blk) * kBP + q] = 0.5 * (r + rc);
+    block_sum(s_dyn, reg_bytes, threadIdx.x >> 4, threadIdx.x & 15, part);
   } else if (threadIdx.x < 162) {
     const int q = threadIdx.x - 160;
-    b.blockpart[((size_t)parity * nblk + blk) * kBP + 10 + q] =
-        0.5 * (s_cnt[0][q] + s_cnt[1][q] + s_cnt[2][q] + s_cnt[3][q]);
+    part[10 + q] = 0.5 * (s_cnt[0][q] + s_cnt[1][q] + s_cnt[2][q] + s_cnt[3][q]);
   }
 }
 
@@ -956,52 +998,541 @@ constexpr int main_waves_per_eu() {
   return (M != G6_ST2 && M != G6_NVDE && sizeof(R) == 4) ? 4 : 1;
 }
 
+// ---- the step kernel ---------------------------------------------------------
+// One kernel per step of a fixed-box system on the rows: the pair forces of
+// step q at the predicted positions, the corrector of the block's four
+// molecules with the Nose drag, and their predictor, records, binning and
+// skin test for step q + 1.  A step of two kernels (predictor and forces) at
+// 4096 molecules spent 6 us in the per-molecule kernel, which is latency
+// alone, and a launch boundary between them.
+//
+// The corrector needs zeta of this step, that is, the whole system's kinetic
+// energy of the step before.  That step's kernel left the kinetic energy of
+// every block of four molecules, and every block sums them again, in the same
+// order, in the shadow of its pair phase: 1024 values at 4096 molecules.  No
+// block waits for another.
+//
+// Buffers alternate so that no block writes what another may still read:
+// records, scanned COMs, the thermostat state and the partials by parity,
+// cell lists and rebuild flags in threes (read, filled, cleared).
+//
+// Roles after the pair phase, 16 lanes each (a quad per molecule, a lane per
+// component): wave 0 translation, binning and skin test; wave 1 angular
+// velocity; wave 2 quaternions, rotation and site offsets; wave 3 kinetic
+// sums; waves 1 to 3 the block's energy and virial sums.  Every component
+// keeps md_pre_body's operation order, which is the reference's, so the
+// states are the same bits as the two-kernel step's.
+
+struct StepArgs {
+  int parity;       // of this step's records, partials and thermostat state
+  int list;         // cell list and rebuild flag of this step
+  int first, last;  // no step before (the thermostat state is this step's) / after
+  int nose_active;
+  double dt;
+};
+
+// blk: the index of the block's four molecules, one per wave; nblk: the
+// system's blocks.
 template <int M, typename R, int BOX>
-__global__ __launch_bounds__(256, (main_waves_per_eu<M, R>())) void k_md_main(ModelTable mt, Geom g, MdBuf b, PairK<R> pk,
-                                                 double *out, int parity, CloseArgs ca,
-                                                 int reg_bytes) {
-  if (ca.mode) {
-    // block 0 closes the previous step while the other blocks run the rows
-    if (blockIdx.x == 0) {
-      __shared__ double s_close[4][kRed];
-      close_body<false>(mt, b, g.n, ca.dt, ca.nblk_pre, ca.bpart, ca.nblk_main, g.ncell,
-                        ca.nose_active, ca.mode, parity, box_volume(g.L), s_close);
-      return;
+__device__ __forceinline__ void md_step_body(const ModelTable &mt, const Geom &g, const MdBuf &b,
+                                             const PairK<R> &pk, const StepArgs &st, int reg_bytes,
+                                             int blk, int nblk) {
+  extern __shared__ __align__(16) unsigned char s_dyn[];  // [4][reg_bytes]
+  __shared__ double s_cnt[4][2], s_kin[4], s_z[9];
+  __shared__ double s_st[kStateRows * 4];   // the Gear state of the block's molecules
+  __shared__ double s_ft[4][6];             // force and lab torque
+  __shared__ double s_v[4][3], s_W[4][12];  // corrected dx(1) and w levels 0..3
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int n = g.n;
+  const int par = st.parity;
+  const int rebuild = b.flags[2 + st.list];
+  // What the corrector reads - the state block's columns of the molecules, the
+  // kinetic energies and the thermostat state of the step before - is fetched
+  // ahead of the pairs and parked in LDS once the row has been tested: each
+  // block starts on cold caches, and a load after the pairs would add a
+  // memory latency to the step (4096 molecules: 0.8 us of 19).
+  const bool kin_sum = st.nose_active && !st.first;
+  const double *kin_in = b.stepkin + (size_t)(1 - par) * nblk;
+  double pst, pkin[4], pz = 0.0;
+  {
+    const int row = threadIdx.x >> 2, i = blk * 4 + (threadIdx.x & 3);
+    pst = row < kStateRows && i < n ? b.com[(size_t)row * n + i] : 0.0;
+  }
+#pragma unroll
+  for (int u = 0; u < 4; u++) {
+    const int k = threadIdx.x + 256 * u;
+    pkin[u] = kin_sum && k < nblk ? kin_in[k] : 0.0;
+  }
+  if (threadIdx.x < 9) pz = b.nose[9 * (st.first ? par : 1 - par) + threadIdx.x];
+  auto park = [&]() {
+    if (threadIdx.x < kStateRows * 4) s_st[threadIdx.x] = pst;
+    if (threadIdx.x < 9) s_z[threadIdx.x] = pz;
+    if (kin_sum) {
+      double s = 0.0;
+#pragma unroll
+      for (int u = 0; u < 4; u++) s += pkin[u];
+#pragma unroll 4
+      for (int k = threadIdx.x + 1024; k < nblk; k += 256) s += kin_in[k];
+      s = wsum63(s);
+      if (lane == 63) s_kin[wid] = s;
     }
-    md_main_body<M, R, BOX>(mt, g, b, pk, out, parity, ca, reg_bytes, blockIdx.x - 1,
-                            gridDim.x - 1);
+  };
+  unsigned char *reg = s_dyn + (size_t)wid * reg_bytes;
+  PairOut<R> o;
+  pair_zero(o);
+  if (blk * 4 + wid < n)
+    pair_phase<M, R, BOX>(g, b, pk, rebuild, st.list, par, blk * 4 + wid, lane, reg, o, park);
+  else
+    park();
+  double F[3], Ti[3];
+#pragma unroll
+  for (int c = 0; c < 3; c++) {
+    F[c] = wsum63((double)o.F[c]);
+    Ti[c] = wsum63((double)o.T[c]);
+  }
+  if (lane == 63) {
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+      s_ft[wid][c] = F[c];
+      s_ft[wid][3 + c] = Ti[c];
+    }
+  }
+  wsync();  // every lane has read the compacted entries
+  park_sums(o, reg, lane, s_cnt[wid]);
+  __syncthreads();
+  double *part = b.blockpart + ((size_t)par * nblk + blk) * kBP;
+
+  // lane m * 4 + a holds component a of molecule m
+  const int m = (lane >> 2) & 3, a = lane & 3;
+  const int i = blk * 4 + m;
+  const bool ok = lane < 16 && i < n;
+  const int ax = a < 3 ? a : 0;
+  double S[6], X[4], cref = 0.0;
+#pragma unroll
+  for (int k = 0; k < 6; k++) S[k] = 0.0;
+#pragma unroll
+  for (int k = 0; k < 4; k++) X[k] = 0.0;
+  auto state = [&](int row) { return s_st[row * 4 + m]; };
+  if (wid == 0) {
+#pragma unroll
+    for (int k = 0; k < 6; k++) S[k] = state(3 * k + ax);  // com, dx levels
+    cref = state(kRowRef + ax);
+  } else if (wid == 1) {
+#pragma unroll
+    for (int k = 0; k < 5; k++) S[k] = state(kRowW + 3 * k + ax);
+#pragma unroll
+    for (int c = 0; c < 4; c++) X[c] = state(kRowQ + c);
+  } else if (wid == 2) {
+#pragma unroll
+    for (int k = 0; k < 5; k++) S[k] = state(kRowQ + 4 * k + a);
+#pragma unroll
+    for (int c = 0; c < 3; c++) X[c] = state(kRowW + c);
+  }
+  const int rs = b.rs;
+  double *rec = b.rec + (size_t)(1 - par) * n * rs;  // the next step's records
+  double *com = b.com;
+  const double dt = st.dt;
+  if (wid < 2) {
+    // zeta of this step: the state of the step before, corrected with its
+    // temperature and predicted (the step close stores the same values)
+    double zeta0 = 0.0;
+    if (st.nose_active) {
+      double z[9];
+#pragma unroll
+      for (int q = 0; q < 9; q++) z[q] = s_z[q];
+      if (!st.first) {
+        const double ek = s_kin[0] + s_kin[1] + s_kin[2] + s_kin[3];
+        nose_correct(z, temperature_of(ek, n));
+        nose_predict(z);
+      }
+      zeta0 = z[3];
+    }
+    const double nc = zeta0 * dt;
+    if (wid == 0) {
+      if (!ok || a == 3) {
+        // idle lanes and the quads' fourth lanes carry zeros
+      } else {
+        const double tf = dt * dt * 0.5 * mt.inv_mass;
+        double nf = s_ft[m][a] * tf;
+        nf = nf - S[1] * (nc * 0.5);
+        const double d = nf - S[2];
+        if (rebuild) cref = S[0];  // the rows of this step were built here
+        S[0] = S[0] + kG5_0 * d;
+        S[1] = S[1] + kG5_1 * d;
+        S[2] = nf;
+        S[3] = S[3] + kG5_3 * d;
+        S[4] = S[4] + kG5_4 * d;
+        S[5] = S[5] + kG5_5 * d;
+      }
+      if (lane < 16 && a < 3) s_v[m][a] = S[1];
+    } else {
+      // rigid_collectforce's body-frame torque with the rotation matrix of
+      // the predicted orientation
+      const double qa = X[0], qb = X[1], qc = X[2], qd = X[3];
+      double t[3];  // column a
+      if (a == 0) {
+        t[0] = (qa * qa + qb * qb - (qc * qc + qd * qd));
+        t[1] = 2.0 * (qa * qd - qb * qc);
+        t[2] = 2.0 * (qa * qc + qb * qd);
+      } else if (a == 1) {
+        t[0] = -2.0 * (qa * qd + qb * qc);
+        t[1] = qa * qa + qc * qc - (qb * qb + qd * qd);
+        t[2] = 2.0 * (qa * qb - qc * qd);
+      } else {
+        t[0] = 2.0 * (qb * qd - qa * qc);
+        t[1] = -2.0 * (qa * qb + qc * qd);
+        t[2] = qa * qa + qd * qd - (qb * qb + qc * qc);
+      }
+      const double tq = t[0] * s_ft[m][3] + t[1] * s_ft[m][4] + t[2] * s_ft[m][5];
+      const double di = a == 0 ? mt.Iyy - mt.Izz : a == 1 ? mt.Izz - mt.Ixx : mt.Ixx - mt.Iyy;
+      const double ii = a == 0 ? mt.inv_ixx : a == 1 ? mt.inv_iyy : mt.inv_izz;
+      const double w1 = dpp_d<0xC9>(S[0]);  // lanes a + 1 and a + 2 of the three
+      const double w2 = dpp_d<0xD2>(S[0]);
+      if (ok && a < 3) {
+        double nf = (tq + di * w1 * w2) * dt * ii;
+        nf = nf - S[0] * nc;
+        const double d = nf - S[1];
+        S[0] = S[0] + kG4_0 * d;
+        S[1] = nf;
+        S[2] = S[2] + kG4_2 * d;
+        S[3] = S[3] + kG4_3 * d;
+        S[4] = S[4] + kG4_4 * d;
+      }
+      if (lane < 16 && a < 3)
+#pragma unroll
+        for (int k = 0; k < 4; k++) s_W[m][3 * k + a] = S[k];
+    }
   } else {
-    md_main_body<M, R, BOX>(mt, g, b, pk, out, parity, ca, reg_bytes, blockIdx.x, gridDim.x);
+    block_sum(s_dyn, reg_bytes, 4 * (wid - 2) + (lane >> 4), lane & 15, part);
+  }
+  // quaternion corrector of level 0 (with the uncorrected w).  Component a
+  // of a product with (wx, wy, wz) is -+wx q(a^1) -+ wy q(a^2) -+ wz q(a^3)
+  const double sx = (a & 1) ? 1.0 : -1.0, sy = (a == 0 || a == 3) ? 1.0 : -1.0,
+               sz = a >= 2 ? 1.0 : -1.0;
+  auto turn3 = [](double wx, double wy, double wz, double q1, double q2, double q3) {
+    return wx * q1 + wy * q2 + wz * q3;
+  };
+  if (wid == 2) {
+    const double nw = turn3(sx * X[0], sy * X[1], sz * X[2], dpp_d<0xB1>(S[0]), dpp_d<0x4E>(S[0]),
+                            dpp_d<0x1B>(S[0])) * dt * 0.5;
+    S[0] = S[0] + kG4_0 * (nw - S[1]);
+  }
+  __syncthreads();
+
+  if (wid == 0) {
+    if (!st.last && ok && a < 3) {
+      S[0] = S[0] + S[1] + S[2] + S[3] + S[4] + S[5];
+      S[1] = S[1] + 2.0 * S[2] + 3.0 * S[3] + 4.0 * S[4] + 5.0 * S[5];
+      S[2] = S[2] + 3.0 * S[3] + 6.0 * S[4] + 10.0 * S[5];
+      S[3] = S[3] + 4.0 * S[4] + 10.0 * S[5];
+      S[4] = S[4] + 5.0 * S[5];
+    }
+    if (ok && a < 3)
+#pragma unroll
+      for (int k = 0; k < 6; k++) com[(size_t)(3 * k + a) * n + i] = S[k];
+    if (!st.last) {
+      const bool scan = b.scan != 0;
+      const int nl = st.list == 2 ? 0 : st.list + 1;  // the next step's list
+      if (ok && a < 3) {
+        rec[(size_t)i * rs + a] = S[0];
+        if (scan) b.comp[(3 * (1 - par) + a) * n + i] = S[0];
+      }
+      if (!scan) {
+        const int e = BOX == kBoxCube ? 0 : ax;
+        const double L = g.L[e], invL = g.invL[e], ci = g.cellinv[e];
+        const int nda = g.nd[e];
+        double d = S[0];
+        const double os = round(d * invL) * L;
+        d = d - os;
+        int j = (int)round(d * ci);
+        if (j < 0) j += nda;
+        j = ((j % nda) + nda) % nda;
+        const int j0 = __builtin_amdgcn_mov_dpp(j, 0x00, 0xF, 0xF, false);
+        const int j1 = __builtin_amdgcn_mov_dpp(j, 0x55, 0xF, 0xF, false);
+        const int j2 = __builtin_amdgcn_mov_dpp(j, 0xAA, 0xF, 0xF, false);
+        if (ok && a == 0) {
+          const int c = (j2 * g.nd[BOX == kBoxCube ? 0 : 1] + j1) * g.nd[0] + j0;
+          b.cell[i] = c;
+          const int cap = b.cell_cap;
+          int *cr = b.cellres + ((size_t)nl * g.ncell + c) * cap;
+          const int slot = atomicAdd(cr, 1) + 1;
+          if (slot < cap)
+            cr[slot] = i;
+          else
+            raise_flag(b.flags, 3);  // cell capacity exceeded
+        }
+      }
+      const double h2 = b.half_skin2;
+      if (h2 > 0.0) {
+        const double e = S[0] - cref, ee = e * e;
+        const double e0 = quad_d<0>(ee), e1 = quad_d<1>(ee), e2 = quad_d<2>(ee);
+        if (ok && a == 0 && e0 + e1 + e2 > h2) b.flags[2 + nl] = 1;
+      } else if (ok && a == 0 && i == 0) {
+        b.flags[2 + nl] = 1;  // no skin: the reference rebuilds every step
+      }
+    }
+  } else if (wid == 1) {
+    if (!st.last && ok && a < 3) {
+      S[0] = S[0] + S[1] + S[2] + S[3] + S[4];
+      S[1] = S[1] + 2.0 * S[2] + 3.0 * S[3] + 4.0 * S[4];
+      S[2] = S[2] + 3.0 * S[3] + 6.0 * S[4];
+      S[3] = S[3] + 4.0 * S[4];
+    }
+    if (ok && a < 3)
+#pragma unroll
+      for (int k = 0; k < 5; k++) com[(size_t)(kRowW + 3 * k + a) * n + i] = S[k];
+    // the last two energy and virial sums (rows of 16 lanes) and the counts
+    if (lane < 32) block_sum(s_dyn, reg_bytes, 8 + (lane >> 4), lane & 15, part);
+    else if (lane < 34) {
+      const int q = lane - 32;
+      part[10 + q] = 0.5 * (s_cnt[0][q] + s_cnt[1][q] + s_cnt[2][q] + s_cnt[3][q]);
+    }
+  } else if (wid == 2) {
+    // quaternion derivatives from the corrected w: level k + 1 of component
+    // a from the lower levels' partner components
+    double w1[3], w2[3], w3[3], w4[3];
+    {
+      const double sg[3] = {sx, sy, sz};
+#pragma unroll
+      for (int c = 0; c < 3; c++) {
+        w1[c] = sg[c] * s_W[m][c];
+        w2[c] = sg[c] * s_W[m][3 + c];
+        w3[c] = sg[c] * s_W[m][6 + c];
+        w4[c] = sg[c] * s_W[m][9 + c];
+      }
+    }
+    const double q1 = dpp_d<0xB1>(S[0]), q2 = dpp_d<0x4E>(S[0]), q3 = dpp_d<0x1B>(S[0]);
+    const double p = (w1[0] * q1 + w1[1] * q2 + w1[2] * q3) * dt * 0.5;
+    const double p1 = dpp_d<0xB1>(p), p2 = dpp_d<0x4E>(p), p3 = dpp_d<0x1B>(p);
+    const double r = (w2[0] * q1 + w2[1] * q2 + w2[2] * q3 + w1[0] * p1 + w1[1] * p2 + w1[2] * p3) *
+                     dt * 0.25;
+    const double r1 = dpp_d<0xB1>(r), r2 = dpp_d<0x4E>(r), r3 = dpp_d<0x1B>(r);
+    const double s = (w3[0] * q1 + w3[1] * q2 + w3[2] * q3 + w1[0] * r1 + w1[1] * r2 + w1[2] * r3 +
+                      w2[0] * p1 + w2[1] * p2 + w2[2] * p3) * dt * (1.0 / 6.0);
+    const double s1 = dpp_d<0xB1>(s), s2 = dpp_d<0x4E>(s), s3 = dpp_d<0x1B>(s);
+    const double u = (w4[0] * q1 + w4[1] * q2 + w4[2] * q3 + w3[0] * p1 + w3[1] * p2 + w3[2] * p3 +
+                      w2[0] * r1 + w2[1] * r2 + w2[2] * r3 + w1[0] * s1 + w1[1] * s2 + w1[2] * s3) *
+                     dt * (1.0 / 8.0);
+    S[1] = p;
+    S[2] = r;
+    S[3] = s;
+    S[4] = u;
+    if (!st.last) {
+      S[0] = S[0] + S[1] + S[2] + S[3] + S[4];
+      S[1] = S[1] + 2.0 * S[2] + 3.0 * S[3] + 4.0 * S[4];
+      double qa = quad_d<0>(S[0]), qb = quad_d<1>(S[0]), qc = quad_d<2>(S[0]),
+             qd = quad_d<3>(S[0]);
+      const double re = 1.0 / sqrt(qa * qa + qb * qb + qc * qc + qd * qd);
+      qa = qa * re;
+      qb = qb * re;
+      qc = qc * re;
+      qd = qd * re;
+      S[0] = S[0] * re;
+      double t[9];
+      t[0] = (qa * qa + qb * qb - (qc * qc + qd * qd));
+      t[1] = -2.0 * (qa * qd + qb * qc);
+      t[2] = 2.0 * (qb * qd - qa * qc);
+      t[3] = 2.0 * (qa * qd - qb * qc);
+      t[4] = qa * qa + qc * qc - (qb * qb + qd * qd);
+      t[5] = -2.0 * (qa * qb + qc * qd);
+      t[6] = 2.0 * (qa * qc + qb * qd);
+      t[7] = 2.0 * (qa * qb - qc * qd);
+      t[8] = qa * qa + qd * qd - (qb * qb + qc * qc);
+      // lane a places sites a and a + 4
+      const int nq = mt.nsite - 1;
+#pragma unroll
+      for (int k = 0; k < 2; k++) {
+        const int q = 4 * k + a;
+        if (!ok || q >= nq) continue;
+        const double bx = mt.bx[q], by = mt.by[q], bz = mt.bz[q];
+        const double r0 = t[0] * bx + t[1] * by + t[2] * bz;
+        const double r1 = t[3] * bx + t[4] * by + t[5] * bz;
+        const double r2 = t[6] * bx + t[7] * by + t[8] * bz;
+        double *ri = rec + (size_t)i * rs + 4;
+        if (sizeof(R) == 4) {
+          float *rf = reinterpret_cast<float *>(ri) + 3 * q;
+          rf[0] = (float)r0;
+          rf[1] = (float)r1;
+          rf[2] = (float)r2;
+        } else {
+          ri[3 * q] = r0;
+          ri[3 * q + 1] = r1;
+          ri[3 * q + 2] = r2;
+        }
+      }
+    }
+    if (ok)
+#pragma unroll
+      for (int k = 0; k < 5; k++) com[(size_t)(kRowQ + 4 * k + a) * n + i] = S[k];
+  } else {
+    // kinetic partials of the block: lane (q, molecule) one term of quantity
+    // q (Rigid_Ek and Rigid_PressureTensor sums, as md_pre_body's), summed
+    // over the quad; then the block's kinetic energy
+    const int q = lane >> 2;
+    double e = 0.0;
+    if (q == 0) e = s_v[a][0] * s_v[a][0] + s_v[a][1] * s_v[a][1] + s_v[a][2] * s_v[a][2];
+    else if (q < 4) e = s_W[a][q - 1] * s_W[a][q - 1];
+    else if (q < kEkLen) {
+      const int l = q < 7 ? 0 : q < 9 ? 1 : 2;  // xx xy xz yy yz zz
+      const int h = q < 7 ? q - 4 : q < 9 ? q - 6 : 2;
+      e = s_v[a][l] * s_v[a][h];
+    }
+    e = quad_sum_d(e);
+    const size_t grp = (size_t)par * nblk + blk;
+    if (a == 0 && q < kEkLen) b.stepek[grp * kEkLen + q] = e;
+    const double et = __shfl(e, 0, 64), ex = __shfl(e, 4, 64), ey = __shfl(e, 8, 64),
+                 ez = __shfl(e, 12, 64);
+    if (lane == 0) b.stepkin[grp] = kin_energy(mt, dt, et, ex, ey, ez);
   }
 }
 
-// Ladder form (map as k_md_pre_lad); the block of index -1 of each system
-// closes that system's previous step when close_mode != 0.
+// The force phase of a step whose corrector is a kernel of its own; block 0
+// closes the previous step while the other blocks run the rows (ca.mode != 0).
+template <int M, typename R, int BOX>
+__global__ __launch_bounds__(256, (main_waves_per_eu<M, R>())) void k_md_main(ModelTable mt, Geom g,
+                                                                            MdBuf b, PairK<R> pk,
+                                                                            double *out, int parity,
+                                                                            CloseArgs ca,
+                                                                            int reg_bytes) {
+  const int close = ca.mode != 0;
+  if (close && blockIdx.x == 0) {
+    __shared__ double s_close[4][kRed];
+    close_body<false>(mt, b, g.n, g.ncell, box_volume(g.L), ca, s_close);
+    return;
+  }
+  md_main_body<M, R, BOX>(g, b, pk, out, parity, reg_bytes, blockIdx.x - close, gridDim.x - close);
+}
+
+// Workgroups are dealt to the eight XCDs round-robin by index.  The index-th
+// of nblk workgroups takes this block of four molecules: those of one XCD a
+// contiguous run, so the cache lines of the state arrays (16 molecules of one
+// component) and the records that near molecules share stay in one XCD's L2.
+__device__ inline int xcd_run(int index, int nblk) {
+  const int q = nblk >> 3, r = nblk & 7, x = index & 7, p = index >> 3;
+  return x < r ? x * (q + 1) + p : r * (q + 1) + (x - r) * q + p;
+}
+
+template <int M, typename R, int BOX>
+__global__ __launch_bounds__(256, (main_waves_per_eu<M, R>())) void k_md_step(
+    ModelTable mt, Geom g, MdBuf b, PairK<R> pk, StepArgs st, CloseArgs ca, int reg_bytes) {
+  // block 0 closes the previous step while the other blocks step
+  const int close = ca.mode != 0;
+  if (close && blockIdx.x == 0) {
+    __shared__ double s_close[4][kRed];
+    close_body<false>(mt, b, g.n, g.ncell, box_volume(g.L), ca, s_close);
+    return;
+  }
+  const int nblk = gridDim.x - close;
+  md_step_body<M, R, BOX>(mt, g, b, pk, st, reg_bytes, xcd_run(blockIdx.x - close, nblk), nblk);
+}
+
+// Ladder forms (map as k_md_pre_lad; the block of index -1 of each system
+// closes that system's previous step).
+// Arguments of the close in or around step q of a call of k steps: the pair
+// and kinetic partials of the step before, the thermostat state from its half
+// into this step's, and the list after next cleared.
+__device__ __host__ inline CloseArgs step_close_args(const MdBuf &b, int nose_active, int nblk,
+                                                     double dt, int mode, int parity, int list) {
+  CloseArgs ca;
+  ca.mode = mode;
+  ca.nose_active = nose_active;
+  ca.nblk_pre = ca.nblk_main = nblk;
+  ca.dt = dt;
+  ca.bpart = b.blockpart + (size_t)(1 - parity) * nblk * kBP;
+  ca.ek = b.stepek + (size_t)(1 - parity) * nblk * kEkLen;
+  ca.kin = b.stepkin + (size_t)(1 - parity) * nblk;
+  ca.nose_in = b.nose + 9 * (1 - parity);
+  ca.nose_out = b.nose + 9 * parity;
+  ca.clear = 1 << ((list + 2) % 3);
+  return ca;
+}
+// the closes before the first step (mode 2: the thermostat state of the call's
+// start, predicted into the first step's half; lists 1 and 2 cleared) and
+// after the last (mode 1: the last step has parity 0; every list cleared)
+__device__ __host__ inline CloseArgs step_end_args(const MdBuf &b, int nose_active, int nblk,
+                                                   double dt, int mode, int k) {
+  CloseArgs ca = step_close_args(b, nose_active, nblk, dt, mode, 1, 0);
+  ca.nose_in = b.nose;
+  ca.nose_out = b.nose + (mode == 2 ? 9 * ((k - 1) & 1) : 0);
+  ca.clear = mode == 2 ? 6 : 7;
+  return ca;
+}
+
+// the close of a step whose corrector was k_md_pre: the pair partials of
+// src_parity, the kinetic partials and the thermostat state in the first halves
+__device__ __host__ inline CloseArgs pre_close_args(const MdBuf &b, int n, int nose_active,
+                                                    int nblk, double dt, int mode, int clear,
+                                                    int src_parity) {
+  CloseArgs ca;
+  ca.mode = mode;
+  ca.nose_active = nose_active;
+  ca.nblk_pre = (n + 3) / 4;
+  ca.nblk_main = nblk;
+  ca.dt = dt;
+  ca.bpart = b.blockpart + (size_t)src_parity * nblk * kBP;
+  ca.ek = b.stepek;
+  ca.kin = b.stepkin;
+  ca.nose_in = ca.nose_out = b.nose;
+  ca.clear = clear;
+  return ca;
+}
+
 template <int M, typename R>
-__global__ __launch_bounds__(256, (main_waves_per_eu<M, R>())) void k_md_main_lad(ModelTable mt, const MdRep *__restrict__ reps,
-                                                     const int2 *__restrict__ map, PairK<R> pk,
-                                                     int parity, int close_mode, int reg_bytes) {
+__global__ __launch_bounds__(256, (main_waves_per_eu<M, R>())) void k_md_main_lad(
+    ModelTable mt, const MdRep *__restrict__ reps, const int2 *__restrict__ map, PairK<R> pk,
+    int parity, int close_mode, int reg_bytes) {
   const int2 m = map[blockIdx.x];
   if (m.x < 0) return;
   const Geom g = reps[m.x].g;
   const MdBuf b = reps[m.x].b;
   const int nm = reps[m.x].nblk_main;
-  CloseArgs ca;
-  ca.mode = close_mode;
-  ca.nose_active = reps[m.x].nose_active;
-  ca.nblk_pre = (g.n + 63) / 64 * 4;
-  ca.nblk_main = nm;
-  ca.bpart = b.blockpart + (size_t)(1 - parity) * nm * kBP;
-  ca.dt = reps[m.x].dt;
   if (m.y < 0) {
     if (close_mode) {
       __shared__ double s_close[4][kRed];
-      close_body<false>(mt, b, g.n, ca.dt, ca.nblk_pre, ca.bpart, ca.nblk_main, g.ncell,
-                        ca.nose_active, ca.mode, parity, box_volume(g.L), s_close);
+      const CloseArgs ca = pre_close_args(b, g.n, reps[m.x].nose_active, nm, reps[m.x].dt,
+                                          close_mode, 1 << (1 - parity), 1 - parity);
+      close_body<false>(mt, b, g.n, g.ncell, box_volume(g.L), ca, s_close);
     }
     return;
   }
-  md_main_body<M, R, kBoxCube>(mt, g, b, pk, nullptr, parity, ca, reg_bytes, m.y, nm);
+  md_main_body<M, R, kBoxCube>(g, b, pk, nullptr, parity, reg_bytes, m.y, nm);
+}
+
+template <int M, typename R>
+__global__ __launch_bounds__(256, (main_waves_per_eu<M, R>())) void k_md_step_lad(
+    ModelTable mt, const MdRep *__restrict__ reps, const int2 *__restrict__ map, PairK<R> pk,
+    StepArgs st, int reg_bytes) {
+  const int2 m = map[blockIdx.x];
+  if (m.x < 0) return;
+  const Geom g = reps[m.x].g;
+  const MdBuf b = reps[m.x].b;
+  const int nm = reps[m.x].nblk_main;
+  StepArgs s1 = st;
+  s1.nose_active = reps[m.x].nose_active;
+  s1.dt = reps[m.x].dt;
+  if (m.y < 0) {
+    if (!st.first) {
+      __shared__ double s_close[4][kRed];
+      const CloseArgs ca = step_close_args(b, s1.nose_active, nm, s1.dt, 1 | 2, st.parity, st.list);
+      close_body<false>(mt, b, g.n, g.ncell, box_volume(g.L), ca, s_close);
+    }
+    return;
+  }
+  md_step_body<M, R, kBoxCube>(mt, g, b, pk, s1, reg_bytes, m.y, nm);
+}
+
+// block r closes system r before (mode 2) or after (mode 1) the k steps of a
+// call; one: they run as step kernels
+__global__ __launch_bounds__(256) void k_md_close_lad(ModelTable mt, const MdRep *__restrict__ reps,
+                                                      int mode, int k, int one) {
+  __shared__ double s_red[4][kRed];
+  const MdRep &r = reps[blockIdx.x];
+  const MdBuf b = r.b;
+  const CloseArgs ca =
+      one ? step_end_args(b, r.nose_active, r.nblk_main, r.dt, mode, k)
+          : pre_close_args(b, r.g.n, r.nose_active, r.nblk_main, r.dt, mode, mode == 2 ? 2 : 7,
+                           (k - 1) & 1);
+  close_body<false>(mt, b, r.g.n, r.g.ncell, box_volume(r.g.L), ca, s_red);
 }
 
 __global__ void k_flag_set(int *flags, int k, int v) {
@@ -1010,41 +1541,31 @@ __global__ void k_flag_set(int *flags, int k, int v) {
 
 void md_launch_flag(System &s, int k, int v) { k_flag_set<<<1, 64, 0, s.stream>>>(s.md.flags, k, v); }
 
-void md_launch_pre(System &s, bool correct, bool predict, bool sites, int parity) {
-  const int nb = pre_waves(s.n) / 4, na = s.nose_active ? 1 : 0;
-  if (s.andersen)
-    k_md_pre<kBoxBaro><<<nb, 256, 0, s.stream>>>(s.mt, s.geo_md, s.md, s.dt, na, correct ? 1 : 0,
-                                                 predict ? 1 : 0, sites ? 1 : 0, parity);
-  else if (is_cubic(s))
-    k_md_pre<kBoxCube><<<nb, 256, 0, s.stream>>>(s.mt, s.geo_md, s.md, s.dt, na, correct ? 1 : 0,
-                                                 predict ? 1 : 0, sites ? 1 : 0, parity);
-  else
-    k_md_pre<kBoxOrtho><<<nb, 256, 0, s.stream>>>(s.mt, s.geo_md, s.md, s.dt, na,
-                                                  correct ? 1 : 0, predict ? 1 : 0, sites ? 1 : 0,
-                                                  parity);
+void md_launch_pre(System &s, bool correct, bool predict, bool sites, int list, int half) {
+  const int nb = pre_blocks(s.n), na = s.nose_active ? 1 : 0;
+  const int co = correct ? 1 : 0, pr = predict ? 1 : 0, si = sites ? 1 : 0;
+  auto launch = [&](auto kern) {
+    kern<<<nb, 256, 0, s.stream>>>(s.mt, s.geo_md, s.md, s.dt, na, co, pr, si, list, half);
+  };
+  if (s.andersen) launch(k_md_pre<kBoxBaro>);
+  else if (is_cubic(s)) launch(k_md_pre<kBoxCube>);
+  else launch(k_md_pre<kBoxOrtho>);
 }
 
-static CloseArgs close_args(System &s, int mode, int src_parity) {
-  CloseArgs ca;
-  ca.mode = mode;
-  ca.nose_active = s.nose_active ? 1 : 0;
-  ca.nblk_pre = pre_waves(s.n);
-  ca.nblk_main = s.nblk_md;
-  ca.bpart = s.md.blockpart + (size_t)src_parity * s.nblk_md * kBP;
-  ca.dt = s.dt;
-  return ca;
+static CloseArgs close_args(System &s, int mode, int clear, int src_parity) {
+  return pre_close_args(s.md, s.n, s.nose_active ? 1 : 0, s.nblk_md, s.dt, mode, clear, src_parity);
 }
 
-void md_launch_close(System &s, int mode, int parity, int src_parity) {
-  const CloseArgs ca = close_args(s, mode, src_parity);
-  if (s.andersen)
-    k_md_close<true><<<1, 256, 0, s.stream>>>(s.mt, s.md, s.n, s.dt, ca.nblk_pre, ca.bpart,
-                                              ca.nblk_main, s.geo_md.ncell, ca.nose_active, mode,
-                                              parity, box_volume(s.Lb));
-  else
-    k_md_close<false><<<1, 256, 0, s.stream>>>(s.mt, s.md, s.n, s.dt, ca.nblk_pre, ca.bpart,
-                                               ca.nblk_main, s.geo_md.ncell, ca.nose_active,
-                                               mode, parity, box_volume(s.Lb));
+static void launch_close(System &s, const CloseArgs &ca) {
+  auto launch = [&](auto kern) {
+    kern<<<1, 256, 0, s.stream>>>(s.mt, s.md, s.n, s.geo_md.ncell, box_volume(s.Lb), ca);
+  };
+  if (s.andersen) launch(k_md_close<true>);
+  else launch(k_md_close<false>);
+}
+
+void md_launch_close(System &s, int mode, int clear, int src_parity) {
+  launch_close(s, close_args(s, mode, clear, src_parity));
 }
 
 template <typename R>
@@ -1054,79 +1575,112 @@ const PairK<float> &pair_k<float>(const System &s) { return s.pkf; }
 template <>
 const PairK<double> &pair_k<double>(const System &s) { return s.pkd; }
 
-template <int M, typename R>
-static void md_main_t(System &s, double *out, int parity, const CloseArgs &ca) {
-  const int rb = main_region_bytes(s.md.maxnb, (int)sizeof(R));
-  const unsigned grid = s.nblk_md + (ca.mode ? 1 : 0);
-  const size_t lds = 4 * (size_t)rb;
-  if (s.andersen)
-    k_md_main<M, R, kBoxBaro><<<grid, 256, lds, s.stream>>>(s.mt, s.geo_md, s.md, pair_k<R>(s),
-                                                            out, parity, ca, rb);
-  else if (is_cubic(s))
-    k_md_main<M, R, kBoxCube><<<grid, 256, lds, s.stream>>>(s.mt, s.geo_md, s.md, pair_k<R>(s),
-                                                            out, parity, ca, rb);
-  else
-    k_md_main<M, R, kBoxOrtho><<<grid, 256, lds, s.stream>>>(s.mt, s.geo_md, s.md, pair_k<R>(s),
-                                                             out, parity, ca, rb);
+// calls f with the pair-kernel layout and the pair precision of a system
+// (or ladder) as std::integral_constant and a value of the type
+template <class F>
+static void with_model(int kmodel, int prec, F &&f) {
+  auto pr = [&](auto m) {
+    if (prec == G6_FP32) f(m, 0.0f);
+    else f(m, 0.0);
+  };
+  if (kmodel == G6_TIP4P) pr(std::integral_constant<int, G6_TIP4P>());
+  else if (kmodel == G6_TIP5P) pr(std::integral_constant<int, G6_TIP5P>());
+  else if (kmodel == G6_SPCE) pr(std::integral_constant<int, G6_SPCE>());
+  else if (kmodel == G6_NVDE) pr(std::integral_constant<int, G6_NVDE>());
+  else if (kmodel == G6_OPLSMEOH) pr(std::integral_constant<int, G6_OPLSMEOH>());
+  else pr(std::integral_constant<int, G6_ST2>());
 }
 
 void md_launch_main(System &s, double *out, int parity, int close_mode) {
-  const CloseArgs ca = close_args(s, close_mode, 1 - parity);
+  const CloseArgs ca =
+      close_args(s, close_mode, close_mode ? 1 << (1 - parity) : 0, 1 - parity);
   if (s.tiles) {
     md_launch_tile(s, parity, ca);
     if (out) md_launch_part_reduce(s, out);
     return;
   }
-  if (s.prec == G6_FP32) {
-    if (s.kmodel == G6_TIP4P) md_main_t<G6_TIP4P, float>(s, out, parity, ca);
-    else if (s.kmodel == G6_TIP5P) md_main_t<G6_TIP5P, float>(s, out, parity, ca);
-    else if (s.kmodel == G6_SPCE) md_main_t<G6_SPCE, float>(s, out, parity, ca);
-    else if (s.kmodel == G6_NVDE) md_main_t<G6_NVDE, float>(s, out, parity, ca);
-    else if (s.kmodel == G6_OPLSMEOH) md_main_t<G6_OPLSMEOH, float>(s, out, parity, ca);
-    else md_main_t<G6_ST2, float>(s, out, parity, ca);
-  } else {
-    if (s.kmodel == G6_TIP4P) md_main_t<G6_TIP4P, double>(s, out, parity, ca);
-    else if (s.kmodel == G6_TIP5P) md_main_t<G6_TIP5P, double>(s, out, parity, ca);
-    else if (s.kmodel == G6_SPCE) md_main_t<G6_SPCE, double>(s, out, parity, ca);
-    else if (s.kmodel == G6_NVDE) md_main_t<G6_NVDE, double>(s, out, parity, ca);
-    else if (s.kmodel == G6_OPLSMEOH) md_main_t<G6_OPLSMEOH, double>(s, out, parity, ca);
-    else md_main_t<G6_ST2, double>(s, out, parity, ca);
-  }
+  with_model(s.kmodel, s.prec, [&](auto mm, auto rr) {
+    constexpr int M = decltype(mm)::value;
+    using R = decltype(rr);
+    const int rb = main_region_bytes(s.md.maxnb, (int)sizeof(R));
+    auto launch = [&](auto kern) {
+      kern<<<s.nblk_md + (ca.mode ? 1 : 0), 256, 4 * (size_t)rb, s.stream>>>(
+          s.mt, s.geo_md, s.md, pair_k<R>(s), out, parity, ca, rb);
+    };
+    if (s.andersen) launch(k_md_main<M, R, kBoxBaro>);
+    else if (is_cubic(s)) launch(k_md_main<M, R, kBoxCube>);
+    else launch(k_md_main<M, R, kBoxOrtho>);
+  });
 }
 
-void md_launch_pre_lad(Ladder &l, bool correct, bool predict, bool sites, int parity) {
+// step q of k has parity (k - 1 - q) mod 2: the last one leaves its records,
+// partials and thermostat state in the first halves
+static StepArgs step_args(int q, int k) {
+  StepArgs st{};
+  st.parity = (k - 1 - q) & 1;
+  st.list = q % 3;
+  st.first = q == 0;
+  st.last = q == k - 1;
+  return st;
+}
+
+void md_launch_step(System &s, int q, int k) {
+  StepArgs st = step_args(q, k);
+  st.nose_active = s.nose_active ? 1 : 0;
+  st.dt = s.dt;
+  const CloseArgs ca = step_close_args(s.md, st.nose_active, s.nblk_md, s.dt, q > 0 ? 1 | 2 : 0,
+                                       st.parity, st.list);
+  with_model(s.kmodel, s.prec, [&](auto mm, auto rr) {
+    constexpr int M = decltype(mm)::value;
+    using R = decltype(rr);
+    const int rb = main_region_bytes(s.md.maxnb, (int)sizeof(R));
+    auto launch = [&](auto kern) {
+      kern<<<s.nblk_md + (ca.mode ? 1 : 0), 256, 4 * (size_t)rb, s.stream>>>(
+          s.mt, s.geo_md, s.md, pair_k<R>(s), st, ca, rb);
+    };
+    if (is_cubic(s)) launch(k_md_step<M, R, kBoxCube>);
+    else launch(k_md_step<M, R, kBoxOrtho>);
+  });
+}
+
+void md_launch_step_close(System &s, int mode, int k) {
+  launch_close(s, step_end_args(s.md, s.nose_active ? 1 : 0, s.nblk_md, s.dt, mode, k));
+}
+
+void md_launch_pre_lad(Ladder &l, bool correct, bool predict, int list, int half) {
   k_md_pre_lad<<<l.grid_pre, 256, 0, l.stream>>>(l.mt, l.reps, l.map_pre, correct ? 1 : 0,
-                                                 predict ? 1 : 0, sites ? 1 : 0, parity);
+                                                 predict ? 1 : 0, list, half);
 }
 
-void md_launch_close_lad(Ladder &l, int mode, int parity, int src_parity) {
-  k_md_close_lad<<<(int)l.sys.size(), 256, 0, l.stream>>>(l.mt, l.reps, mode, parity, src_parity);
+void md_launch_close_lad(Ladder &l, int mode, int k) {
+  k_md_close_lad<<<(int)l.sys.size(), 256, 0, l.stream>>>(l.mt, l.reps, mode, k,
+                                                          l.one_kernel ? 1 : 0);
 }
 
-template <int M, typename R>
-static void md_main_lad_t(Ladder &l, const PairK<R> &pk, int parity, int close_mode) {
-  k_md_main_lad<M, R><<<l.grid_main, 256, 4 * (size_t)l.reg_bytes, l.stream>>>(
-      l.mt, l.reps, l.map_main, pk, parity, close_mode, l.reg_bytes);
+template <typename R>
+static const PairK<R> &pair_k(const Ladder &l);
+template <>
+const PairK<float> &pair_k<float>(const Ladder &l) { return l.pkf; }
+template <>
+const PairK<double> &pair_k<double>(const Ladder &l) { return l.pkd; }
+
+void md_launch_step_lad(Ladder &l, int q, int k) {
+  const StepArgs st = step_args(q, k);
+  with_model(l.model, l.prec, [&](auto mm, auto rr) {
+    constexpr int M = decltype(mm)::value;
+    using R = decltype(rr);
+    k_md_step_lad<M, R><<<l.grid_main, 256, 4 * (size_t)l.reg_bytes, l.stream>>>(
+        l.mt, l.reps, l.map_main, pair_k<R>(l), st, l.reg_bytes);
+  });
 }
 
 void md_launch_main_lad(Ladder &l, int parity, int close_mode) {
-  if (l.prec == G6_FP32) {
-    if (l.model == G6_TIP4P) md_main_lad_t<G6_TIP4P, float>(l, l.pkf, parity, close_mode);
-    else if (l.model == G6_TIP5P) md_main_lad_t<G6_TIP5P, float>(l, l.pkf, parity, close_mode);
-    else if (l.model == G6_SPCE) md_main_lad_t<G6_SPCE, float>(l, l.pkf, parity, close_mode);
-    else if (l.model == G6_NVDE) md_main_lad_t<G6_NVDE, float>(l, l.pkf, parity, close_mode);
-    else if (l.model == G6_OPLSMEOH)
-      md_main_lad_t<G6_OPLSMEOH, float>(l, l.pkf, parity, close_mode);
-    else md_main_lad_t<G6_ST2, float>(l, l.pkf, parity, close_mode);
-  } else {
-    if (l.model == G6_TIP4P) md_main_lad_t<G6_TIP4P, double>(l, l.pkd, parity, close_mode);
-    else if (l.model == G6_TIP5P) md_main_lad_t<G6_TIP5P, double>(l, l.pkd, parity, close_mode);
-    else if (l.model == G6_SPCE) md_main_lad_t<G6_SPCE, double>(l, l.pkd, parity, close_mode);
-    else if (l.model == G6_NVDE) md_main_lad_t<G6_NVDE, double>(l, l.pkd, parity, close_mode);
-    else if (l.model == G6_OPLSMEOH)
-      md_main_lad_t<G6_OPLSMEOH, double>(l, l.pkd, parity, close_mode);
-    else md_main_lad_t<G6_ST2, double>(l, l.pkd, parity, close_mode);
-  }
+  with_model(l.model, l.prec, [&](auto mm, auto rr) {
+    constexpr int M = decltype(mm)::value;
+    using R = decltype(rr);
+    k_md_main_lad<M, R><<<l.grid_main, 256, 4 * (size_t)l.reg_bytes, l.stream>>>(
+        l.mt, l.reps, l.map_main, pair_k<R>(l), parity, close_mode, l.reg_bytes);
+  });
 }
 
 }  // namespace g6

@@ -149,20 +149,42 @@ __device__ inline void andersen_rescale(const double *a, double *box) {
   }
 }
 
+// Nose_Correct with the temperature of the step (NoseModule.F90:43-63) and
+// Nose_Predict (NoseModule.F90:65-87); z = temp, q, dump, zeta0..4, zetasum.
+__device__ inline void nose_correct(double (&z)[9], double temp) {
+  const double zetaf = (temp - z[0]) / z[1] - z[2] * z[3];
+  const double dz2 = zetaf - z[4];
+  z[3] = z[3] + kG4_0 * dz2;
+  z[4] = zetaf;
+  z[5] = z[5] + kG4_2 * dz2;
+  z[6] = z[6] + kG4_3 * dz2;
+  z[7] = z[7] + kG4_4 * dz2;
+  z[8] = z[8] + z[3];
+}
+__device__ inline void nose_predict(double (&z)[9]) {
+  z[3] = z[3] + z[4] + z[5] + z[6] + z[7];
+  z[4] = z[4] + 2.0 * z[5] + 3.0 * z[6] + 4.0 * z[7];
+  z[5] = z[5] + 3.0 * z[6] + 6.0 * z[7];
+  z[6] = z[6] + 4.0 * z[7];
+}
+__device__ inline double temperature_of(double ek, int n) {
+  return 10.0 * 2.0 * ek / (G6_RGAS_MD * (6.0 * n));
+}
+
 // ---- step close: one block of 256 threads ---------------------------------
-// mode bits: 1 the kinetic partials of k_md_pre + the pair partials of the
-// previous k_md_main (bpart) form the thermo record, then Nose_Correct;
-// 2 Nose_Predict; 4 clear the cell counts and rebuild flag of parity 1-p
-// (8: both parities); 16 force evaluation: the pair partials alone go to the
-// thermo record.  Runs as its own kernel (k_md_close) or at the start of
-// block 0 of k_md_main, which neither reads nor writes what it touches.
-template <bool NPT>
-__device__ inline void close_body(const ModelTable &mt, const MdBuf &b, int n, double dt,
-                                  int nblk_pre, const double *bpart, int nblk_main, int ncell,
-                                  int nose_active, int mode, int parity, double box_vol,
-                                  double (&s_red)[4][kRed]) {
-  constexpr int NR = 12 + kEkLen;
-  const int wid = threadIdx.x >> 6;
+// mode bits: 1 the kinetic partials and the pair partials of the step
+// (ca.bpart) form the thermo record, then Nose_Correct; 2 Nose_Predict;
+// 16 force evaluation: the pair partials alone go to the thermo record.
+// ca.clear: the cell lists and rebuild flags to clear.  Runs as its own
+// kernel (k_md_close) or in block 0 of the force or step kernel, which
+// neither reads nor writes what it touches.
+// U: rounds of partials with their loads in flight together (registers).
+template <bool NPT, int U = 2>
+__device__ inline void close_body(const ModelTable &mt, const MdBuf &b, int n, int ncell,
+                                  double box_vol, const CloseArgs &ca, double (&s_red)[4][kRed]) {
+  constexpr int NR = kRed;
+  const int wid = threadIdx.x >> 6, mode = ca.mode;
+  const double dt = ca.dt;
   // the work runs on threads 0..255; wider blocks (the tile kernel's) only
   // take part in the barriers
   if (threadIdx.x < 256) {
@@ -170,22 +192,22 @@ __device__ inline void close_body(const ModelTable &mt, const MdBuf &b, int n, d
   // (one memory round trip fewer; the sums keep their order)
   double ek0[kEkLen];
   {
-    const bool first = (mode & 1) && (int)threadIdx.x < nblk_pre;
+    const bool first = (mode & 1) && (int)threadIdx.x < ca.nblk_pre;
 #pragma unroll
     for (int q = 0; q < kEkLen; q++)
-      ek0[q] = first ? b.blockek[(size_t)threadIdx.x * kEkLen + q] : 0.0;
+      ek0[q] = first ? ca.ek[(size_t)threadIdx.x * kEkLen + q] : 0.0;
   }
   {
-    // the pair partials of k_md_main (each rounded once from its compensated
-    // block sum), summed over blocks in a fixed order
+    // the pair partials (each rounded once from its compensated block sum),
+    // summed over blocks in a fixed order
     double ps[12];
 #pragma unroll
     for (int q = 0; q < 12; q++) ps[q] = 0.0;
     if (mode & 17) {
 #pragma unroll 4
-      for (int k = threadIdx.x; k < nblk_main; k += 256)
+      for (int k = threadIdx.x; k < ca.nblk_main; k += 256)
 #pragma unroll
-        for (int q = 0; q < 12; q++) ps[q] += bpart[(size_t)k * kBP + q];
+        for (int q = 0; q < 12; q++) ps[q] += ca.bpart[(size_t)k * kBP + q];
     }
 #pragma unroll
     for (int q = 0; q < 12; q++) ps[q] = wsum63(ps[q]);
@@ -194,29 +216,33 @@ __device__ inline void close_body(const ModelTable &mt, const MdBuf &b, int n, d
       for (int q = 0; q < 12; q++) s_red[wid][q] = ps[q];
   }
   {
-    // the kinetic partials of k_md_pre
-    double ek[kEkLen];
+    // the kinetic partials
+    double ek[kEkLen], kin = 0.0;
 #pragma unroll
     for (int q = 0; q < kEkLen; q++) ek[q] = 0.0 + ek0[q];
     if (mode & 1) {
-#pragma unroll 1
-      for (int k = threadIdx.x + 256; k < nblk_pre; k += 256)
+#pragma unroll U
+      for (int k = threadIdx.x + 256; k < ca.nblk_pre; k += 256)
 #pragma unroll
-        for (int q = 0; q < kEkLen; q++) ek[q] += b.blockek[(size_t)k * kEkLen + q];
+        for (int q = 0; q < kEkLen; q++) ek[q] += ca.ek[(size_t)k * kEkLen + q];
+#pragma unroll 4
+      for (int k = threadIdx.x; k < ca.nblk_pre; k += 256) kin += ca.kin[k];
     }
 #pragma unroll
     for (int q = 0; q < kEkLen; q++) ek[q] = wsum63(ek[q]);
-    if ((threadIdx.x & 63) == 63)
+    kin = wsum63(kin);
+    if ((threadIdx.x & 63) == 63) {
 #pragma unroll
       for (int q = 0; q < kEkLen; q++) s_red[wid][12 + q] = ek[q];
-  }
-  if (mode & 12) {
-    const int p0 = (mode & 8) ? 0 : 1 - parity, p1 = (mode & 8) ? 1 : 1 - parity;
-    for (int p = p0; p <= p1; p++) {
-      int *cr = b.cellres + (size_t)p * ncell * b.cell_cap;
-      for (int c = threadIdx.x; c < ncell; c += 256) cr[(size_t)c * b.cell_cap] = 0;
-      if (threadIdx.x == 0 && b.half_skin2 > 0.0) b.flags[2 + p] = 0;
+      s_red[wid][12 + kEkLen] = kin;
     }
+  }
+  for (int p = 0; p < 3; p++) {
+    if (!(ca.clear >> p & 1)) continue;
+    int *cr = b.cellres + (size_t)p * ncell * b.cell_cap;
+    if (!b.scan)
+      for (int c = threadIdx.x; c < ncell; c += 256) cr[(size_t)c * b.cell_cap] = 0;
+    if (threadIdx.x == 0 && b.half_skin2 > 0.0) b.flags[2 + p] = 0;
   }
   }
   __syncthreads();
@@ -228,7 +254,9 @@ __device__ inline void close_body(const ModelTable &mt, const MdBuf &b, int n, d
   __syncthreads();
   if (threadIdx.x == 0) {
     const double *r = s_red[0];
-    double *z = b.nose, *th = b.thermo;
+    double *th = b.thermo;
+    double z[9];
+    for (int q = 0; q < 9; q++) z[q] = ca.nose_in[q];
     if (mode & 17) {
       th[0] = r[0];
       for (int q = 0; q < 9; q++) th[4 + q] = r[1 + q];
@@ -240,18 +268,11 @@ __device__ inline void close_body(const ModelTable &mt, const MdBuf &b, int n, d
       const double ekt = r[12] * mt.mass * 0.5 * (1.0 / (dt * dt));
       const double ekr = (r[13] * mt.Ixx + r[14] * mt.Iyy + r[15] * mt.Izz) * 0.5;
       const double dof = 6.0 * n;
-      const double temp = 10.0 * 2.0 * (ekt + ekr) / (G6_RGAS_MD * dof);
+      const double temp = temperature_of(r[12 + kEkLen], n);
       double h = (ep + ekt + ekr) * 10.0;
       double nose_ep = 0.0, nose_ek = 0.0;
-      if (nose_active) {
-        const double zetaf = (temp - z[0]) / z[1] - z[2] * z[3];
-        const double dz2 = zetaf - z[4];
-        z[3] = z[3] + kG4_0 * dz2;
-        z[4] = zetaf;
-        z[5] = z[5] + kG4_2 * dz2;
-        z[6] = z[6] + kG4_3 * dz2;
-        z[7] = z[7] + kG4_4 * dz2;
-        z[8] = z[8] + z[3];
+      if (ca.nose_active) {
+        nose_correct(z, temp);
         nose_ek = (z[3] * z[3] * z[1] * dt * dof * 0.5) * G6_RGAS_MD;
         nose_ep = (dof * z[0] * (z[8] - 0.5 * z[3]) * dt) * G6_RGAS_MD;
         h = h + nose_ep + nose_ek;
@@ -294,16 +315,13 @@ __device__ inline void close_body(const ModelTable &mt, const MdBuf &b, int n, d
       th[26] = volc;
       th[27] = nose_ep;
       th[28] = nose_ek;
-      th[29] = nose_active ? z[0] : 0.0;
+      th[29] = ca.nose_active ? z[0] : 0.0;
       th[30] = and_ep;
       th[31] = and_ek;
     }
-    if ((mode & 2) && nose_active) {
-      z[3] = z[3] + z[4] + z[5] + z[6] + z[7];
-      z[4] = z[4] + 2.0 * z[5] + 3.0 * z[6] + 4.0 * z[7];
-      z[5] = z[5] + 3.0 * z[6] + 6.0 * z[7];
-      z[6] = z[6] + 4.0 * z[7];
-    }
+    if ((mode & 2) && ca.nose_active) nose_predict(z);
+    if (!(mode & 16))
+      for (int q = 0; q < 9; q++) ca.nose_out[q] = z[q];
     if (NPT && (mode & 2)) {
       // Andersen_Predict (AndersenModule.F90:84-93)
       double *a = b.anders;
@@ -316,7 +334,6 @@ __device__ inline void close_body(const ModelTable &mt, const MdBuf &b, int n, d
     }
   }
 }
-
 
 // site offsets of the sites before the CoM site from a record
 template <int M, typename R>

@@ -500,7 +500,7 @@ static MixSide mix_side(const System &s) {
   d.Ixx = s.mt.Ixx;
   d.Iyy = s.mt.Iyy;
   d.Izz = s.mt.Izz;
-  d.blockek = s.md.blockek;
+  d.blockek = s.md.stepek;
   d.cellres = s.md.cellres;
   d.flags = s.md.flags;
   d.cell_cap = s.md.cell_cap;
@@ -517,8 +517,8 @@ static MixClose mix_close_args(const Mix &m, int src_parity) {
   c.thermo = a.md.thermo;
   c.na = a.n;
   c.nb = b.n;
-  c.nblk_pre_a = pre_waves(a.n);
-  c.nblk_pre_b = pre_waves(b.n);
+  c.nblk_pre_a = (a.n + 3) / 4;
+  c.nblk_pre_b = (b.n + 3) / 4;
   c.nblk_main_a = a.nblk_md;
   c.nblk_main_b = b.nblk_md;
   c.nblk_x = m.nblk_a + m.nblk_b;

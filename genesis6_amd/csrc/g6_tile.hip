@@ -518,8 +518,7 @@ __global__ __launch_bounds__(512) void k_md_tile(ModelTable mt, Geom g, MdBuf b,
     // block 0 closes the previous step while the other blocks run the tiles
     if (blockIdx.x == 0) {
       __shared__ double s_close[4][kRed];
-      close_body<false>(mt, b, g.n, ca.dt, ca.nblk_pre, ca.bpart, ca.nblk_main, g.ncell,
-                        ca.nose_active, ca.mode, parity, box_volume(g.L), s_close);
+      close_body<false>(mt, b, g.n, g.ncell, box_volume(g.L), ca, s_close);
       return;
     }
     tile_body<M, STAGE>(g, b, pk, parity, lay, blockIdx.x - 1, gridDim.x - 1);

@@ -1,6 +1,6 @@
-"""The row build of the MD force kernel: rows from a scan of every molecule
+"""The forms of the MD step on the rows: rows from a scan of every molecule
 and rows from the cell lists hold the oracle's pairs and give the same
-trajectory."""
+trajectory, and so do one kernel per step and two."""
 import os
 
 import numpy as np
@@ -12,17 +12,19 @@ from oracle import pyoracle as O
 pytestmark = pytest.mark.gpu
 
 
-def system(n, L, rc, skin, prec, scan_max):
-    old = os.environ.get("G6_SCAN_MAX")
-    os.environ["G6_SCAN_MAX"] = str(scan_max)
+def system(n, L, rc, skin, prec, model=g6.TIP4P, **env):
+    old = {k: os.environ.get(k) for k in env}
+    os.environ.update({k: str(v) for k, v in env.items()})
     try:
-        s = g6.System(g6.TIP4P, n, L, rc, 0.5, 0.002, prec=prec, skin=skin)
+        s = g6.System(model, n, L, rc, 0.5, 0.002, prec=prec, skin=skin)
     finally:
-        if old is None:
-            del os.environ["G6_SCAN_MAX"]
-        else:
-            os.environ["G6_SCAN_MAX"] = old
-    com, q = g6.lattice_start(n, L, 31 + n)
+        for k, v in old.items():
+            if v is None:
+                del os.environ[k]
+            else:
+                os.environ[k] = v
+    com, q = g6.lattice_start(n, np.max(L), 31 + n)
+    com *= np.asarray(L) / np.max(L)
     # off the lattice, and some molecules boxes away (unwrapped COMs)
     com += np.random.default_rng(n).normal(0.0, 0.05, com.shape)
     com[::7] += L * np.random.default_rng(n + 1).integers(-3, 4, com[::7].shape)
@@ -42,7 +44,7 @@ def test_scan_and_cell_rows(n, skin, prec):
     rc = min(8.5, 0.5 * L - skin - 0.01)
     out = []
     for scan_max in (0, 1 << 20):
-        s, com = system(n, L, rc, skin, prec, scan_max)
+        s, com = system(n, L, rc, skin, prec, G6_SCAN_MAX=scan_max)
         print("rows n %d skin %g scan_max %d" % (n, skin, scan_max), flush=True)
         _, _, th = s.eval_forces()
         s.step(12)
@@ -54,3 +56,34 @@ def test_scan_and_cell_rows(n, skin, prec):
     for a, b in zip(out[0][1], out[1][1]):
         assert np.array_equal(a, b)
     assert np.array_equal(out[0][2], out[1][2])
+
+
+# blocks of four molecules with one to four of them; a thousand kinetic
+# energies and more (four per thread); boxes, thermostat, models of three to
+# six sites; calls of one, two and several steps between other calls
+@pytest.mark.parametrize("n,model,prec,skin,nose,ortho", [
+    (2, g6.TIP4P, g6.FP64, 0.0, True, False), (65, g6.TIP5P, g6.FP32, 0.5, True, False),
+    (127, g6.SPCE, g6.FP64, 1.0, False, True), (216, g6.NVDE, g6.FP32, 0.0, True, False),
+    (510, g6.ST2, g6.FP64, 1.0, True, True), (4101, g6.TIP4P, g6.FP32, 1.0, True, False)])
+def test_one_kernel_and_two_kernel_steps(n, model, prec, skin, nose, ortho):
+    L = (n / 0.0334) ** (1.0 / 3.0) if n > 2 else 12.0
+    rc = min(8.5, 0.45 * L - skin - 0.01)
+    box = np.array([L, 1.1 * L, L]) if ortho else L
+    out = []
+    for step_max in (1 << 30, 0):
+        s, _ = system(n, box, rc, skin, prec, model, G6_STEP_MAX=step_max)
+        if nose:
+            s.set_nose(300.0, 7.5e5)
+        print("steps n %d model %d step_max %d" % (n, model, step_max), flush=True)
+        got = []
+        for k in (1, 2, 1, 7, 50):
+            s.step(k)
+            got += [s.thermo(), s.nose(), *s.download()]
+            if k == 7:
+                got += list(s.eval_forces())
+                if nose:
+                    s.set_temperature(320.0)
+        out.append(got)
+        s.close()
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
