@@ -12,7 +12,7 @@
 //     count so that no two cells share a counter's cache line
 //   nbr_j/nbr_code[n][maxnb], nbr_cnt[n]: full (both-direction) Verlet rows
 //     within rc + skin; nbr_code packs the image shift ox = kx*L etc. as
-//     10-bit fields (kx+512) | (ky+512)<<10 | (kz+512)<<20 (COMs are
+//     10-bit signed fields kx | ky<<10 | kz<<20 (COMs are
 //     unwrapped, so |k| can exceed 1).  The -0.0 shift that dnint gives for
 //     small negative differences is stored as 0: x - (-0.0) and x - 0.0 are
 //     equal for every x but a zero x, whose sign no force term can see
@@ -374,7 +374,7 @@ constexpr int kRowWords = 128;
 inline int main_region_bytes(int maxnb, int rsize) {
   auto up16 = [](int x) { return (x + 15) / 16 * 16; };
   const int sort = 8 * maxnb + 8 * kRowWords + 4 * (128 + 132);  // entries, window, stencil
-  const int comp = up16(4 * maxnb) + 3 * up16(rsize * maxnb);
+  const int comp = rsize == 4 ? 16 * maxnb : up16(4 * maxnb) + 3 * up16(8 * maxnb);
   const int acc = 10 * 64 * 8;
   const int mx = sort > comp ? sort : comp;
   return up16(mx > acc ? mx : acc);

@@ -546,7 +546,7 @@ __device__ inline bool row_test(const BoxNow &bx, const MdBuf &b, double rr, dou
   d2 = d2 - k2 * bx.L[2];
   const double dd = d0 * d0 + d1 * d1 + d2 * d2;
   const bool pass = dd < rr;
-  code = ((int)k0 + 512) | (((int)k1 + 512) << 10) | (((int)k2 + 512) << 20);
+  code = ((int)k0 & 1023) | (((int)k1 & 1023) << 10) | (((int)k2 & 1023) << 20);
   if (pass && (fabs(k0) > 511.0 || fabs(k1) > 511.0 || fabs(k2) > 511.0)) raise_flag(b.flags, 2);
   return pass;
 }
@@ -764,6 +764,55 @@ __device__ inline int build_row(const Geom &g, const MdBuf &b, int list, int hal
   return m;
 }
 
+// A wave's interacting entries in its LDS region: the index of j and the COM
+// separation in the pair precision, one 16-byte entry (FP32) or an index and
+// three component arrays (FP64).
+template <typename R>
+struct PairList;
+template <>
+struct PairList<float> {
+  float4 *e;
+  __device__ PairList(unsigned char *reg, int) : e(reinterpret_cast<float4 *>(reg)) {}
+  __device__ void put(int p, int j, double d0, double d1, double d2) {
+    e[p] = make_float4((float)d0, (float)d1, (float)d2, __int_as_float(j));
+  }
+  __device__ void get(int p, int &j, float (&d)[3]) const {
+    const float4 v = e[p];
+    d[0] = v.x;
+    d[1] = v.y;
+    d[2] = v.z;
+    j = __float_as_int(v.w);
+  }
+};
+template <>
+struct PairList<double> {
+  int *j_;
+  double *d_;
+  int stride;
+  __device__ PairList(unsigned char *reg, int cap)
+      : j_(reinterpret_cast<int *>(reg)),
+        d_(reinterpret_cast<double *>(reg + (4 * cap + 15) / 16 * 16)),
+        stride((8 * cap + 15) / 16 * 2) {}
+  __device__ void put(int p, int j, double d0, double d1, double d2) {
+    j_[p] = j;
+    d_[p] = d0;
+    d_[stride + p] = d1;
+    d_[2 * stride + p] = d2;
+  }
+  __device__ void get(int p, int &j, double (&d)[3]) const {
+    j = j_[p];
+    d[0] = d_[p];
+    d[1] = d_[stride + p];
+    d[2] = d_[2 * stride + p];
+  }
+};
+
+// image shift of axis A in a row entry's code (10-bit signed fields)
+template <int A>
+__device__ inline int shift_of(int code) {
+  return (int)((unsigned)code << (22 - 10 * A)) >> 22;
+}
+
 // The pair forces on molecule i by its wave: its row is rebuilt if a rebuild
 // is due, the row's pairs within rc are compacted into the wave's LDS region
 // `reg`, then evaluated.  The results are each lane's sums over its own pairs
@@ -783,7 +832,6 @@ __device__ __forceinline__ void pair_phase(const Geom &g, const MdBuf &b, const 
   const double *rec = b.rec + (size_t)half * g.n * b.rs;
   const int *nj = b.nbr_j + (size_t)i * cap;
   const int *nc = b.nbr_code + (size_t)i * cap;
-  constexpr int kIdle = 512 | (512 << 10) | (512 << 20);  // zero shift
   // the first round of row entries is fetched with the row length (or
   // right after a rebuild)
   int jj[4], cc[4];
@@ -798,7 +846,7 @@ __device__ __forceinline__ void pair_phase(const Geom &g, const MdBuf &b, const 
   for (int u = 0; u < 4; u++) {
     const int k = 64 * u + lane;
     jj[u] = k < cap ? nj[k] : i;
-    cc[u] = k < cap ? nc[k] : kIdle;
+    cc[u] = k < cap ? nc[k] : 0;
   }
   // entries at or past the row length hold stale or never-written values:
   // they are replaced before any of them forms an address
@@ -806,32 +854,31 @@ __device__ __forceinline__ void pair_phase(const Geom &g, const MdBuf &b, const 
   for (int u = 0; u < 4; u++) {
     if (64 * u + lane >= m) {
       jj[u] = i;
-      cc[u] = kIdle;
+      cc[u] = 0;
     }
   }
   const double *reci = rec + (size_t)i * b.rs;
   const double xi = reci[0], yi = reci[1], zi = reci[2];
   // pass 1: the reference's FP64 interaction test on every row entry; the
   // entries that pass are compacted in row order into LDS
-  int *cj = reinterpret_cast<int *>(reg);
-  R *dv = reinterpret_cast<R *>(reg + (4 * cap + 15) / 16 * 16);
-  const int dstride = (int)(((size_t)cap * sizeof(R) + 15) / 16 * 16 / sizeof(R));
+  PairList<R> pl(reg, cap);
   wsync();  // the sort buffers of build_row share this region
   int np = 0;
   // four entries per lane per round: the index loads, then the record
-  // loads, are in flight together
+  // loads, are in flight together; whole waves past the row are skipped
   for (int k0 = 0; k0 < m; k0 += 256) {
     if (k0 > 0) {
 #pragma unroll
       for (int u = 0; u < 4; u++) {
         const int k = k0 + 64 * u + lane;
         jj[u] = k < m ? nj[k] : i;
-        cc[u] = k < m ? nc[k] : kIdle;
+        cc[u] = k < m ? nc[k] : 0;
       }
     }
     double xj[4], yj[4], zj[4];
 #pragma unroll
     for (int u = 0; u < 4; u++) {
+      if (k0 + 64 * u >= m) break;
       const double *recj = rec + (size_t)jj[u] * b.rs;
       xj[u] = recj[0];
       yj[u] = recj[1];
@@ -839,22 +886,14 @@ __device__ __forceinline__ void pair_phase(const Geom &g, const MdBuf &b, const 
     }
 #pragma unroll
     for (int u = 0; u < 4; u++) {
+      if (k0 + 64 * u >= m) break;
       const int code = cc[u];
-      const double ox = (double)((code & 1023) - 512) * bl.L[0];
-      const double oy = (double)(((code >> 10) & 1023) - 512) * bl.L[1];
-      const double oz = (double)(((code >> 20) & 1023) - 512) * bl.L[2];
-      const double d0 = (xi - xj[u]) - ox;
-      const double d1 = (yi - yj[u]) - oy;
-      const double d2 = (zi - zj[u]) - oz;
+      const double d0 = (xi - xj[u]) - (double)shift_of<0>(code) * bl.L[0];
+      const double d1 = (yi - yj[u]) - (double)shift_of<1>(code) * bl.L[1];
+      const double d2 = (zi - zj[u]) - (double)shift_of<2>(code) * bl.L[2];
       const bool pass = k0 + 64 * u + lane < m && d0 * d0 + d1 * d1 + d2 * d2 < g.rc2;
       const unsigned long long mask = __ballot(pass);
-      if (pass) {
-        const int pos = np + __popcll(mask & ((1ull << lane) - 1ull));
-        cj[pos] = jj[u];
-        dv[pos] = R(d0);
-        dv[dstride + pos] = R(d1);
-        dv[2 * dstride + pos] = R(d2);
-      }
+      if (pass) pl.put(np + __popcll(mask & ((1ull << lane) - 1ull)), jj[u], d0, d1, d2);
       np += __popcll(mask);
     }
   }
@@ -867,7 +906,7 @@ __device__ __forceinline__ void pair_phase(const Geom &g, const MdBuf &b, const 
   R(&Fr)[3] = o.F;
   R(&Tr)[3] = o.T;
   R(&vr)[9] = o.v;
-  auto eval = [&](int j, R d0, R d1, R d2, const R (&rj)[T::NS][3]) {
+  auto eval = [&](R d0, R d1, R d2, const R (&rj)[T::NS][3]) {
     R Fp[3], Tp[3];
     const R e = pair_on_i<M, R>(pk, d0 * d0 + d1 * d1 + d2 * d2, d0, d1, d2, ri, rj, Fp, Tp);
     Fr[0] += Fp[0]; Fr[1] += Fp[1]; Fr[2] += Fp[2];
@@ -882,12 +921,15 @@ __device__ __forceinline__ void pair_phase(const Geom &g, const MdBuf &b, const 
   };
   for (int k0 = 0; k0 < np; k0 += 128) {
     const int ka = k0 + lane, kb = k0 + 64 + lane;
-    const int ja = ka < np ? cj[ka] : i, jb = kb < np ? cj[kb] : i;
+    R da[3] = {R(0), R(0), R(0)}, db[3] = {R(0), R(0), R(0)};
+    int ja = i, jb = i;
+    if (ka < np) pl.get(ka, ja, da);
+    if (kb < np) pl.get(kb, jb, db);
     R ra[T::NS][3], rb[T::NS][3];
     RecSites<M, R>::load(rec + (size_t)ja * b.rs, ra);
     RecSites<M, R>::load(rec + (size_t)jb * b.rs, rb);
-    if (ka < np) eval(ja, dv[ka], dv[dstride + ka], dv[2 * dstride + ka], ra);
-    if (kb < np) eval(jb, dv[kb], dv[dstride + kb], dv[2 * dstride + kb], rb);
+    if (ka < np) eval(da[0], da[1], da[2], ra);
+    if (kb < np) eval(db[0], db[1], db[2], rb);
   }
 }
 
@@ -899,6 +941,14 @@ __device__ inline void pair_zero(PairOut<R> &o) {
 #pragma unroll
   for (int q = 0; q < 9; q++) o.v[q] = R(0);
   o.npair = o.nlist = 0;
+}
+
+// The wave's force and lab torque of its molecule: lane l < 6 component l.
+template <typename R>
+__device__ inline double force_torque(const PairOut<R> &o, int lane) {
+  const double v[6] = {(double)o.F[0], (double)o.F[1], (double)o.F[2],
+                       (double)o.T[0], (double)o.T[1], (double)o.T[2]};
+  return wsum_six(v, lane);
 }
 
 // each lane's energy and virial into its wave's LDS region [10][64], which
@@ -949,30 +999,17 @@ __device__ __forceinline__ void md_main_body(const Geom &g, const MdBuf &b, cons
   pair_zero(o);
   if (i < n) {
     pair_phase<M, R, BOX>(g, b, pk, b.flags[2 + parity], parity, 0, i, lane, reg, o, [] {});
-    double F[3], Ti[3];
-#pragma unroll
-    for (int a = 0; a < 3; a++) {
-      F[a] = wsum63((double)o.F[a]);
-      Ti[a] = wsum63((double)o.T[a]);
-    }
-    if (lane == 63) {
-      if (out) {
-        // molecule force (lab) and body torque, as rigid_collectforce
-        double t[9];
-        for (int a = 0; a < 9; a++) t[a] = b.tmat[a * n + i];
-        out[i] = F[0];
-        out[n + i] = F[1];
-        out[2 * n + i] = F[2];
-        out[3 * n + i] = t[0] * Ti[0] + t[3] * Ti[1] + t[6] * Ti[2];
-        out[4 * n + i] = t[1] * Ti[0] + t[4] * Ti[1] + t[7] * Ti[2];
-        out[5 * n + i] = t[2] * Ti[0] + t[5] * Ti[1] + t[8] * Ti[2];
-      } else {
-#pragma unroll
-        for (int a = 0; a < 3; a++) {
-          b.frc[a * n + i] = F[a];
-          b.frc[(3 + a) * n + i] = Ti[a];
-        }
+    const double ft = force_torque(o, lane);
+    if (out) {
+      // molecule force (lab) and body torque, as rigid_collectforce
+      const double t0 = __shfl(ft, 3, 64), t1 = __shfl(ft, 4, 64), t2 = __shfl(ft, 5, 64);
+      if (lane < 3) {
+        const double *t = b.tmat + i;
+        out[lane * n + i] = ft;
+        out[(3 + lane) * n + i] = t[lane * n] * t0 + t[(3 + lane) * n] * t1 + t[(6 + lane) * n] * t2;
       }
+    } else if (lane < 6) {
+      b.frc[lane * n + i] = ft;
     }
     wsync();  // every lane has read the compacted entries
   }
@@ -1084,19 +1121,8 @@ __device__ __forceinline__ void md_step_body(const ModelTable &mt, const Geom &g
     pair_phase<M, R, BOX>(g, b, pk, rebuild, st.list, par, blk * 4 + wid, lane, reg, o, park);
   else
     park();
-  double F[3], Ti[3];
-#pragma unroll
-  for (int c = 0; c < 3; c++) {
-    F[c] = wsum63((double)o.F[c]);
-    Ti[c] = wsum63((double)o.T[c]);
-  }
-  if (lane == 63) {
-#pragma unroll
-    for (int c = 0; c < 3; c++) {
-      s_ft[wid][c] = F[c];
-      s_ft[wid][3 + c] = Ti[c];
-    }
-  }
+  const double ft = force_torque(o, lane);
+  if (lane < 6) s_ft[wid][lane] = ft;
   wsync();  // every lane has read the compacted entries
   park_sums(o, reg, lane, s_cnt[wid]);
   __syncthreads();

@@ -55,6 +55,41 @@ __device__ inline double wsum63(double v) {
   return v;
 }
 
+// Lane-wise sum with the lane 32 apart (permlane32_swap) or in the other row
+// of the row pair (permlane16_swap); both lanes get the same bits.
+__device__ inline double swap32_add(double v) {
+  const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+  const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)u, (unsigned)u, false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(u >> 32), (unsigned)(u >> 32), false,
+                                                   false);
+  return __builtin_bit_cast(double, ((unsigned long long)hi[0] << 32) | lo[0]) +
+         __builtin_bit_cast(double, ((unsigned long long)hi[1] << 32) | lo[1]);
+}
+__device__ inline double swap16_add(double v) {
+  const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+  const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)u, (unsigned)u, false, false);
+  const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)(u >> 32), (unsigned)(u >> 32), false,
+                                                   false);
+  return __builtin_bit_cast(double, ((unsigned long long)hi[0] << 32) | lo[0]) +
+         __builtin_bit_cast(double, ((unsigned long long)hi[1] << 32) | lo[1]);
+}
+
+// Sums of six values over the 64 lanes in a fixed order: lane l (l mod 8 < 6)
+// returns the sum of v[l mod 8].  Each of the first three steps also halves
+// the number of values a lane carries (a lane keeps one of two and gives the
+// other away), about 50 instructions where six wsum63 take 108.
+__device__ inline double wsum_six(const double (&v)[6], int lane) {
+  const bool b0 = lane & 1, b1 = lane & 2, b2 = lane & 4;
+  const double p0 = (b0 ? v[1] : v[0]) + dpp_d<0xB1>(b0 ? v[0] : v[1]);
+  const double p1 = (b0 ? v[3] : v[2]) + dpp_d<0xB1>(b0 ? v[2] : v[3]);
+  const double p2 = (b0 ? v[5] : v[4]) + dpp_d<0xB1>(b0 ? v[4] : v[5]);
+  const double q0 = (b1 ? p1 : p0) + dpp_d<0x4E>(b1 ? p0 : p1);
+  const double q1 = p2 + dpp_d<0x4E>(p2);
+  double r = (b2 ? q1 : q0) + dpp_d<0x124>(b2 ? q0 : q1);  // row_ror:4
+  r += dpp_d<0x128>(r);                                    // row_ror:8
+  return swap32_add(swap16_add(r));
+}
+
 // Compensated sums (Knuth's TwoSum): the pair (s, c) holds s + c, the
 // rounding error of every addition carried in c.
 __device__ inline void two_sum_acc(double &s, double &c, double x) {
