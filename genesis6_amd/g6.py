@@ -197,7 +197,7 @@ class System:
 
     def download(self):
         n = self.n
-        com = np.zeros(3 * n); q = np.zeros(20 * n); dx = np.zeros(15 * n); w = np.zeros(15 * n)
+        com = np.empty(3 * n); q = np.empty(20 * n); dx = np.empty(15 * n); w = np.empty(15 * n)
         check(lib().g6_download_state(self.h, com, q, dx, w), "g6_download_state")
         return (com.reshape(3, n).T.copy(), q.reshape(5, 4, n), dx.reshape(5, 3, n),
                 w.reshape(5, 3, n))
