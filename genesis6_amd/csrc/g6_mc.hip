@@ -22,6 +22,7 @@
 #include <vector>
 
 #include "g6_internal.h"
+#include "g6_md_common.h"
 #include "g6_mc_q6.h"
 #include "g6_std.h"
 
@@ -34,7 +35,7 @@ constexpr double kI2J = 10.0, kJ2K = 0.120273;  // PhysConst.F90:48, 56
 // reference (mc2.F90:61, 811): their single-precision values
 constexpr double kIncrement = (double)1.05f, kDeltaMin = (double)0.05f;
 constexpr int kMcThreads = 512;
-constexpr int kMcMaxPer = 4;  // molecules per thread: n <= 2048
+constexpr int kMcMaxPer = 3;  // molecules per thread: n <= 1536
 
 void make_std_table(const ModelTable &m, StdTable *t) { make_std_table(m, m, t); }
 
@@ -378,42 +379,112 @@ __device__ inline double umbrella_potential(double coeffi, double center, double
   return coeffi * ((op - center) * (op - center));
 }
 
-// mc2's trial loop, ntrial trials, one block.  The configuration (COM,
+// mc2's trial loop, ntrial trials, one block.  The chain of trials is serial,
+// so the kernel is bound by the latency of one trial, not by a unit of the
+// chip; what a trial does is spread over the block and overlapped:
+// - Eight waves test two to four molecules a thread against the moved target
+//   and append those within the cutoff to one list; the list's site pairs are
+//   then spread densely, a site pair per lane.  (A molecule's site terms in
+//   the thread that owns it kept about five of 64 lanes busy, in every wave:
+//   5.9 of the 6.0 us a trial took at 1024 TIP4P molecules.)
+// - Two more waves prepare the next trial's proposal meanwhile, one for each
+//   position the stream can be at (a Metropolis draw or none); the eight
+//   waves have the PairInfo rows of both targets in flight.  If the next
+//   target is the one just decided, its proposal is made again.
+// 1024 TIP4P molecules: 6.0 -> 3.4 us a trial.  The configuration (COM,
 // quaternion, step sizes) lives in LDS for the whole call, and the random
 // stream is staged into LDS kMcChunk trials at a time; the only global
-// traffic per trial is the PairInfo row of the target (issued first) and,
-// on acceptance, the PairInfo and configuration write-back.
-constexpr int kMcChunk = 192;                 // trials per staged chunk
-constexpr int kMcStage = kMcChunk * 14 + 2;   // stream entries per chunk
-template <int M, bool UQ6>
-__global__ __launch_bounds__(kMcThreads) void k_mc_trials(McArgs a, StdTable st, int ntrial) {
-  constexpr int NS = StdPattern<M>::NS;
+// traffic per trial are the PairInfo rows and, on acceptance, the PairInfo
+// and configuration write-back.
+constexpr int kMcChunk = 32;   // trials per staged chunk
+// stream entries per chunk: the last trial's next proposal reads up to 14 + 13
+// entries past the chunk's 14 a trial
+constexpr int kMcStage = kMcChunk * 14 + 30;
+constexpr int kMcBlock = kMcThreads + 256;  // and two proposal and two switch waves
+
+constexpr int kMcPropWave = kMcThreads / 64, kMcSwitchWave = kMcPropWave + 2;
+
+struct McProposal {
+  double t[3], q[4], move[3], turn[3], dt;
+  double site[3][kMaxSite];
+  int target;
+};
+
+// a listed molecule: its index and the image shift of its COM vector in box
+// edges (kMcFar: past 16 bits, formed again from the COMs)
+constexpr short kMcFar = -32768;
+struct McListed {
+  unsigned short j;
+  short image[3];
+};
+static_assert(sizeof(McListed) == sizeof(double), "an entry's energy takes its place");
+
+// round(x), half away from zero, for |x| < 2^51: adding the number below 1/2
+// reaches the next integer exactly where x is at least half way to it
+__device__ inline double round_away(double x) {
+  return trunc(x + copysign(0.49999999999999994, x));
+}
+
+// sum over the wave, the tree of lane distances 32, 16, 8, 4, 2, 1
+__device__ inline double mc_wave_sum(double v) {
+  v = swap16_add(swap32_add(v));
+  v += dpp_d<0x128>(v);  // row_ror:8
+  v += dpp_d<0x124>(v);  // row_ror:4 of values with period 8: lane distance 4
+  v += dpp_d<0x4E>(v);
+  return v + dpp_d<0xB1>(v);
+}
+
+// UMB: 0 without umbrellas, 1 with them, 2 with the Q6 umbrella among them
+template <int M, int UMB>
+__global__ __launch_bounds__(kMcBlock) void k_mc_trials(McArgs a, StdTable st, int ntrial) {
+  using P = StdPattern<M>;
+  constexpr int NS = P::NS, NT = P::NT;
+  constexpr int PPW = 64 / NT;  // listed molecules a wave takes at once
+  static_assert(PPW >= 1, "a molecule's site pairs fit a wave");
   extern __shared__ __align__(16) double s_mem[];
   const int n = a.n;
   double *l_com = s_mem;                      // [3][n]
   double *l_q = l_com + 3 * n;                // [4][n]
   double *l_delta = l_q + 4 * n;              // [n]
   double *l_rtr = l_delta + n;                // [n]
-  double *l_u = l_rtr + n;                    // [kMcStage]
+  // the listed molecules: index
+  // and nearest image, then their energies in place; their switch values
+  double *l_list = l_rtr + n;                 // [n]
+  double *l_er = l_list + n;                  // [n]
+  double *l_u = l_er + n;                     // [kMcStage]
   double *l_z = l_u + kMcStage;               // [kMcStage]
-  __shared__ double s_red[kMcThreads / 64];
+  __shared__ double s_red[kMcThreads / 64], s_patch[2], s_step[3];
+  __shared__ double s_term[kMcThreads / 64 + 2][64];
+  __shared__ McProposal s_prop[3];
+  __shared__ int s_cnt;
   // umbrella state: histogram, the trial's change, reference, order
   // parameters now and after the trial, the trial's total energy change
   __shared__ int s_hist[21], s_dh[21], s_abort;
   __shared__ double s_ref[21], s_op[kUmbMax], s_newop[kUmbMax], s_des;
-  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-  const int numb = a.u.numb;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const bool eval = wid < kMcThreads / 64;  // uniform over the wave
+  constexpr bool UQ6 = UMB == 2;
+  const int numb = UMB ? a.u.numb : 0;
   if (numb > 0 && *a.b.uflag != 0) return;  // the tables did not fit
-  for (int k = tid; k < 3 * n; k += kMcThreads) l_com[k] = a.b.com[k];
-  for (int k = tid; k < 4 * n; k += kMcThreads) l_q[k] = a.b.quat[k];
-  for (int k = tid; k < n; k += kMcThreads) {
+  for (int k = tid; k < 3 * n; k += kMcBlock) l_com[k] = a.b.com[k];
+  for (int k = tid; k < 4 * n; k += kMcBlock) l_q[k] = a.b.quat[k];
+  for (int k = tid; k < n; k += kMcBlock) {
     l_delta[k] = a.b.delta[k];
     l_rtr[k] = a.b.rtr[k];
   }
+  // this lane's site pair of a listed molecule (pl of a wave's PPW)
+  const int pl = lane / NT, pu = lane - pl * NT;
+  const StdTerm term = st.t[pu];
+  // this lane's site of a proposal
+  const int ps = lane < NS ? lane : 0;
+  const double bxs = a.bx[ps], bys = a.by[ps], bzs = a.bz[ps];
+  const double rc2 = a.rc * a.rc;
   int pos = 0;    // position in the call's stream
   int base = -1;  // stream position of l_u[0]
   long long nacc = 0;
   double epsum = *a.b.epsum;
+  if (tid == 0) s_cnt = 0;
   if (numb > 0) {
     if (tid < 21) {
       s_hist[tid] = a.u.tri ? a.b.tri_hist[tid] : 0;
@@ -430,35 +501,31 @@ __global__ __launch_bounds__(kMcThreads) void k_mc_trials(McArgs a, StdTable st,
       }
     }
   }
-  bool aborted = false;
-  for (int trial = 0; trial < ntrial; trial++) {
-    if (trial % kMcChunk == 0) {  // stage the next chunk (a trial reads <= 14)
-      __syncthreads();
-      base = pos;
-      for (int k = tid; k < kMcStage; k += kMcThreads) {
-        l_u[k] = a.b.u[base + k];
-        l_z[k] = a.b.z[base + k];
-      }
-      __syncthreads();
-    }
-    const int p = pos - base;
-    const int trial_pos = pos;
-    // target = random_getnext*nmol + 1 (1-based); u = 1 exactly would name
-    // molecule n+1, which the reference does not guard: clamped here
-    int target = (int)(l_u[p] * (double)n + 1.0) - 1;
-    if (target >= n) target = n - 1;
-    double pold[kMcMaxPer];
-#pragma unroll
-    for (int m = 0; m < kMcMaxPer; m++) {
-      const int j = tid + m * kMcThreads;
-      pold[m] = j < n ? a.b.pinfo[(size_t)target * n + j] : 0.0;
-    }
+  // target = random_getnext*nmol + 1 (1-based); u = 1 exactly would name
+  // molecule n+1, which the reference does not guard: clamped here
+  auto target_at = [&](int p) {
+    const int t = (int)(l_u[p] * (double)n + 1.0) - 1;
+    return __builtin_amdgcn_readfirstlane(t >= n ? n - 1 : t);
+  };
+  // the proposal of the trial that starts at stream entry p (one wave), in
+  // two halves about as long as the phases of the other waves they run beside
+  auto propose_turn = [&](McProposal &o, int p) {
+    const int target = target_at(p);
     const double dt = l_delta[target];
     const double dr = l_delta[target] * l_rtr[target];
-    const double rotx = l_z[p + 1] * sqrt(dr * dr) + 0.0;
-    const double roty = l_z[p + 3] * sqrt(dr * dr) + 0.0;
-    const double rotz = l_z[p + 5] * sqrt(dr * dr) + 0.0;
-    const double avgrot = (fabs(rotx) + fabs(roty) + fabs(rotz)) / 3.0;
+    const double sr = sqrt(dr * dr), sd = sqrt(dt * dt);
+    if (lane < 3) {
+      o.turn[lane] = l_z[p + 1 + 2 * lane] * sr + 0.0;
+      o.move[lane] = l_z[p + 7 + 2 * lane] * sd + 0.0;
+    }
+    if (lane == 0) {
+      o.dt = dt;
+      o.target = target;
+    }
+  };
+  auto propose = [&](McProposal &o) {
+    const int target = o.target;
+    const double rotx = o.turn[0], roty = o.turn[1], rotz = o.turn[2];
     // qinfrotator (QuatModule.F90:203-211) + qnormalize (215-223)
     double qa = 1.0, qb = rotx, qc = roty, qd = rotz;
     {
@@ -487,53 +554,200 @@ __global__ __launch_bounds__(kMcThreads) void k_mc_trials(McArgs a, StdTable st,
         qd = -qd;
       }
     }
-    const double deltax = l_z[p + 7] * sqrt(dt * dt) + 0.0;
-    const double deltay = l_z[p + 9] * sqrt(dt * dt) + 0.0;
-    const double deltaz = l_z[p + 11] * sqrt(dt * dt) + 0.0;
-    const double avgtrans = (fabs(deltax) + fabs(deltay) + fabs(deltaz)) / 3.0;
-    pos += 13;
-    const double tx = deltax + l_com[target], ty = deltay + l_com[n + target],
-                 tz = deltaz + l_com[2 * n + target];
-    double sxt[kMaxSite], syt[kMaxSite], szt[kMaxSite];
-    place_sites_t<NS>(a, qa, qb, qc, qd, tx, ty, tz, sxt, syt, szt);
-    // the compressed list of the moved target (radius rc + dt) and dE; the
-    // sites of a listed molecule are placed again from its COM and quaternion
-    const double rr = (a.rc + dt) * (a.rc + dt);
-    double enew[kMcMaxPer], local = 0.0;
-#pragma unroll
-    for (int m = 0; m < kMcMaxPer; m++) {
-      const int j = tid + m * kMcThreads;
-      enew[m] = 0.0;
-      if (j < n) {
-        if (j != target) {
-          double d0 = l_com[j] - tx, d1 = l_com[n + j] - ty, d2 = l_com[2 * n + j] - tz;
-          const double k0 = round(d0 * a.invL) * a.L, k1 = round(d1 * a.invL) * a.L,
-                       k2 = round(d2 * a.invL) * a.L;
-          d0 = d0 - k0;
-          d1 = d1 - k1;
-          d2 = d2 - k2;
-          const double dd = d0 * d0 + d1 * d1 + d2 * d2;
-          if (dd < rr) {
-            const double er = mc_switch(a, dd);
-            double xj[kMaxSite], yj[kMaxSite], zj[kMaxSite];
-            place_sites_t<NS>(a, l_q[j], l_q[n + j], l_q[2 * n + j], l_q[3 * n + j], l_com[j],
-                              l_com[n + j], l_com[2 * n + j], xj, yj, zj);
-            enew[m] = std_energy_t<M>(st, xj, yj, zj, sxt, syt, szt, k0, k1, k2, er);
-          }
+    const double tx = o.move[0] + l_com[target], ty = o.move[1] + l_com[n + target],
+                 tz = o.move[2] + l_com[2 * n + target];
+    double x, y, z;
+    place_site(bxs, bys, bzs, qa, qb, qc, qd, tx, ty, tz, x, y, z);
+    if (lane < NS) {
+      o.site[0][lane] = x;
+      o.site[1][lane] = y;
+      o.site[2][lane] = z;
+    }
+    if (lane == 0) {
+      o.t[0] = tx;
+      o.t[1] = ty;
+      o.t[2] = tz;
+      o.q[0] = qa;
+      o.q[1] = qb;
+      o.q[2] = qc;
+      o.q[3] = qd;
+    }
+  };
+  double pold[kMcMaxPer];
+  int cur = 0;  // the trial's proposal; the other two slots take the next one's
+  bool aborted = false;
+  // the proposals are the longest chain: their waves issue first
+  if (wid == kMcPropWave || wid == kMcPropWave + 1) __builtin_amdgcn_s_setprio(3);
+  for (int trial = 0; trial < ntrial; trial++) {
+    if (trial % kMcChunk == 0) {  // stage the next chunk (a trial reads <= 14)
+      __syncthreads();
+      base = pos;
+      for (int k = tid; k < kMcStage; k += kMcBlock) {
+        l_u[k] = a.b.u[base + k];
+        l_z[k] = a.b.z[base + k];
+      }
+      __syncthreads();
+      if (trial == 0) {
+        if (wid == kMcPropWave) {
+          propose_turn(s_prop[0], 0);
+          wsync();
+          propose(s_prop[0]);
         }
-        local = local + (enew[m] - pold[m]);
+        const int t0 = target_at(0);
+#pragma unroll
+        for (int m = 0; m < kMcMaxPer; m++) {
+          const int j = tid + m * kMcThreads;
+          pold[m] = !UQ6 && eval && j < n ? a.b.pinfo[(size_t)t0 * n + j] : 0.0;
+        }
+        __syncthreads();
       }
     }
+    const int trial_pos = pos;
+    pos += 13;
+    const McProposal &pr = s_prop[cur];
+    const int target = __builtin_amdgcn_readfirstlane(pr.target);
+    // addresses are formed anew in every trial: held over the loop, they and
+    // the constants spill, and a reload from scratch waits for the rows
+    int own = tid;
+    asm volatile("" : "+v"(own));
+    // the next trial's target if this one draws no Metropolis number, if it does
+    const int tn0 = target_at(pos - base), tn1 = target_at(pos + 1 - base);
+    double pn0[kMcMaxPer], pn1[kMcMaxPer], enew[kMcMaxPer];
+    int slot[kMcMaxPer];
+    // the compressed list of the moved target (radius rc + dt), less what the
+    // switch takes to zero
+    // the slot of a proposal wave
+    McProposal &next = s_prop[(cur + 1 + (wid == kMcPropWave + 1)) % 3];
+    if (wid == kMcPropWave || wid == kMcPropWave + 1) {
+      propose_turn(next, pos + wid - kMcPropWave - base);
+    } else if (eval) {
+      const double tx = pr.t[0], ty = pr.t[1], tz = pr.t[2];
+      const double rr = (a.rc + pr.dt) * (a.rc + pr.dt);
+      double dd[kMcMaxPer];
+      McListed e[kMcMaxPer];
+      unsigned long long in[kMcMaxPer];
+      int cnt = 0;
 #pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) local += __shfl_xor(local, d, 64);
-    if (lane == 0) s_red[wid] = local;
+      for (int m = 0; m < kMcMaxPer; m++) {
+        const int j = own + m * kMcThreads;
+        pn0[m] = pn1[m] = 0.0;
+        slot[m] = -1;
+        in[m] = 0;
+        if (m * kMcThreads >= n) continue;
+        if (!UQ6 && j < n) {
+          pn0[m] = (a.b.pinfo + (size_t)tn0 * n)[j];
+          pn1[m] = (a.b.pinfo + (size_t)tn1 * n)[j];
+        }
+        const int jc = j < n ? j : 0;
+        double d0 = l_com[jc] - tx, d1 = l_com[n + jc] - ty, d2 = l_com[2 * n + jc] - tz;
+        const double i0 = round_away(d0 * a.invL), i1 = round_away(d1 * a.invL),
+                     i2 = round_away(d2 * a.invL);
+        d0 = d0 - i0 * a.L;
+        d1 = d1 - i1 * a.L;
+        d2 = d2 - i2 * a.L;
+        dd[m] = d0 * d0 + d1 * d1 + d2 * d2;
+        in[m] = __ballot(j < n && j != target && dd[m] < rr && dd[m] < rc2);
+        const bool far = fmax(fmax(fabs(i0), fabs(i1)), fabs(i2)) > 32767.0;
+        e[m].j = (unsigned short)j;
+        e[m].image[0] = far ? kMcFar : (short)(int)i0;
+        e[m].image[1] = (short)(int)i1;
+        e[m].image[2] = (short)(int)i2;
+        cnt += __popcll(in[m]);
+      }
+      if (cnt > 0) {
+        int at = 0;
+        if (lane == 0) at = atomicAdd(&s_cnt, cnt);
+        at = __builtin_amdgcn_readfirstlane(at);
+#pragma unroll
+        for (int m = 0; m < kMcMaxPer; m++) {
+          if (in[m] >> lane & 1) {
+            slot[m] = at + __popcll(in[m] & ((1ull << lane) - 1ull));
+            reinterpret_cast<McListed *>(l_list)[slot[m]] = e[m];
+            l_er[slot[m]] = dd[m];
+          }
+          at += __popcll(in[m]);
+        }
+      }
+    }
+    __syncthreads();
+    if (wid == kMcPropWave || wid == kMcPropWave + 1) {
+      propose(next);
+    } else {
+      // the new pair energies of dE: the site pairs of PPW listed molecules a
+      // wave at a time, each molecule's added in the order of the term list.
+      // The switch waves, which first take the switch of every listed
+      // molecule, have one turn in three.
+      const int cnt = s_cnt;
+      const bool sw = wid >= kMcSwitchWave;
+      if (sw)
+        for (int k = tid - kMcSwitchWave * 64; k < cnt; k += 128)
+          l_er[k] = mc_switch(a, l_er[k]);
+      const double xt = pr.site[0][term.b], yt = pr.site[1][term.b], zt = pr.site[2][term.b];
+      constexpr int EW = kMcThreads / 64, CY = 2 * EW + 2;  // turns of a cycle
+      const int w = sw ? wid - kMcSwitchWave : wid;
+      for (int g = sw ? 2 * EW + w : w; g * PPW < cnt;
+           // a wave's turns: w, w + EW of every cycle; a switch wave's: 2 EW + w
+           g += sw ? CY : g % CY < EW ? EW : CY - EW) {
+        const int k0 = g * PPW;
+        if (pl < PPW && k0 + pl < cnt) {
+          const McListed c = reinterpret_cast<const McListed *>(l_list)[k0 + pl];
+          const int at = (int)c.j * a.ns + term.a;
+          const double dx = a.b.sx[at] - xt, dy = a.b.sy[at] - yt, dz = a.b.sz[at] - zt;
+          double o0 = c.image[0] * a.L, o1 = c.image[1] * a.L, o2 = c.image[2] * a.L;
+          if (c.image[0] == kMcFar) {
+            o0 = round_away((l_com[c.j] - pr.t[0]) * a.invL) * a.L;
+            o1 = round_away((l_com[n + c.j] - pr.t[1]) * a.invL) * a.L;
+            o2 = round_away((l_com[2 * n + c.j] - pr.t[2]) * a.invL) * a.L;
+          }
+          s_term[sw ? EW + w : w][lane] = std_term(term, dx, dy, dz, o0, o1, o2);
+        }
+        wsync();
+        if (lane < PPW && k0 + lane < cnt) {
+          double ep = 0.0;
+#pragma unroll
+          for (int q = 0; q < NT; q++) ep = ep + s_term[sw ? EW + w : w][lane * NT + q];
+          l_list[k0 + lane] = ep;
+        }
+        wsync();
+      }
+    }
+    __syncthreads();
+    if (eval) {
+      double local = 0.0;
+#pragma unroll
+      for (int m = 0; m < kMcMaxPer; m++) {
+        const int j = own + m * kMcThreads;
+        enew[m] = slot[m] >= 0 ? l_list[slot[m]] * l_er[slot[m]] : 0.0;
+        if (j < n) {
+          // (the Q6 umbrella's trial is long and short of registers)
+          if constexpr (UQ6) pold[m] = (a.b.pinfo + (size_t)target * n)[j];
+          local = local + (enew[m] - pold[m]);
+          if (j == tn0) s_patch[0] = enew[m];
+          if (j == tn1) s_patch[1] = enew[m];
+        }
+      }
+      local = mc_wave_sum(local);
+      if (lane == 0) s_red[wid] = local;
+    } else if (wid == kMcSwitchWave) {
+      // the target's step sizes after either decision
+      s_cnt = 0;
+      const double avgtrans = (fabs(pr.move[0]) + fabs(pr.move[1]) + fabs(pr.move[2])) / 3.0;
+      const double avgrot = (fabs(pr.turn[0]) + fabs(pr.turn[1]) + fabs(pr.turn[2])) / 3.0;
+      const double rt = l_rtr[target];
+      double down = pr.dt / kIncrement;
+      if (down < kDeltaMin) down = kDeltaMin;
+      s_step[0] = down;
+      s_step[1] = pr.dt * kIncrement;
+      s_step[2] = avgtrans * rt < avgrot ? rt * kIncrement : rt / kIncrement;
+    }
+    const double deltax = pr.move[0], deltay = pr.move[1], deltaz = pr.move[2];
     // the triangle rows the trial changes: the target (tid 0) and the
     // molecules of its table (tid 1..nt); tslot = the row's entry of the
     // target, whose vector the move changes
     int trow = -1, tslot = -1;
-    if (a.u.tri) {
+    if (UMB && a.u.tri) {
       const int nt = a.b.tri_nn[target];
-      if (tid <= nt) {
+      if (tid <= nt && eval) {
         trow = tid == 0 ? target : a.b.tri_near[(size_t)target * kTriNear + tid - 1];
         const int m = a.b.tri_nn[trow];
         const double4 *row = reinterpret_cast<const double4 *>(a.b.tri_v) + (size_t)trow * kTriNear;
@@ -593,7 +807,7 @@ __global__ __launch_bounds__(kMcThreads) void k_mc_trials(McArgs a, StdTable st,
         aborted = true;
         break;
       }
-      for (int k = tid; k < n; k += kMcThreads) a.b.q6.dq6[k] = q6_of(a.b.q6, k);
+      for (int k = tid; k < n; k += kMcBlock) a.b.q6.dq6[k] = q6_of(a.b.q6, k);
       __syncthreads();
     }
     double de = 0.0;
@@ -636,8 +850,9 @@ __global__ __launch_bounds__(kMcThreads) void k_mc_trials(McArgs a, StdTable st,
     if (de < 0.0) {
       accept = true;
     } else {
-      const double ratio = exp(-(de * kI2J * kJ2K) * a.beta);
-      accept = l_u[pos - base] < ratio;
+      // the stream's smallest number is 2^-31: exp(-22) is below it
+      const double x = (de * kI2J * kJ2K) * a.beta;
+      accept = !(x > 22.0) && l_u[pos - base] < exp(-x);
       pos += 1;
     }
     if (numb > 0) {
@@ -668,47 +883,63 @@ __global__ __launch_bounds__(kMcThreads) void k_mc_trials(McArgs a, StdTable st,
           q6_reject(a.b.q6, qt, target, lane);
       }
     }
+    const int sel = pos - trial_pos - 13, tnext = sel ? tn1 : tn0;
     if (accept) {
       nacc += 1;
       epsum = epsum + deltae;
+    }
+    if (eval) {
 #pragma unroll
       for (int m = 0; m < kMcMaxPer; m++) {
-        const int j = tid + m * kMcThreads;
-        if (j < n) {
-          a.b.pinfo[(size_t)j * n + target] = enew[m];
-          a.b.pinfo[(size_t)target * n + j] = enew[m];
+        const int j = own + m * kMcThreads;
+        // the next target's row, with what this trial changes in it
+        if constexpr (!UQ6) pold[m] = sel ? pn1[m] : pn0[m];
+        if (accept && j < n) {
+          (a.b.pinfo + target)[(unsigned)(j * n)] = enew[m];
+          (a.b.pinfo + (size_t)target * n)[j] = enew[m];
+          if (UQ6) continue;
+          if (tnext == target)
+            pold[m] = enew[m];
+          else if (j == target)
+            pold[m] = s_patch[sel];
         }
       }
-      if (tid == 0) {
-        l_com[target] = tx;
-        l_com[n + target] = ty;
-        l_com[2 * n + target] = tz;
-        l_q[target] = qa;
-        l_q[n + target] = qb;
-        l_q[2 * n + target] = qc;
-        l_q[3 * n + target] = qd;
-        l_delta[target] = l_delta[target] * kIncrement;
-        if (avgtrans * l_rtr[target] < avgrot)
-          l_rtr[target] = l_rtr[target] * kIncrement;
-        else
-          l_rtr[target] = l_rtr[target] / kIncrement;
-      } else if (tid == 64) {  // the site positions the host may read back
-#pragma unroll
-        for (int s = 0; s < NS; s++) {
-          a.b.sx[(size_t)target * a.ns + s] = sxt[s];
-          a.b.sy[(size_t)target * a.ns + s] = syt[s];
-          a.b.sz[(size_t)target * a.ns + s] = szt[s];
+    } else if (wid == kMcSwitchWave) {
+      if (lane == 0) {
+        l_delta[target] = s_step[accept];
+        if (accept) {
+          l_com[target] = pr.t[0];
+          l_com[n + target] = pr.t[1];
+          l_com[2 * n + target] = pr.t[2];
+          l_q[target] = pr.q[0];
+          l_q[n + target] = pr.q[1];
+          l_q[2 * n + target] = pr.q[2];
+          l_q[3 * n + target] = pr.q[3];
+          l_rtr[target] = s_step[2];
         }
       }
-    } else if (tid == 0) {
-      l_delta[target] = l_delta[target] / kIncrement;
-      if (l_delta[target] < kDeltaMin) l_delta[target] = kDeltaMin;
+    } else if (wid == kMcSwitchWave + 1 && accept && lane < NS) {
+      // the site positions the next trials' terms (and the host) read
+      a.b.sx[(size_t)target * a.ns + lane] = pr.site[0][lane];
+      a.b.sy[(size_t)target * a.ns + lane] = pr.site[1][lane];
+      a.b.sz[(size_t)target * a.ns + lane] = pr.site[2][lane];
     }
     __syncthreads();
+    cur = cur + 1 + sel < 3 ? cur + 1 + sel : cur - 2 + sel;
+    // the next trial moves the molecule this one decided on: its proposal was
+    // made from the state before the decision
+    if (tnext == target && trial + 1 < ntrial) {
+      if (wid == kMcPropWave) {
+        propose_turn(s_prop[cur], pos - base);
+        wsync();
+        propose(s_prop[cur]);
+      }
+      __syncthreads();
+    }
   }
-  for (int k = tid; k < 3 * n; k += kMcThreads) a.b.com[k] = l_com[k];
-  for (int k = tid; k < 4 * n; k += kMcThreads) a.b.quat[k] = l_q[k];
-  for (int k = tid; k < n; k += kMcThreads) {
+  for (int k = tid; k < 3 * n; k += kMcBlock) a.b.com[k] = l_com[k];
+  for (int k = tid; k < 4 * n; k += kMcBlock) a.b.quat[k] = l_q[k];
+  for (int k = tid; k < n; k += kMcBlock) {
     a.b.delta[k] = l_delta[k];
     a.b.rtr[k] = l_rtr[k];
   }
@@ -721,8 +952,10 @@ __global__ __launch_bounds__(kMcThreads) void k_mc_trials(McArgs a, StdTable st,
   }
 }
 
-// LDS bytes of k_mc_trials for n molecules
-static size_t mc_lds(int n) { return sizeof(double) * ((size_t)9 * n + 2 * kMcStage); }
+// LDS bytes of k_mc_trials for n molecules, and the largest n it takes (11 n
+// doubles, the staged stream and 6 KiB of static LDS fit the 160 KiB of a CU)
+static size_t mc_lds(int n) { return sizeof(double) * ((size_t)11 * n + 2 * kMcStage); }
+constexpr int kMcMaxN = 1535;
 
 static McArgs mc_args(const System &s) {
   McArgs a{};
@@ -794,7 +1027,7 @@ int g6_mc_begin(g6_handle h, double temp, uint32_t seed, const double *delta,
   if (!s || !(temp > 0) || !delta || !rtratio) return G6_EARG;
   if (!is_cubic(*s)) return G6_EARG;  // mc2's trial loop runs cubic boxes here
   const int n = s->n, ns = s->ns;
-  if (n > kMcThreads * kMcMaxPer || mc_lds(n) > 150 * 1024) return G6_EARG;
+  if (n > kMcMaxN) return G6_EARG;
   mc_free(*s);
   McBuf &m = s->mc;
   auto A = [](void **p, size_t b) { return hipMalloc(p, b > 0 ? b : 8); };
@@ -893,14 +1126,16 @@ int g6_mc_trials(g6_handle h, int ntrial, long long *naccept) {
   auto launch = [&](auto kern) {
     attr = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
                                (int)lds);
-    if (attr == hipSuccess) kern<<<1, kMcThreads, lds, s->stream>>>(a, s->std, ntrial);
+    if (attr == hipSuccess) kern<<<1, kMcBlock, lds, s->stream>>>(a, s->std, ntrial);
   };
   std_model(s->model, [&](auto m) {
     constexpr int M = decltype(m)::value;
     if (s->mc_umb.q6)
-      launch(k_mc_trials<M, true>);
+      launch(k_mc_trials<M, 2>);
+    else if (s->mc_umb.numb > 0)
+      launch(k_mc_trials<M, 1>);
     else
-      launch(k_mc_trials<M, false>);
+      launch(k_mc_trials<M, 0>);
   });
   G6_CHECK(attr);
   G6_CHECK(hipGetLastError());

@@ -144,6 +144,18 @@ __device__ inline double std_energy(const StdTable &st, const double *xi, const 
   return ep * er;
 }
 
+// one site pair of std_energy: the site vector before the image shift o
+__device__ inline double std_term(const StdTerm &s, double dx, double dy, double dz, double ox,
+                                  double oy, double oz) {
+  dx = dx - ox;
+  dy = dy - oy;
+  dz = dz - oz;
+  const double dd = 1.0 / (dx * dx + dy * dy + dz * dz);
+  const double d6 = dd * dd * dd, d12 = d6 * d6;
+  const double c = s.qq * sqrt(dd), w = s.aa * d12;
+  return s.kind == 2 ? c : (s.kind == 1 ? c + w : w) + s.bb * d6;
+}
+
 // std_energy with the term list of model M: j's sites from memory, the
 // other molecule's sites in registers (constant indices)
 template <int M>
@@ -236,6 +248,24 @@ __device__ inline void place_sites(const A &a, double qa, double qb, double qc, 
     y[s] = cy + r1;
     z[s] = cz + r2;
   }
+}
+
+// one site of place_sites: body coordinates (bx, by, bz)
+__device__ inline void place_site(double bx, double by, double bz, double qa, double qb, double qc,
+                                  double qd, double cx, double cy, double cz, double &x,
+                                  double &y, double &z) {
+  const double t0 = (qa * qa + qb * qb - (qc * qc + qd * qd));
+  const double t1 = -2.0 * (qa * qd + qb * qc);
+  const double t2 = 2.0 * (qb * qd - qa * qc);
+  const double t3 = 2.0 * (qa * qd - qb * qc);
+  const double t4 = qa * qa + qc * qc - (qb * qb + qd * qd);
+  const double t5 = -2.0 * (qa * qb + qc * qd);
+  const double t6 = 2.0 * (qa * qc + qb * qd);
+  const double t7 = 2.0 * (qa * qb - qc * qd);
+  const double t8 = qa * qa + qd * qd - (qb * qb + qc * qc);
+  x = cx + (t0 * bx + t1 * by + t2 * bz);
+  y = cy + (t3 * bx + t4 * by + t5 * bz);
+  z = cz + (t6 * bx + t7 * by + t8 * bz);
 }
 
 // place_sites with a constant site count (the trial kernel's registers)
