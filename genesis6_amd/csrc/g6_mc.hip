@@ -419,12 +419,6 @@ struct McListed {
 };
 static_assert(sizeof(McListed) == sizeof(double), "an entry's energy takes its place");
 
-// round(x), half away from zero, for |x| < 2^51: adding the number below 1/2
-// reaches the next integer exactly where x is at least half way to it
-__device__ inline double round_away(double x) {
-  return trunc(x + copysign(0.49999999999999994, x));
-}
-
 // sum over the wave, the tree of lane distances 32, 16, 8, 4, 2, 1
 __device__ inline double mc_wave_sum(double v) {
   v = swap16_add(swap32_add(v));

@@ -113,6 +113,13 @@ __device__ inline void rowsum16_dd(double &s, double &c) {
   dd_add(s, c, dpp_d<0x140>(s), dpp_d<0x140>(c));
 }
 
+// round(x), half away from zero, for |x| < 2^51: adding the number below 1/2
+// reaches the next integer exactly where x is at least half way to it (three
+// operations, eight in round())
+__device__ inline double round_away(double x) {
+  return trunc(x + copysign(0.49999999999999994, x));
+}
+
 __device__ inline void wsync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();

@@ -304,9 +304,9 @@ __global__ __launch_bounds__(kMixThreads) void k_mix_cross(CrossArgs x, MixClose
         for (int u = 0; u < 4; u++) {
           const int j = j0 + GL * u + sub;
           double d0 = xi - xj[u], d1 = yi - yj[u], d2 = zi - zj[u];
-          d0 = d0 - round(d0 * x.invL[0]) * x.L[0];
-          d1 = d1 - round(d1 * x.invL[1]) * x.L[1];
-          d2 = d2 - round(d2 * x.invL[2]) * x.L[2];
+          d0 = d0 - round_away(d0 * x.invL[0]) * x.L[0];
+          d1 = d1 - round_away(d1 * x.invL[1]) * x.L[1];
+          d2 = d2 - round_away(d2 * x.invL[2]) * x.L[2];
           const bool pass = live && j < je && d0 * d0 + d1 * d1 + d2 * d2 < x.rc2;
           unsigned long long mask = __ballot(pass);
           if constexpr (GL < 64) mask = (mask >> (grp * GL)) & ((1ull << GL) - 1ull);
@@ -324,7 +324,7 @@ __global__ __launch_bounds__(kMixThreads) void k_mix_cross(CrossArgs x, MixClose
         const double *rj = x.recj + (size_t)j * x.rs;
         // the COM vector again, by pass 1's expression (the same bits)
         double d[3] = {xi - x.comj[j], yi - x.comj[x.nj + j], zi - x.comj[2 * x.nj + j]};
-        for (int a = 0; a < 3; a++) d[a] = d[a] - round(d[a] * x.invL[a]) * x.L[a];
+        for (int a = 0; a < 3; a++) d[a] = d[a] - round_away(d[a] * x.invL[a]) * x.L[a];
         const double dd = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
         // cutoff_func (CutoffModule.F90:38-59) on the COM distance
         double hh = 1.0, dh = 0.0;
@@ -353,10 +353,11 @@ __global__ __launch_bounds__(kMixThreads) void k_mix_cross(CrossArgs x, MixClose
           const double dx = (d[0] + si[a][0]) - sj[b][0];
           const double dy = (d[1] + si[a][1]) - sj[b][1];
           const double dz = (d[2] + si[a][2]) - sj[b][2];
-          const double inv2 = 1.0 / (dx * dx + dy * dy + dz * dz);
+          double inv2, inv1;
+          inv_r<double>(dx * dx + dy * dy + dz * dz, inv2, inv1);
           double e0 = 0.0, f0 = 0.0;
           if (tm.kind != 3) {
-            const double ec = tm.qq * sqrt(inv2);
+            const double ec = tm.qq * inv1;
             e0 = ec;
             f0 = ec * inv2;
           }
