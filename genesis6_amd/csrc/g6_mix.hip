@@ -101,32 +101,32 @@ __device__ inline void mix_close_body(const MixClose &c, int mode, int parity) {
   const int wid = threadIdx.x >> 6;
   {
     // pair partials of each set, then kinetic partials of each component,
-    // per thread in block order, then over the wave and the four waves
-    double v[kMixRed];
+    // per thread in block order, then over the wave and the four waves.  A
+    // set at a time: all 56 sums at once held 112 registers, which the cross
+    // kernel this rides in had to have too.
+    auto sums = [&](const double *p, int nb, int stride, auto len, int at) {
+      constexpr int N = decltype(len)::value;
+      double v[N];
 #pragma unroll
-    for (int q = 0; q < kMixRed; q++) v[q] = 0.0;
-    if (mode & 1) {
-      for (int k = threadIdx.x; k < c.nblk_main_a; k += 256)
+      for (int q = 0; q < N; q++) v[q] = 0.0;
+      if (mode & 1)
+#pragma unroll 2
+        for (int k = threadIdx.x; k < nb; k += 256)
 #pragma unroll
-        for (int q = 0; q < 12; q++) v[q] += c.bpart_a[(size_t)k * kBP + q];
-      for (int k = threadIdx.x; k < c.nblk_main_b; k += 256)
+          for (int q = 0; q < N; q++) v[q] += p[(size_t)k * stride + q];
 #pragma unroll
-        for (int q = 0; q < 12; q++) v[12 + q] += c.bpart_b[(size_t)k * kBP + q];
-      for (int k = threadIdx.x; k < c.nblk_x; k += 256)
+      for (int q = 0; q < N; q++) v[q] = wsum63(v[q]);
+      if ((threadIdx.x & 63) == 63)
 #pragma unroll
-        for (int q = 0; q < 12; q++) v[24 + q] += c.bpart_x[(size_t)k * kBP + q];
-      for (int k = threadIdx.x; k < c.nblk_pre_a; k += 256)
-#pragma unroll
-        for (int q = 0; q < kEkLen; q++) v[36 + q] += c.a.blockek[(size_t)k * kEkLen + q];
-      for (int k = threadIdx.x; k < c.nblk_pre_b; k += 256)
-#pragma unroll
-        for (int q = 0; q < kEkLen; q++) v[36 + kEkLen + q] += c.b.blockek[(size_t)k * kEkLen + q];
-    }
-#pragma unroll
-    for (int q = 0; q < kMixRed; q++) v[q] = wsum63(v[q]);
-    if ((threadIdx.x & 63) == 63)
-#pragma unroll
-      for (int q = 0; q < kMixRed; q++) s_red[wid][q] = v[q];
+        for (int q = 0; q < N; q++) s_red[wid][at + q] = v[q];
+    };
+    const std::integral_constant<int, 12> pairs;
+    const std::integral_constant<int, kEkLen> kin;
+    sums(c.bpart_a, c.nblk_main_a, kBP, pairs, 0);
+    sums(c.bpart_b, c.nblk_main_b, kBP, pairs, 12);
+    sums(c.bpart_x, c.nblk_x, kBP, pairs, 24);
+    sums(c.a.blockek, c.nblk_pre_a, kEkLen, kin, 36);
+    sums(c.b.blockek, c.nblk_pre_b, kEkLen, kin, 36 + kEkLen);
   }
   if (mode & 12) {
     const int p0 = (mode & 8) ? 0 : 1 - parity, p1 = (mode & 8) ? 1 : 1 - parity;
@@ -287,23 +287,36 @@ __global__ __launch_bounds__(kMixThreads) void k_mix_cross(CrossArgs x, MixClose
     const double xi = ri[0], yi = ri[1], zi = ri[2];
     int *cj = s_j[wid] + grp * CAP;
     int np = 0;  // this group's entries (equal over its lanes)
+    // a chunk's COMs are loaded while the chunk before is tested: with few
+    // waves in flight a load's latency was most of a chunk's time
+    double xj[4], yj[4], zj[4];
+    auto fetch = [&](int j0) {
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        const int jr = j0 + GL * u + sub, j = jr < je ? jr : 0;
+        xj[u] = x.comj[j];
+        yj[u] = x.comj[x.nj + j];
+        zj[u] = x.comj[2 * x.nj + j];
+      }
+    };
+    fetch(jb);
     for (int j0 = jb; j0 < je; j0 += CH) {
       // pass 1: the COM test on the chunk's candidates, four per lane with
       // their loads in flight together; the pairs within rc are appended in
       // index order to this wave's LDS rows
       {
-        double xj[4], yj[4], zj[4];
+        double d[4][3];
 #pragma unroll
         for (int u = 0; u < 4; u++) {
-          const int jr = j0 + GL * u + sub, j = jr < je ? jr : 0;
-          xj[u] = x.comj[j];
-          yj[u] = x.comj[x.nj + j];
-          zj[u] = x.comj[2 * x.nj + j];
+          d[u][0] = xi - xj[u];
+          d[u][1] = yi - yj[u];
+          d[u][2] = zi - zj[u];
         }
+        fetch(j0 + CH);
 #pragma unroll
         for (int u = 0; u < 4; u++) {
           const int j = j0 + GL * u + sub;
-          double d0 = xi - xj[u], d1 = yi - yj[u], d2 = zi - zj[u];
+          double d0 = d[u][0], d1 = d[u][1], d2 = d[u][2];
           d0 = d0 - round_away(d0 * x.invL[0]) * x.L[0];
           d1 = d1 - round_away(d1 * x.invL[1]) * x.L[1];
           d2 = d2 - round_away(d2 * x.invL[2]) * x.L[2];
