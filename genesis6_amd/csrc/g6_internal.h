@@ -16,9 +16,9 @@
 //     unwrapped, so |k| can exceed 1).  The -0.0 shift that dnint gives for
 //     small negative differences is stored as 0: x - (-0.0) and x - 0.0 are
 //     equal for every x but a zero x, whose sign no force term can see
-//   blockpart[2][nblk_md][16], blockek[pre waves][10]: per-block energy/virial
-//     and per-wave kinetic partials, reduced in a fixed order by the step
-//     close (one block)
+//   blockpart[2][nblk_md][16], stepek[2][groups of 4 molecules][10]: per-block
+//     energy/virial and per-group kinetic partials, reduced in a fixed order by
+//     the step close (one block)
 // Reference-list entry point (g6_pairlist.hip): cell residents in molecule
 //   order and the half-shell candidate rows of Grid_NeighborList
 //   (GridModule.F90:557-752) with counts cnt[2n], offsets off[2n+1], and the

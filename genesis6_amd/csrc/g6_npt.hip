@@ -39,6 +39,7 @@
 #include <vector>
 
 #include "g6_internal.h"
+#include "g6_md_common.h"
 #include "g6_mlp.h"
 #include "g6_std.h"
 
@@ -174,9 +175,9 @@ __device__ inline int cell_at(double x, double y, double z, double L, int nd) {
   int jc[3];
   for (int a = 0; a < 3; a++) {
     double d = c[a];
-    const double o = round(d * invL) * L;
+    const double o = round_away(d * invL) * L;
     d = d - o;
-    int j = (int)round(d * cellinv);
+    int j = (int)round_away(d * cellinv);
     if (j < 0) j += nd;
     j = ((j % nd) + nd) % nd;
     jc[a] = j;
@@ -340,7 +341,7 @@ __device__ inline void volume_row(const NptArgs &A, const StdTable &st, int w, i
     double e = 0.0;
     if (j > w) {
       double d0 = xi - A.com2[j], d1 = yi - A.com2[n + j], d2 = zi - A.com2[2 * n + j];
-      const double k0 = round(d0 * invL) * L, k1 = round(d1 * invL) * L, k2 = round(d2 * invL) * L;
+      const double k0 = round_away(d0 * invL) * L, k1 = round_away(d1 * invL) * L, k2 = round_away(d2 * invL) * L;
       d0 = d0 - k0;
       d1 = d1 - k1;
       d2 = d2 - k2;
@@ -408,7 +409,7 @@ __global__ __launch_bounds__(256) void k_npt_eval(NptArgs A, StdTable st, int da
     // PairInfo orientation: the lower index first, d = com_lo - com_hi
     double d0 = i < j ? xi - xj : xj - xi, d1 = i < j ? yi - yj : yj - yi,
            d2 = i < j ? zi - zj : zj - zi;
-    const double k0 = round(d0 * invL) * L, k1 = round(d1 * invL) * L, k2 = round(d2 * invL) * L;
+    const double k0 = round_away(d0 * invL) * L, k1 = round_away(d1 * invL) * L, k2 = round_away(d2 * invL) * L;
     d0 = d0 - k0;
     d1 = d1 - k1;
     d2 = d2 - k2;
@@ -688,9 +689,9 @@ __global__ __launch_bounds__(256) void k_nbl(NptArgs A, int always) {
     if (j < n && j != i) {
       double dx = A.sx[(size_t)j * ns] - ox, dy = A.sy[(size_t)j * ns] - oy,
              dz = A.sz[(size_t)j * ns] - oz;
-      dx = dx - round(dx * invL) * L;
-      dy = dy - round(dy * invL) * L;
-      dz = dz - round(dz * invL) * L;
+      dx = dx - round_away(dx * invL) * L;
+      dy = dy - round_away(dy * invL) * L;
+      dz = dz - round_away(dz * invL) * L;
       in = dx * dx + dy * dy + dz * dz < kNblR * kNblR;
     }
     const unsigned long long m = __ballot(in);
@@ -929,7 +930,7 @@ __global__ __launch_bounds__(256) void k_npt_pairinfo(NptArgs A, StdTable st, do
     double e = 0.0;
     if (j > w) {
       double d0 = xi - A.com[j], d1 = yi - A.com[n + j], d2 = zi - A.com[2 * n + j];
-      const double k0 = round(d0 * invL) * L, k1 = round(d1 * invL) * L, k2 = round(d2 * invL) * L;
+      const double k0 = round_away(d0 * invL) * L, k1 = round_away(d1 * invL) * L, k2 = round_away(d2 * invL) * L;
       d0 = d0 - k0;
       d1 = d1 - k1;
       d2 = d2 - k2;
