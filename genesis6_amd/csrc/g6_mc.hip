@@ -391,7 +391,7 @@ __device__ inline double umbrella_potential(double coeffi, double center, double
 //   position the stream can be at (a Metropolis draw or none); the eight
 //   waves have the PairInfo rows of both targets in flight.  If the next
 //   target is the one just decided, its proposal is made again.
-// 1024 TIP4P molecules: 6.0 -> 3.4 us a trial.  The configuration (COM,
+// 1024 TIP4P molecules: 6.0 -> 3.8 us a trial.  The configuration (COM,
 // quaternion, step sizes) lives in LDS for the whole call, and the random
 // stream is staged into LDS kMcChunk trials at a time; the only global
 // traffic per trial are the PairInfo rows and, on acceptance, the PairInfo
