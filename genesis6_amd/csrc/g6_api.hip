@@ -783,8 +783,10 @@ static void launch_steps(System &s, int k) {
     for (int q = 0; q < k; q++) {
       const int p = q & 1;
       if (q > 0) md_launch_pre(s, true, false, false, 0);
-      // clears the cells and rebuild flag of list p before they are filled
-      md_launch_close(s, (q > 0 ? 1 : 0) | 2, 1 << p, 1 - p);
+      // clears the cells and rebuild flag of list p before they are filled;
+      // list 0 is clear where a call starts but for a rebuild flag that the
+      // host set (a state given back, a new box), which this step has to see
+      md_launch_close(s, (q > 0 ? 1 : 0) | 2, q > 0 ? 1 << p : 0, 1 - p);
       md_launch_pre(s, false, true, true, p);
       md_launch_main(s, nullptr, p, 0);
     }

@@ -116,3 +116,80 @@ def test_fp32_follows_fp64_under_the_barostat(golden):
     b, _ = run_g6md(str(f["deck_npt"]), "fp32", "1.0")
     assert np.abs(b[:, 3] / a[:, 3] - 1).max() < 1e-6
     assert np.abs(b[:, 1] / a[:, 1] - 1).max() < 1e-4
+
+
+def baro_start(n, L, rc, pex, mass, skin=1.0, dt=0.001, tiles=False, **env):
+    """A hot lattice start under the barostat; env is read at g6_init."""
+    old = {k: os.environ.get(k) for k in env}
+    os.environ.update({k: str(v) for k, v in env.items()})
+    try:
+        s = g6.System(g6.TIP4P, n, L, rc, 0.5, dt, prec=g6.FP32, skin=skin)
+    finally:
+        for k, v in old.items():
+            if v is None:
+                del os.environ[k]
+            else:
+                os.environ[k] = v
+    com, q = g6.lattice_start(n, L, 9)
+    s.upload(com, q)
+    s.set_nose(1500.0, 1500.0 * 2500.0)
+    s.vreset(1500.0, 9)
+    if not tiles:
+        s.set_andersen(pex, mass)
+    return s
+
+
+def same_run(s, f, steps=3):
+    """Both handles step on alike: every bit of state and thermo but the
+    listed-pair count [15], which depends on when rows were last built."""
+    for _ in range(steps):
+        s.step(1)
+        f.step(1)
+        a, b = s.thermo(), f.thermo()
+        assert a[14] == b[14], (a[14], b[14])
+        np.testing.assert_array_equal(np.delete(a, 15), np.delete(b, 15))
+    for x, y in zip(s.download(), f.download()):
+        np.testing.assert_array_equal(x, y)
+    assert s.box() == f.box()
+
+
+# the call that fails runs far enough that its last rows are of other
+# positions: a cell list of 8 residents overflows once the lattice has melted;
+# a box with 0.05 A to spare above its grid's smallest edge is pressed past it
+@pytest.mark.parametrize("kw", [
+    dict(n=1024, L=31.289, rc=8.5, pex=1.0, mass=1e-2, G6_CELL_CAP=9),
+    dict(n=160, L=19.05, rc=8.5, pex=2e4, mass=1e-2)], ids=["cells", "box"])
+def test_a_failed_barostat_call_leaves_no_rows_behind(kw):
+    print("failed barostat call", kw, flush=True)
+    s, f = baro_start(**kw), baro_start(**kw)
+    s.step(2)  # rows, which a small displacement would keep
+    f.step(2)
+    before = s.download()
+    with pytest.raises(g6.G6Error):
+        s.step(400)
+    for x, y in zip(before, s.download()):
+        np.testing.assert_array_equal(x, y)
+    same_run(s, f)
+    s.close()
+    f.close()
+
+
+def test_the_barostat_after_the_tiles_builds_its_rows():
+    """A system that stepped on the cell tiles has no rows of both directions
+    yet: the barostat's first step builds them."""
+    kw = dict(n=1024, L=31.289, rc=9.0, pex=1.0, mass=1e-4)
+    print("barostat after the tiles", flush=True)
+    s = baro_start(tiles=True, G6_TILE_MIN=0, **kw)
+    assert s.md_kernel()[0] == 1
+    s.step(20)
+    com, quat, dx, w = s.download()
+    f = baro_start(tiles=True, G6_TILES=0, **kw)
+    f.upload(com, None, dx=dx, w=w, quat=quat)
+    z = s.nose()
+    f.set_nose(z[0], z[1] / 0.001, z[2], z[3:8], z[8])
+    np.testing.assert_array_equal(f.nose(), z)
+    for h in (s, f):
+        h.set_andersen(1.0, 1e-4)
+    same_run(s, f)
+    s.close()
+    f.close()
