@@ -10,6 +10,7 @@
 #include <vector>
 
 #include "g6_internal.h"
+#include "g6_stage.h"
 
 namespace g6 {
 
@@ -403,89 +404,6 @@ static System *get(g6_handle h) {
 }
 
 System *system_of(g6_handle h) { return get(h); }
-
-// Downloads of several arrays that lie one after another in device memory:
-// through two pinned buffers, the copy of one piece to the host arrays beside
-// the transfer of the next.  A copy to pageable memory costs its own staging
-// and synchronization per array: the four state arrays took 54 us for 216
-// molecules, 113 for 4096 and 1570 for 65,536, and take 25, 86 and 970 in
-// pieces of 1 MiB (512 KiB: 26, 102, 1300; 4 MiB: 26, 96, 1030; each piece costs
-// about 17 us).  The buffers live while any handle does; a
-// download holds them to its end, so several threads take turns.
-struct HostPart {
-  double *p;   // nullptr: skipped
-  size_t len;  // doubles
-};
-struct Staging {
-  std::mutex mu;
-  int users = 0;
-  char *buf[2] = {nullptr, nullptr};
-  hipEvent_t ev[2];
-};
-constexpr size_t kStageBytes = (size_t)1 << 20;
-static Staging g_stage;
-
-static int staging_open() {
-  std::lock_guard<std::mutex> lk(g_stage.mu);
-  if (g_stage.users == 0) {
-    for (int k = 0; k < 2; k++) {
-      if (hipHostMalloc((void **)&g_stage.buf[k], kStageBytes, hipHostMallocDefault) != hipSuccess ||
-          hipEventCreateWithFlags(&g_stage.ev[k], hipEventDisableTiming) != hipSuccess) {
-        if (g_stage.buf[k]) (void)hipHostFree(g_stage.buf[k]);
-        if (k == 1) {
-          (void)hipHostFree(g_stage.buf[0]);
-          (void)hipEventDestroy(g_stage.ev[0]);
-        }
-        g_stage.buf[0] = g_stage.buf[1] = nullptr;
-        return G6_EHIP;
-      }
-    }
-  }
-  g_stage.users++;
-  return 0;
-}
-
-static void staging_close() {
-  std::lock_guard<std::mutex> lk(g_stage.mu);
-  if (--g_stage.users > 0) return;
-  for (int k = 0; k < 2; k++) {
-    (void)hipHostFree(g_stage.buf[k]);
-    (void)hipEventDestroy(g_stage.ev[k]);
-    g_stage.buf[k] = nullptr;
-  }
-}
-
-static int staged_download(hipStream_t stream, const double *src, const HostPart *part, int np) {
-  size_t total = 0;
-  for (int k = 0; k < np; k++) total += part[k].len * sizeof(double);
-  std::lock_guard<std::mutex> lk(g_stage.mu);
-  const size_t pieces = (total + kStageBytes - 1) / kStageBytes;
-  auto piece_len = [&](size_t q) { return std::min(kStageBytes, total - q * kStageBytes); };
-  auto issue = [&](size_t q) -> int {
-    G6_CHECK(hipMemcpyAsync(g_stage.buf[q & 1], (const char *)src + q * kStageBytes, piece_len(q),
-                            hipMemcpyDeviceToHost, stream));
-    G6_CHECK(hipEventRecord(g_stage.ev[q & 1], stream));
-    return 0;
-  };
-  int rc = pieces > 0 ? issue(0) : 0;
-  for (size_t q = 0; rc == 0 && q < pieces; q++) {
-    if (q + 1 < pieces) rc = issue(q + 1);
-    if (rc == 0 && hipEventSynchronize(g_stage.ev[q & 1]) != hipSuccess) rc = G6_EHIP;
-    if (rc != 0) break;
-    size_t at = 0;  // the parts' byte ranges that the piece holds
-    const size_t b0 = q * kStageBytes, b1 = b0 + piece_len(q);
-    for (int k = 0; k < np; k++) {
-      const size_t e = at + part[k].len * sizeof(double);
-      const size_t lo = std::max(at, b0), hi = std::min(e, b1);
-      if (part[k].p && lo < hi)
-        memcpy((char *)part[k].p + (lo - at), g_stage.buf[q & 1] + (lo - b0), hi - lo);
-      at = e;
-    }
-  }
-  // no transfer into the buffers is left behind by an error
-  if (rc != 0) (void)hipStreamSynchronize(stream);
-  return rc;
-}
 
 static int env_int(const char *name, int dflt) {
   const char *e = getenv(name);
@@ -937,12 +855,13 @@ static int init_system(g6_handle *h, int model, int n, const double *box3, doubl
     void *scr = nullptr;
     rcode = scratch_address(&scr);
   }
-  if (rcode == 0) rcode = staging_open();
+  if (rcode == 0 && hipGetDevice(&s->device) != hipSuccess) rcode = G6_EHIP;
   if (rcode != 0) {
     free_all(*s);
     delete s;
     return rcode;
   }
+  staging_open(s->device);
   std::lock_guard<std::mutex> lk(g_mu);
   g_sys.push_back(s);
   *h = (g6_handle)g_sys.size();
@@ -967,8 +886,8 @@ int g6_finalize(g6_handle h) {
   (void)hipStreamSynchronize(s->stream);
   npt_forget(s);
   free_all(*s);
+  staging_close(s->device);
   delete s;
-  staging_close();
   std::lock_guard<std::mutex> lk(g_mu);
   g_sys[h - 1] = nullptr;
   return 0;
@@ -992,7 +911,8 @@ int g6_download_state(g6_handle h, double *com, double *quat, double *dx, double
   const size_t n = s->n;
   // the state block's rows com, dx, w, quat
   const HostPart part[4] = {{com, 3 * n}, {dx, 15 * n}, {w, 15 * n}, {quat, 20 * n}};
-  return staged_download(s->stream, s->md.com, part, 4);
+  G6_CHECK(staged_download(s->device, s->stream, s->md.com, part, 4));
+  return 0;
 }
 
 int g6_set_nose(g6_handle h, int active, const double *nose) {

@@ -301,6 +301,7 @@ struct System {
   PairK<float> pkf{};
   PairK<double> pkd{};
   hipStream_t stream = nullptr;
+  int device = 0;  // the device that was current at g6_init
   hipGraphExec_t graph = nullptr;  // graph_steps steps
   int graph_steps = 0;
   // graphs of shorter runs, by step count (g6_step of any count replays)

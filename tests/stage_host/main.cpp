@@ -1,0 +1,79 @@
+// Checks of genesis6_amd/csrc/g6_stage.h on the host (hip/hip_runtime.h of
+// this folder stands in for the runtime).  Each check is an argument; a
+// failed one ends the program with status 1.
+#include "g6_stage.h"
+
+#include <stdio.h>
+
+#include <chrono>
+#include <string>
+#include <thread>
+
+using namespace g6;
+#define REQUIRE(c)                                          \
+  do {                                                      \
+    if (!(c)) {                                             \
+      printf("line %d: %s does not hold\n", __LINE__, #c);  \
+      exit(1);                                              \
+    }                                                       \
+  } while (0)
+
+// The state arrays of n molecules: a download of the parts in mask; whether
+// those come out whole and the others stay untouched.
+static bool download(int dev, hipStream_t s, size_t n, int mask) {
+  const size_t len[4] = {3 * n, 15 * n, 15 * n, 20 * n};
+  std::vector<double> src(53 * n), out[4];
+  for (size_t k = 0; k < src.size(); k++) src[k] = 0.5 + (double)k;
+  HostPart part[4];
+  for (int k = 0; k < 4; k++) {
+    out[k].assign(len[k], -1.0);
+    part[k] = {mask >> k & 1 ? out[k].data() : nullptr, len[k]};
+  }
+  if (staged_download(dev, s, src.data(), part, 4) != hipSuccess) return false;
+  size_t at = 0;
+  for (int k = 0; k < 4; k++)
+    for (size_t q = 0; q < len[k]; q++, at++)
+      if (out[k][q] != (mask >> k & 1 ? src[at] : -1.0)) return false;
+  return true;
+}
+
+// handles on two devices, whichever is current at a download
+static void devices() {
+  stub::Stream s0, s1;
+  s1.dev = 1;
+  staging_open(0);
+  staging_open(1);
+  for (int cur = 0; cur < 2; cur++) {
+    stub::device = cur;
+    REQUIRE(download(0, &s0, 3000, 15));
+    REQUIRE(download(1, &s1, 3000, 15));
+    REQUIRE(stub::device == cur);
+  }
+  REQUIRE(stub::pinned == 4 && stub::events == 4);
+  staging_close(0);
+  REQUIRE(stub::pinned == 2 && stub::events == 2);
+  REQUIRE(download(1, &s1, 100, 15));
+  staging_close(1);
+  REQUIRE(stub::pinned == 0 && stub::events == 0);
+  // without buffers (no memory, a device past the table) the arrays come
+  // straight
+  staging_open(0);
+  stub::out_of_memory = true;
+  REQUIRE(download(0, &s0, 3000, 15));
+  REQUIRE(download(kStageDevices, &s0, 3000, 15));
+  staging_close(0);
+}
+
+int main(int argc, char **argv) {
+  for (int k = 1; k < argc; k++) {
+    const std::string name = argv[k];
+    for (int e = 0; e < 2; e++) {
+      stub::eager = e;
+      stub::out_of_memory = false;
+      if (name == "devices") devices();
+      else return 2;
+    }
+    printf("%s ok\n", argv[k]);
+  }
+  return 0;
+}
