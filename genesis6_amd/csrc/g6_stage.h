@@ -1,10 +1,11 @@
 // Downloads of arrays that lie one after another in device memory: through two
 // pinned buffers, the copy of one piece to the host arrays beside the transfer
 // of the next.  A copy to pageable memory costs its own staging and
-// synchronization per array: the four state arrays took 54 us for 216
-// molecules, 113 for 4096 and 1570 for 65,536, and take 25, 86 and 970 in
-// pieces of 1 MiB (512 KiB: 26, 102, 1300; 4 MiB: 26, 96, 1030; each piece costs
-// about 17 us).
+// synchronization per array: the four state arrays took 82 us for 216
+// molecules, 105 for 4096 and 1530 for 65,536, and take 16, 79 and 990 in
+// pieces of 1 MiB (pieces of 512 KiB and 4 MiB: 102 and 96 us for 4096, 1300 and
+// 1030 for 65,536); the COMs alone 15, 13 and 86 before, 13, 14 and 76 now.
+// Arrays that the caller skips are not moved.
 //
 // An event may be recorded on the streams of its own device alone, so every
 // device has its own buffers and events.  They are made at the device's first
@@ -26,6 +27,7 @@ struct HostPart {
 
 constexpr size_t kStageBytes = (size_t)1 << 20;
 constexpr int kStageDevices = 64;
+constexpr int kStageParts = 8;  // arrays of one download
 
 struct Staging {
   std::mutex mu;
@@ -98,36 +100,66 @@ inline hipError_t plain_download(hipStream_t stream, const double *src, const Ho
 
 inline hipError_t staged_download(int dev, hipStream_t stream, const double *src,
                                   const HostPart *part, int np) {
-  if (dev < 0 || dev >= kStageDevices) return plain_download(stream, src, part, np);
+  if (dev < 0 || dev >= kStageDevices || np > kStageParts)
+    return plain_download(stream, src, part, np);
   Staging &g = staging_of(dev);
   std::lock_guard<std::mutex> lk(g.mu);
   if (!staging_make(g, dev)) {
     (void)hipGetLastError();
     return plain_download(stream, src, part, np);
   }
-  size_t total = 0;
-  for (int k = 0; k < np; k++) total += part[k].len * sizeof(double);
+  // pieces of the wanted arrays' bytes, packed: f(offset in the piece, part,
+  // offset in the part, bytes) of each range that bytes [b0, b1) hold
+  auto ranges = [&](size_t b0, size_t b1, auto f) {
+    size_t at = 0;
+    for (int k = 0; k < np; k++) {
+      if (!part[k].p) continue;
+      const size_t e = at + part[k].len * sizeof(double);
+      const size_t lo = std::max(at, b0), hi = std::min(e, b1);
+      if (lo < hi) f(lo - b0, k, lo - at, hi - lo);
+      at = e;
+    }
+  };
+  size_t total = 0, start[kStageParts], pos = 0;
+  for (int k = 0; k < np; k++) {
+    if (part[k].p) total += part[k].len * sizeof(double);
+    start[k] = pos;
+    pos += part[k].len * sizeof(double);
+  }
   const size_t pieces = (total + kStageBytes - 1) / kStageBytes;
-  auto piece_len = [&](size_t q) { return std::min(kStageBytes, total - q * kStageBytes); };
+  auto piece_end = [&](size_t q) { return std::min((q + 1) * kStageBytes, total); };
   auto issue = [&](size_t q) {
-    const hipError_t e = hipMemcpyAsync(g.buf[q & 1], (const char *)src + q * kStageBytes,
-                                        piece_len(q), hipMemcpyDeviceToHost, stream);
-    return e == hipSuccess ? hipEventRecord(g.ev[q & 1], stream) : e;
+    hipError_t e = hipSuccess;
+    // neighbouring arrays are one transfer
+    size_t from = 0, into = 0, len = 0;
+    auto send = [&] {
+      if (len > 0 && e == hipSuccess)
+        e = hipMemcpyAsync(g.buf[q & 1] + into, (const char *)src + from, len,
+                           hipMemcpyDeviceToHost, stream);
+    };
+    ranges(q * kStageBytes, piece_end(q), [&](size_t in, int k, size_t off, size_t bytes) {
+      if (start[k] + off != from + len) {
+        send();
+        from = start[k] + off;
+        into = in;
+        len = 0;
+      }
+      len += bytes;
+    });
+    send();
+    // (a single piece is waited for with the stream: an event costs 7 us)
+    if (e == hipSuccess && pieces > 1) e = hipEventRecord(g.ev[q & 1], stream);
+    return e;
   };
   hipError_t rc = pieces > 0 ? issue(0) : hipSuccess;
   for (size_t q = 0; rc == hipSuccess && q < pieces; q++) {
     if (q + 1 < pieces) rc = issue(q + 1);
-    if (rc == hipSuccess) rc = hipEventSynchronize(g.ev[q & 1]);
+    if (rc == hipSuccess)
+      rc = pieces > 1 ? hipEventSynchronize(g.ev[q & 1]) : hipStreamSynchronize(stream);
     if (rc != hipSuccess) break;
-    size_t at = 0;  // the parts' byte ranges that the piece holds
-    const size_t b0 = q * kStageBytes, b1 = b0 + piece_len(q);
-    for (int k = 0; k < np; k++) {
-      const size_t e = at + part[k].len * sizeof(double);
-      const size_t lo = std::max(at, b0), hi = std::min(e, b1);
-      if (part[k].p && lo < hi)
-        memcpy((char *)part[k].p + (lo - at), g.buf[q & 1] + (lo - b0), hi - lo);
-      at = e;
-    }
+    ranges(q * kStageBytes, piece_end(q), [&](size_t in, int k, size_t off, size_t bytes) {
+      memcpy((char *)part[k].p + off, g.buf[q & 1] + in, bytes);
+    });
   }
   // no transfer into the buffers is left behind by an error
   if (rc != hipSuccess) (void)hipStreamSynchronize(stream);

@@ -64,6 +64,24 @@ static void devices() {
   staging_close(0);
 }
 
+// every choice of arrays, with totals before, at and behind a piece's edge:
+// what is skipped is not moved
+static void ranges() {
+  stub::Stream s0;
+  staging_open(0);
+  const size_t piece = kStageBytes / sizeof(double);
+  for (size_t n : {(size_t)1, piece / 53, piece / 15, piece / 15 + 1, 2 * piece / 18 + 1})
+    for (int mask = 0; mask < 16; mask++) {
+      stub::bytes = 0;
+      REQUIRE(download(0, &s0, n, mask));
+      size_t want = 0;
+      const size_t len[4] = {3 * n, 15 * n, 15 * n, 20 * n};
+      for (int k = 0; k < 4; k++) want += mask >> k & 1 ? len[k] * sizeof(double) : 0;
+      REQUIRE(stub::bytes == want);
+    }
+  staging_close(0);
+}
+
 int main(int argc, char **argv) {
   for (int k = 1; k < argc; k++) {
     const std::string name = argv[k];
@@ -71,6 +89,7 @@ int main(int argc, char **argv) {
       stub::eager = e;
       stub::out_of_memory = false;
       if (name == "devices") devices();
+      else if (name == "ranges") ranges();
       else return 2;
     }
     printf("%s ok\n", argv[k]);
