@@ -102,6 +102,10 @@ inline hipError_t staged_download(int dev, hipStream_t stream, const double *src
                                   const HostPart *part, int np) {
   if (dev < 0 || dev >= kStageDevices || np > kStageParts)
     return plain_download(stream, src, part, np);
+  // what the stream has queued ends before the buffers are taken, so that a
+  // handle at work keeps no other thread from its download
+  const hipError_t idle = hipStreamSynchronize(stream);
+  if (idle != hipSuccess) return idle;
   Staging &g = staging_of(dev);
   std::lock_guard<std::mutex> lk(g.mu);
   if (!staging_make(g, dev)) {

@@ -82,6 +82,33 @@ static void ranges() {
   staging_close(0);
 }
 
+// a download that waits for its stream's work keeps no other one waiting
+static void busy() {
+  stub::Stream s0, s1;
+  staging_open(0);
+  s0.busy = true;
+  bool ok0 = false, ok1 = false, done1 = false;
+  std::thread a([&] { ok0 = download(0, &s0, 3000, 15); });
+  std::this_thread::sleep_for(std::chrono::milliseconds(100));
+  std::thread b([&] {
+    ok1 = download(0, &s1, 3000, 15);
+    std::lock_guard<std::mutex> lk(stub::mu);
+    done1 = true;
+    stub::cv.notify_all();
+  });
+  bool in_time;
+  {
+    std::unique_lock<std::mutex> lk(stub::mu);
+    in_time = stub::cv.wait_for(lk, std::chrono::seconds(5), [&] { return done1; });
+    s0.busy = false;
+    stub::cv.notify_all();
+  }
+  a.join();
+  b.join();
+  staging_close(0);
+  REQUIRE(in_time && ok0 && ok1);
+}
+
 int main(int argc, char **argv) {
   for (int k = 1; k < argc; k++) {
     const std::string name = argv[k];
@@ -90,6 +117,7 @@ int main(int argc, char **argv) {
       stub::out_of_memory = false;
       if (name == "devices") devices();
       else if (name == "ranges") ranges();
+      else if (name == "busy") busy();
       else return 2;
     }
     printf("%s ok\n", argv[k]);

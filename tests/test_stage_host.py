@@ -19,7 +19,7 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("name", ["devices", "ranges"])
+@pytest.mark.parametrize("name", ["devices", "ranges", "busy"])
 def test_staged_download(program, name):
     r = subprocess.run([program, name], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout
