@@ -599,8 +599,10 @@ __device__ inline int scan_row(const Geom &g, const MdBuf &b, const double *com,
 // The sort places every entry at the number of smaller j in the row: a bit
 // per molecule index in LDS (a window of 32 * kRowWords indices at a time),
 // the words' running counts, and the bits below j in its word.  (Counting the
-// smaller entries of the row per entry was 3 passes of 176 LDS reads at 4096
-// molecules, skin 1.8 A, twice the instructions of a step without a build.)
+// smaller entries of the row per entry is 3 passes of 176 LDS reads at 4096
+// molecules, skin 1.8 A, twice the instructions of a step without a build; it
+// stays where the windows are many.)
+constexpr int kWindowEntries = 18;
 template <int BOX>
 __device__ inline int cell_row(const Geom &g, const MdBuf &b, const double *rec, int list, int i,
                                int lane, double xi, double yi, double zi, int *s_j, int *nj,
@@ -687,6 +689,22 @@ __device__ inline int cell_row(const Geom &g, const MdBuf &b, const double *rec,
   }
   wsync();
   const int m = min(base, cap);
+  // The windows cost by the molecules of the system, counting the smaller
+  // entries by the square of the row's: the line lies at kWindowEntries row
+  // entries a window.  Step with rows rebuilt, windows / counting, rows of 102
+  // entries: 4096 molecules 31.4 / 34.8 us, 16,384 94 / 97, 32,768 169 / 160,
+  // 65,536 389 / 308; of 38 entries: 8192 43.2 / 42.3, 32,768 129 / 112; of 242:
+  // 32,768 268 / 323, 65,536 599 / 616.
+  if ((n + 32 * kRowWords - 1) / (32 * kRowWords) * kWindowEntries > m) {
+    for (int t = lane; t < m; t += 64) {
+      const int key = s_j[t];
+      int rank = 0;
+      for (int u = 0; u < m; u++) rank += s_j[u] < key;
+      nj[rank] = key;
+      nc[rank] = s_c[t];
+    }
+    return m;
+  }
   // windows of the index range: the bits of the entries, the running counts
   // of the words (two words per lane of the wave), the entries' places
   int below = 0;

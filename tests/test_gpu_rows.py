@@ -34,11 +34,12 @@ def system(n, L, rc, skin, prec, model=g6.TIP4P, **env):
 
 
 # around a wave (64) and a pass (256) of the scan; one, two and three windows
-# of 4096 indices in the sort of the cell rows
+# of 4096 indices in the sort of the cell rows, and windows too many for the
+# rows' entries (the other sort)
 @pytest.mark.parametrize("n,skin,prec", [(63, 1.0, g6.FP64), (65, 0.0, g6.FP64),
                                          (256, 1.0, g6.FP32), (257, 0.5, g6.FP64),
                                          (1000, 0.0, g6.FP32), (4097, 1.0, g6.FP32),
-                                         (8500, 1.0, g6.FP64)])
+                                         (8500, 1.0, g6.FP64), (25003, 0.0, g6.FP64)])
 def test_scan_and_cell_rows(n, skin, prec):
     L = (n / 0.0334) ** (1.0 / 3.0)
     rc = min(8.5, 0.5 * L - skin - 0.01)
