@@ -16,9 +16,9 @@
 //     unwrapped, so |k| can exceed 1).  The -0.0 shift that dnint gives for
 //     small negative differences is stored as 0: x - (-0.0) and x - 0.0 are
 //     equal for every x but a zero x, whose sign no force term can see
-//   blockpart[2][nblk_md][16], stepek[2][groups of 4 molecules][10]: per-block
-//     energy/virial and per-group kinetic partials, reduced in a fixed order by
-//     the step close (one block)
+//   blockpart[2][nblk_md][16], stepek, stepkin: per-block energy/virial and
+//     kinetic partials and per-group kinetic energies, reduced in a fixed order
+//     by the step close (one block)
 // Reference-list entry point (g6_pairlist.hip): cell residents in molecule
 //   order and the half-shell candidate rows of Grid_NeighborList
 //   (GridModule.F90:557-752) with counts cnt[2n], offsets off[2n+1], and the
@@ -126,9 +126,9 @@ struct MdBuf {
   int scan;  // rows from a scan of every molecule instead of the cell lists
   double *frc;        // [6][n] force and torque (lab) of the last k_md_main
   double *blockpart;  // [2][nblk][16] k_md_main block partials, by parity
-  // kinetic partials [2][groups][kEkLen] and kinetic energies [2][groups] of
-  // the groups of four molecules: the step kernel's by parity, k_md_pre's in
-  // the first halves
+  // kinetic energies [2][groups of four molecules] and kinetic partials: the
+  // step kernel's by parity, [2][groups][kEkLen] (a block is a group);
+  // k_md_pre's in the first halves, [kEkLen][blocks of 64 molecules]
   double *stepek, *stepkin;
   double *nose, *thermo;  // nose[2][9]: by parity inside a call, [0] between
   int *flags;  // [0] error code, [2 + list] rebuild rows this step
@@ -357,11 +357,13 @@ PairK<R> make_pair_k(const ModelTable &mt, const Geom &g) {
 // MD launchers (stream-ordered, graph-capturable: no memset, no host sync)
 // Arguments of the step-close work (k_md_close, or block 0 of k_md_main).
 struct CloseArgs {
-  int mode, nose_active, nblk_pre, nblk_main;
+  int mode, nose_active, ngrp, nblk_main;
   const double *bpart;  // pair partials of the force kernel being closed
   double dt;
-  // kinetic partials [nblk_pre][kEkLen] and kinetic energies [nblk_pre]
+  // kinetic energies of the ngrp groups of four molecules, and kinetic partials:
+  // [ngrp][kEkLen] (fine, the step kernel's) or [kEkLen][blocks of 64]
   const double *ek, *kin;
+  int fine;
   const double *nose_in;  // thermostat state read and written
   double *nose_out;
   int clear;  // cell lists and rebuild flags to clear, one bit each
@@ -383,8 +385,8 @@ inline int main_region_bytes(int maxnb, int rsize) {
 // doubles per block partial of k_md_main: the energy and the pair virial
 // [0..9] (each a compensated block sum, rounded once), pair counts [10..11]
 constexpr int kBP = 16;
-// kinetic partials per group of four molecules: sum |dx(1)|^2, sum w_x^2, w_y^2, w_z^2,
-// and the upper triangle xx xy xz yy yz zz of sum dx(1) dx(1)^T
+// kinetic partials of a group of four molecules or a block of 64: sum
+// |dx(1)|^2, sum w_x^2, w_y^2, w_z^2, and the upper triangle xx xy xz yy yz zz of sum dx(1) dx(1)^T
 constexpr int kEkLen = 10;
 // reduction slots of the step close per wave: 12 pair quantities, kEkLen
 // kinetic ones and the kinetic energy

@@ -9,11 +9,13 @@
 //              Address_Assign binning into fixed-capacity cell lists of this
 //              step's parity, and the Verlet-skin test that decides whether
 //              rows are rebuilt.
-//   close      one block: reduces the block partials in a fixed order into
-//              the thermo record (energies, temperature, pressure, conserved
-//              H), Nose_Correct / Nose_Predict, and clears the
-//              cell lists of the other parity (block 0 of k_md_main, or
-//              k_md_close).  Pair partials alternate between two parities.
+//   close      one block: Nose_Correct / Nose_Predict from the kinetic
+//              energies, and the cell lists of the other parity cleared
+//              (block 0 of k_md_main); after the last step of a call, and
+//              every step of the barostat, also the block partials reduced in
+//              a fixed order into the thermo record (energies, temperature,
+//              pressure, conserved H; k_md_close).  Pair partials alternate
+//              between two parities.
 //   k_md_main  one wavefront per molecule i:
 //              (1) if a rebuild is due, i's own neighbour row: every j != i
 //                  (small systems), or every j != i of the cells whose box
@@ -108,10 +110,12 @@ __device__ __forceinline__ void md_pre_body(const ModelTable &mt, const Geom &g,
   const int i = blk * 64 + lane;
   const bool ok = i < n;
   const bool q2 = role == 2;  // wave 2: components a, b; wave 3: c, d
-  // kinetic partials of the group of four molecules of lanes 4 l .. 4 l + 3
+  // the group of four molecules of lanes 4 l .. 4 l + 3
   const int grp = blk * 16 + (lane >> 2);
   const bool grp_ok = (lane & 3) == 0 && grp * 4 < n;
-  double *ek = b.stepek + (size_t)grp * kEkLen;
+  // the block's kinetic partials, stored by lane 63
+  const int nb64 = (n + 63) / 64;
+  double *ek = b.stepek + blk;
   double et = 0.0;
   double S[20];  // wave 0: com, dx; wave 1: w; waves 2-3: q (all four)
 #pragma unroll
@@ -189,15 +193,17 @@ __device__ __forceinline__ void md_pre_body(const ModelTable &mt, const Geom &g,
       // Rigid_Ek and Rigid_PressureTensor sums (RigidModule.F90:576-619),
       // upper triangle
       const double v[3] = {ok ? S[3] : 0.0, ok ? S[4] : 0.0, ok ? S[5] : 0.0};
-      et = quad_sum_d(v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
-      if (grp_ok) ek[0] = et;
+      const double vv = v[0] * v[0] + v[1] * v[1] + v[2] * v[2];
+      et = quad_sum_d(vv);
+      const double es = wsum63(vv);
+      if (lane == 63) ek[0] = es;
       int q = 4;
 #pragma unroll
       for (int l = 0; l < 3; l++)
 #pragma unroll
         for (int h = l; h < 3; h++, q++) {
-          const double e = quad_sum_d(v[l] * v[h]);
-          if (grp_ok) ek[q] = e;
+          const double e = wsum63(v[l] * v[h]);
+          if (lane == 63) ek[(size_t)q * nb64] = e;
         }
     } else if (role == 1) {
       if (ok) {
@@ -223,8 +229,8 @@ __device__ __forceinline__ void md_pre_body(const ModelTable &mt, const Geom &g,
       }
 #pragma unroll
       for (int c = 0; c < 3; c++) {
-        const double w0 = ok ? S[c] : 0.0, e = quad_sum_d(w0 * w0);
-        if (grp_ok) ek[1 + c] = e;
+        const double w0 = ok ? S[c] : 0.0, e = quad_sum_d(w0 * w0), es = wsum63(w0 * w0);
+        if (lane == 63) ek[(size_t)(1 + c) * nb64] = es;
         if ((lane & 3) == 0) s_ew[c][lane >> 2] = e;
       }
 #pragma unroll
@@ -490,10 +496,10 @@ __global__ __launch_bounds__(256) void k_md_pre_lad(ModelTable mt, const MdRep *
 }
 
 template <bool NPT>
-__global__ __launch_bounds__(256) void k_md_close(ModelTable mt, MdBuf b, int n, int ncell,
-                                                  double box_vol, CloseArgs ca) {
+__global__ __launch_bounds__(1024) void k_md_close(ModelTable mt, MdBuf b, int n, int ncell,
+                                                   double box_vol, CloseArgs ca) {
   __shared__ double s_red[4][kRed];
-  close_body<NPT, 8>(mt, b, n, ncell, box_vol, ca, s_red);
+  close_body<NPT, true>(mt, b, n, ncell, box_vol, ca, s_red);
 }
 
 // ---- kernel B --------------------------------------------------------------
@@ -1441,7 +1447,7 @@ __global__ __launch_bounds__(256, (main_waves_per_eu<M, R>())) void k_md_main(Mo
   const int close = ca.mode != 0;
   if (close && blockIdx.x == 0) {
     __shared__ double s_close[4][kRed];
-    close_body<false>(mt, b, g.n, g.ncell, box_volume(g.L), ca, s_close);
+    close_body<false, false>(mt, b, g.n, g.ncell, box_volume(g.L), ca, s_close);
     return;
   }
   md_main_body<M, R, BOX>(g, b, pk, out, parity, reg_bytes, blockIdx.x - close, gridDim.x - close);
@@ -1463,7 +1469,7 @@ __global__ __launch_bounds__(256, (main_waves_per_eu<M, R>())) void k_md_step(
   const int close = ca.mode != 0;
   if (close && blockIdx.x == 0) {
     __shared__ double s_close[4][kRed];
-    close_body<false>(mt, b, g.n, g.ncell, box_volume(g.L), ca, s_close);
+    close_body<false, false>(mt, b, g.n, g.ncell, box_volume(g.L), ca, s_close);
     return;
   }
   const int nblk = gridDim.x - close;
@@ -1480,10 +1486,11 @@ __device__ __host__ inline CloseArgs step_close_args(const MdBuf &b, int nose_ac
   CloseArgs ca;
   ca.mode = mode;
   ca.nose_active = nose_active;
-  ca.nblk_pre = ca.nblk_main = nblk;
+  ca.ngrp = ca.nblk_main = nblk;
   ca.dt = dt;
   ca.bpart = b.blockpart + (size_t)(1 - parity) * nblk * kBP;
   ca.ek = b.stepek + (size_t)(1 - parity) * nblk * kEkLen;
+  ca.fine = 1;
   ca.kin = b.stepkin + (size_t)(1 - parity) * nblk;
   ca.nose_in = b.nose + 9 * (1 - parity);
   ca.nose_out = b.nose + 9 * parity;
@@ -1510,11 +1517,12 @@ __device__ __host__ inline CloseArgs pre_close_args(const MdBuf &b, int n, int n
   CloseArgs ca;
   ca.mode = mode;
   ca.nose_active = nose_active;
-  ca.nblk_pre = (n + 3) / 4;
+  ca.ngrp = (n + 3) / 4;
   ca.nblk_main = nblk;
   ca.dt = dt;
   ca.bpart = b.blockpart + (size_t)src_parity * nblk * kBP;
   ca.ek = b.stepek;
+  ca.fine = 0;
   ca.kin = b.stepkin;
   ca.nose_in = ca.nose_out = b.nose;
   ca.clear = clear;
@@ -1535,7 +1543,7 @@ __global__ __launch_bounds__(256, (main_waves_per_eu<M, R>())) void k_md_main_la
       __shared__ double s_close[4][kRed];
       const CloseArgs ca = pre_close_args(b, g.n, reps[m.x].nose_active, nm, reps[m.x].dt,
                                           close_mode, 1 << (1 - parity), 1 - parity);
-      close_body<false>(mt, b, g.n, g.ncell, box_volume(g.L), ca, s_close);
+      close_body<false, false>(mt, b, g.n, g.ncell, box_volume(g.L), ca, s_close);
     }
     return;
   }
@@ -1558,7 +1566,7 @@ __global__ __launch_bounds__(256, (main_waves_per_eu<M, R>())) void k_md_step_la
     if (!st.first) {
       __shared__ double s_close[4][kRed];
       const CloseArgs ca = step_close_args(b, s1.nose_active, nm, s1.dt, 1 | 2, st.parity, st.list);
-      close_body<false>(mt, b, g.n, g.ncell, box_volume(g.L), ca, s_close);
+      close_body<false, false>(mt, b, g.n, g.ncell, box_volume(g.L), ca, s_close);
     }
     return;
   }
@@ -1567,8 +1575,9 @@ __global__ __launch_bounds__(256, (main_waves_per_eu<M, R>())) void k_md_step_la
 
 // block r closes system r before (mode 2) or after (mode 1) the k steps of a
 // call; one: they run as step kernels
-__global__ __launch_bounds__(256) void k_md_close_lad(ModelTable mt, const MdRep *__restrict__ reps,
-                                                      int mode, int k, int one) {
+__global__ __launch_bounds__(1024) void k_md_close_lad(ModelTable mt,
+                                                       const MdRep *__restrict__ reps, int mode,
+                                                       int k, int one) {
   __shared__ double s_red[4][kRed];
   const MdRep &r = reps[blockIdx.x];
   const MdBuf b = r.b;
@@ -1576,7 +1585,7 @@ __global__ __launch_bounds__(256) void k_md_close_lad(ModelTable mt, const MdRep
       one ? step_end_args(b, r.nose_active, r.nblk_main, r.dt, mode, k)
           : pre_close_args(b, r.g.n, r.nose_active, r.nblk_main, r.dt, mode, mode == 2 ? 2 : 7,
                            (k - 1) & 1);
-  close_body<false>(mt, b, r.g.n, r.g.ncell, box_volume(r.g.L), ca, s_red);
+  close_body<false, true>(mt, b, r.g.n, r.g.ncell, box_volume(r.g.L), ca, s_red);
 }
 
 __global__ void k_flag_set(int *flags, int k, int v) {
@@ -1602,7 +1611,7 @@ static CloseArgs close_args(System &s, int mode, int clear, int src_parity) {
 
 static void launch_close(System &s, const CloseArgs &ca) {
   auto launch = [&](auto kern) {
-    kern<<<1, 256, 0, s.stream>>>(s.mt, s.md, s.n, s.geo_md.ncell, box_volume(s.Lb), ca);
+    kern<<<1, 1024, 0, s.stream>>>(s.mt, s.md, s.n, s.geo_md.ncell, box_volume(s.Lb), ca);
   };
   if (s.andersen) launch(k_md_close<true>);
   else launch(k_md_close<false>);
@@ -1697,7 +1706,7 @@ void md_launch_pre_lad(Ladder &l, bool correct, bool predict, int list, int half
 }
 
 void md_launch_close_lad(Ladder &l, int mode, int k) {
-  k_md_close_lad<<<(int)l.sys.size(), 256, 0, l.stream>>>(l.mt, l.reps, mode, k,
+  k_md_close_lad<<<(int)l.sys.size(), 1024, 0, l.stream>>>(l.mt, l.reps, mode, k,
                                                           l.one_kernel ? 1 : 0);
 }
 

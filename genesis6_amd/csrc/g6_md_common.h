@@ -55,6 +55,16 @@ __device__ inline double wsum63(double v) {
   return v;
 }
 
+// Sum over the 16 lanes of a DPP row in a fixed order (wsum63's first four
+// steps); every lane of the row receives the row total.
+__device__ inline double rowsum16(double v) {
+  v += dpp_d<0xB1>(v);
+  v += dpp_d<0x4E>(v);
+  v += dpp_d<0x141>(v);
+  v += dpp_d<0x140>(v);
+  return v;
+}
+
 // Lane-wise sum with the lane 32 apart (permlane32_swap) or in the other row
 // of the row pair (permlane16_swap); both lanes get the same bits.
 __device__ inline double swap32_add(double v) {
@@ -213,99 +223,151 @@ __device__ inline double temperature_of(double ek, int n) {
   return 10.0 * 2.0 * ek / (G6_RGAS_MD * (6.0 * n));
 }
 
-// ---- step close: one block of 256 threads ---------------------------------
-// mode bits: 1 the kinetic partials and the pair partials of the step
-// (ca.bpart) form the thermo record, then Nose_Correct; 2 Nose_Predict;
+// ---- step close ------------------------------------------------------------
+// mode bits: 1 the step's kinetic energies give Nose_Correct; 2 Nose_Predict;
 // 16 force evaluation: the pair partials alone go to the thermo record.
-// ca.clear: the cell lists and rebuild flags to clear.  Runs as its own
-// kernel (k_md_close) or in block 0 of the force or step kernel, which
-// neither reads nor writes what it touches.
-// U: rounds of partials with their loads in flight together (registers).
-template <bool NPT, int U = 2>
+// ca.clear: the cell lists and rebuild flags to clear, among them the closed
+// step's.
+// REC: the close forms the thermo record of the step (or of the force
+// evaluation) from the pair partials (ca.bpart) and the kinetic ones; its own
+// kernel (k_md_close), 1024 threads.  Else it runs in block 0 of the force or
+// step kernel, which neither reads nor writes what it touches, threads 0..255,
+// and reads the kinetic energies alone: a later close of the same call forms
+// the record, and only the listed-pair count of the last row build outlives a
+// step.  (With the record's 22 sums block 0 was the longest of the launch:
+// 32,768 molecules 69.5 us against 57 without a close.)
+// The pair partials and the kinetic energies are summed every 256th entry in
+// turn, then the 64 sums of each quarter by the tree of wsum63, then the four
+// quarters.  With REC a wave reads whole rows of pair partials, 16 lanes a row,
+// and each lane carries four of a column's 256 sums: one CU takes in about 48
+// GB/s of what the other XCDs wrote, so the close costs by its bytes (65,536
+// molecules 32 us with kinetic partials of four molecules each, 14 with 64).
+template <bool NPT, bool REC>
 __device__ inline void close_body(const ModelTable &mt, const MdBuf &b, int n, int ncell,
                                   double box_vol, const CloseArgs &ca, double (&s_red)[4][kRed]) {
-  constexpr int NR = kRed;
-  const int wid = threadIdx.x >> 6, mode = ca.mode;
+  constexpr int NR = kRed, NT = REC ? 1024 : 256;
+  const int mode = ca.mode, t = threadIdx.x & 255, wid = t >> 6;
   const double dt = ca.dt;
-  // the work runs on threads 0..255; wider blocks (the tile kernel's) only
-  // take part in the barriers
-  if (threadIdx.x < 256) {
-  // the first kinetic partials are fetched together with the pair partials
-  // (one memory round trip fewer; the sums keep their order)
-  double ek0[kEkLen];
-  {
-    const bool first = (mode & 1) && (int)threadIdx.x < ca.nblk_pre;
-#pragma unroll
-    for (int q = 0; q < kEkLen; q++)
-      ek0[q] = first ? ca.ek[(size_t)threadIdx.x * kEkLen + q] : 0.0;
-  }
-  {
-    // the pair partials (each rounded once from its compensated block sum),
-    // summed over blocks in a fixed order
-    double ps[12];
-#pragma unroll
-    for (int q = 0; q < 12; q++) ps[q] = 0.0;
-    if (mode & 17) {
+  // (wider blocks, the tile kernel's, only take part in the barriers)
+  if (threadIdx.x < NT) {
+    if constexpr (REC) {
+      __shared__ double s_acc[12][257], s_col[kEkLen][64];
+      const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+      double ps[4] = {0.0, 0.0, 0.0, 0.0}, ks = 0.0;
+      const int c = lane & 15, j = 4 * w + (lane >> 4);
+      if ((mode & 17) && c < 12) {
+        const double *p = ca.bpart + c;
+        int k0 = 0;
 #pragma unroll 4
-      for (int k = threadIdx.x; k < ca.nblk_main; k += 256)
+        for (; k0 + 256 <= ca.nblk_main; k0 += 256)
 #pragma unroll
-        for (int q = 0; q < 12; q++) ps[q] += ca.bpart[(size_t)k * kBP + q];
+          for (int u = 0; u < 4; u++) ps[u] += p[(size_t)(k0 + 64 * u + j) * kBP];
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+          if (k0 + 64 * u + j < ca.nblk_main) ps[u] += p[(size_t)(k0 + 64 * u + j) * kBP];
+      }
+      if ((mode & 1) && w < kEkLen) {
+        // a kinetic column: the partials of 64 molecules (a step kernel's 16
+        // groups are added by the tree that wsum63 gives k_md_pre's), every
+        // 64th in turn, then the 64 sums
+        if (!ca.fine) {
+          const int nb = (n + 63) / 64;
+          const double *p = ca.ek + (size_t)w * nb;
+#pragma unroll 16
+          for (int k = lane; k < nb; k += 64) ks += p[k];
+        } else {
+          double e[16];
+#pragma unroll
+          for (int u = 0; u < 16; u++) e[u] = 0.0;
+          for (int k0 = 0; k0 < ca.ngrp; k0 += 1024)
+#pragma unroll
+            for (int u = 0; u < 16; u++) {
+              const int k = k0 + 64 * u + lane;
+              e[u] += rowsum16(k < ca.ngrp ? ca.ek[(size_t)k * kEkLen + w] : 0.0);
+            }
+          if (c == 0)
+#pragma unroll
+            for (int u = 0; u < 16; u++) s_col[w][4 * u + (lane >> 4)] = e[u];
+          wsync();
+          ks = s_col[w][lane];
+        }
+      } else if ((mode & 1) && w < kEkLen + 4) {
+        // the kinetic energies of quarter w - kEkLen
+#pragma unroll 16
+        for (int k = 64 * (w - kEkLen) + lane; k < ca.ngrp; k += 256) ks += ca.kin[k];
+      }
+      ks = wsum63(ks);
+      if (lane == 63 && w < kEkLen + 4) {
+        if (w < kEkLen) {
+#pragma unroll
+          for (int u = 0; u < 4; u++) s_red[u][12 + w] = u == 0 ? ks : 0.0;
+        } else {
+          s_red[w - kEkLen][12 + kEkLen] = ks;
+        }
+      }
+      if (c < 12)
+#pragma unroll
+        for (int u = 0; u < 4; u++) s_acc[c][64 * u + j] = ps[u];
+      __syncthreads();
+      if (w < 12)
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+          const double v = wsum63(s_acc[w][64 * u + lane]);
+          if (lane == 63) s_red[u][w] = v;
+        }
+    } else {
+      double listed = 0.0, kin = 0.0;
+      int rebuilt = 0;
+#pragma unroll
+      for (int p = 0; p < 3; p++)
+        if (ca.clear >> p & 1) rebuilt |= b.flags[2 + p];
+      if ((mode & 1) && ca.nose_active) {
+#pragma unroll 8
+        for (int k = t; k < ca.ngrp; k += 256) kin += ca.kin[k];
+      }
+      if ((mode & 1) && rebuilt) {
+#pragma unroll 8
+        for (int k = t; k < ca.nblk_main; k += 256) listed += ca.bpart[(size_t)k * kBP + 11];
+      }
+      listed = wsum63(listed);
+      kin = wsum63(kin);
+      if ((t & 63) == 63) {
+        s_red[wid][11] = listed;
+        s_red[wid][12 + kEkLen] = kin;
+      }
     }
-#pragma unroll
-    for (int q = 0; q < 12; q++) ps[q] = wsum63(ps[q]);
-    if ((threadIdx.x & 63) == 63)
-#pragma unroll
-      for (int q = 0; q < 12; q++) s_red[wid][q] = ps[q];
-  }
-  {
-    // the kinetic partials
-    double ek[kEkLen], kin = 0.0;
-#pragma unroll
-    for (int q = 0; q < kEkLen; q++) ek[q] = 0.0 + ek0[q];
-    if (mode & 1) {
-#pragma unroll U
-      for (int k = threadIdx.x + 256; k < ca.nblk_pre; k += 256)
-#pragma unroll
-        for (int q = 0; q < kEkLen; q++) ek[q] += ca.ek[(size_t)k * kEkLen + q];
-#pragma unroll 4
-      for (int k = threadIdx.x; k < ca.nblk_pre; k += 256) kin += ca.kin[k];
-    }
-#pragma unroll
-    for (int q = 0; q < kEkLen; q++) ek[q] = wsum63(ek[q]);
-    kin = wsum63(kin);
-    if ((threadIdx.x & 63) == 63) {
-#pragma unroll
-      for (int q = 0; q < kEkLen; q++) s_red[wid][12 + q] = ek[q];
-      s_red[wid][12 + kEkLen] = kin;
-    }
-  }
-  for (int p = 0; p < 3; p++) {
-    if (!(ca.clear >> p & 1)) continue;
-    int *cr = b.cellres + (size_t)p * ncell * b.cell_cap;
-    if (!b.scan)
-      for (int c = threadIdx.x; c < ncell; c += 256) cr[(size_t)c * b.cell_cap] = 0;
-    if (threadIdx.x == 0 && b.half_skin2 > 0.0) b.flags[2 + p] = 0;
-  }
   }
   __syncthreads();
   // totals over the four waves, one quantity per thread, into row 0
-  if (threadIdx.x < NR) {
+  if (threadIdx.x < NR && (REC || threadIdx.x == 11 || threadIdx.x == NR - 1)) {
     const int q = threadIdx.x;
     s_red[0][q] = s_red[0][q] + s_red[1][q] + s_red[2][q] + s_red[3][q];
   }
+  if (threadIdx.x < NT)
+    for (int p = 0; p < 3; p++) {
+      if (!(ca.clear >> p & 1)) continue;
+      int *cr = b.cellres + (size_t)p * ncell * b.cell_cap;
+      if (!b.scan)
+        for (int c = threadIdx.x; c < ncell; c += NT) cr[(size_t)c * b.cell_cap] = 0;
+      if (threadIdx.x == 0 && b.half_skin2 > 0.0) b.flags[2 + p] = 0;
+    }
   __syncthreads();
   if (threadIdx.x == 0) {
     const double *r = s_red[0];
     double *th = b.thermo;
     double z[9];
     for (int q = 0; q < 9; q++) z[q] = ca.nose_in[q];
-    if (mode & 17) {
+    if (!REC && (mode & 1)) {
+      if (r[11] > 0) th[15] = r[11];
+      if (ca.nose_active) nose_correct(z, temperature_of(r[12 + kEkLen], n));
+    }
+    if (REC && (mode & 17)) {
       th[0] = r[0];
       for (int q = 0; q < 9; q++) th[4 + q] = r[1 + q];
       th[14] = r[10];
       if (r[11] > 0) th[15] = r[11];
     }
-    if (mode & 1) {
+    if (REC && (mode & 1)) {
       const double ep = r[0];
       const double ekt = r[12] * mt.mass * 0.5 * (1.0 / (dt * dt));
       const double ekr = (r[13] * mt.Ixx + r[14] * mt.Iyy + r[15] * mt.Izz) * 0.5;
@@ -418,15 +480,5 @@ struct RecSites<M, double> {
     for (int a = 0; a < 3; a++) r[Traits<M>::COM][a] = 0.0;
   }
 };
-
-// Sum over the 16 lanes of a DPP row in a fixed order; every lane of the
-// row receives the row total.
-__device__ inline double rowsum16(double v) {
-  v += dpp_d<0xB1>(v);
-  v += dpp_d<0x4E>(v);
-  v += dpp_d<0x141>(v);
-  v += dpp_d<0x140>(v);
-  return v;
-}
 
 }  // namespace g6

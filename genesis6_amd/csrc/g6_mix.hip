@@ -104,7 +104,7 @@ __device__ inline void mix_close_body(const MixClose &c, int mode, int parity) {
     // per thread in block order, then over the wave and the four waves.  A
     // set at a time: all 56 sums at once held 112 registers, which the cross
     // kernel this rides in had to have too.
-    auto sums = [&](const double *p, int nb, int stride, auto len, int at) {
+    auto sums = [&](const double *p, int nb, int sk, int sq, auto len, int at) {
       constexpr int N = decltype(len)::value;
       double v[N];
 #pragma unroll
@@ -113,7 +113,7 @@ __device__ inline void mix_close_body(const MixClose &c, int mode, int parity) {
 #pragma unroll 2
         for (int k = threadIdx.x; k < nb; k += 256)
 #pragma unroll
-          for (int q = 0; q < N; q++) v[q] += p[(size_t)k * stride + q];
+          for (int q = 0; q < N; q++) v[q] += p[(size_t)k * sk + (size_t)q * sq];
 #pragma unroll
       for (int q = 0; q < N; q++) v[q] = wsum63(v[q]);
       if ((threadIdx.x & 63) == 63)
@@ -122,11 +122,11 @@ __device__ inline void mix_close_body(const MixClose &c, int mode, int parity) {
     };
     const std::integral_constant<int, 12> pairs;
     const std::integral_constant<int, kEkLen> kin;
-    sums(c.bpart_a, c.nblk_main_a, kBP, pairs, 0);
-    sums(c.bpart_b, c.nblk_main_b, kBP, pairs, 12);
-    sums(c.bpart_x, c.nblk_x, kBP, pairs, 24);
-    sums(c.a.blockek, c.nblk_pre_a, kEkLen, kin, 36);
-    sums(c.b.blockek, c.nblk_pre_b, kEkLen, kin, 36 + kEkLen);
+    sums(c.bpart_a, c.nblk_main_a, kBP, 1, pairs, 0);
+    sums(c.bpart_b, c.nblk_main_b, kBP, 1, pairs, 12);
+    sums(c.bpart_x, c.nblk_x, kBP, 1, pairs, 24);
+    sums(c.a.blockek, c.nblk_pre_a, 1, c.nblk_pre_a, kin, 36);
+    sums(c.b.blockek, c.nblk_pre_b, 1, c.nblk_pre_b, kin, 36 + kEkLen);
   }
   if (mode & 12) {
     const int p0 = (mode & 8) ? 0 : 1 - parity, p1 = (mode & 8) ? 1 : 1 - parity;
@@ -531,8 +531,8 @@ static MixClose mix_close_args(const Mix &m, int src_parity) {
   c.thermo = a.md.thermo;
   c.na = a.n;
   c.nb = b.n;
-  c.nblk_pre_a = (a.n + 3) / 4;
-  c.nblk_pre_b = (b.n + 3) / 4;
+  c.nblk_pre_a = pre_blocks(a.n);
+  c.nblk_pre_b = pre_blocks(b.n);
   c.nblk_main_a = a.nblk_md;
   c.nblk_main_b = b.nblk_md;
   c.nblk_x = m.nblk_a + m.nblk_b;

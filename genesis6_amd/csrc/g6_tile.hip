@@ -518,7 +518,7 @@ __global__ __launch_bounds__(512) void k_md_tile(ModelTable mt, Geom g, MdBuf b,
     // block 0 closes the previous step while the other blocks run the tiles
     if (blockIdx.x == 0) {
       __shared__ double s_close[4][kRed];
-      close_body<false>(mt, b, g.n, g.ncell, box_volume(g.L), ca, s_close);
+      close_body<false, false>(mt, b, g.n, g.ncell, box_volume(g.L), ca, s_close);
       return;
     }
     tile_body<M, STAGE>(g, b, pk, parity, lay, blockIdx.x - 1, gridDim.x - 1);

@@ -88,3 +88,28 @@ def test_one_kernel_and_two_kernel_steps(n, model, prec, skin, nose, ortho):
         s.close()
     for a, b in zip(*out):
         assert np.array_equal(a, b)
+
+
+# only a call's last close forms the thermo record; the listed pairs [15] are
+# of the call's last row build
+@pytest.mark.parametrize("n,prec,skin,env", [
+    (217, g6.FP64, 0.0, {}), (1000, g6.FP32, 1.0, {}), (4101, g6.FP32, 0.3, {"G6_STEP_MAX": 0}),
+    (6201, g6.FP32, 0.3, {}), (1024, g6.FP32, 1.0, {"G6_TILE_MIN": 0})])
+@pytest.mark.parametrize("nose", [True, False])
+def test_a_call_of_many_steps_and_many_calls(n, prec, skin, env, nose):
+    L = (n / 0.0334) ** (1.0 / 3.0)
+    out = []
+    print("calls n %d skin %g" % (n, skin), env, flush=True)
+    for calls in ([60], [1] * 60):
+        s, _ = system(n, L, min(8.5, 0.45 * L - skin - 0.01), skin, prec, **env)
+        assert s.md_kernel()[0] == ("G6_TILE_MIN" in env)
+        if nose:
+            s.set_nose(300.0, 7.5e5)
+        for k in calls:
+            s.step(k)
+        assert s.md_kernel()[0] == ("G6_TILE_MIN" in env)
+        out.append([s.thermo(), s.nose(), *s.download()])
+        s.close()
+    assert out[0][0][15] > 0
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
