@@ -266,7 +266,13 @@ __device__ __forceinline__ void tile_body(const Geom &g, const MdBuf &b, const P
   park();
 
   // ---- 3. rows, interaction test, dense pair rounds ----
-  const double Lb = g.L[0], invL = g.invL[0], rr = g.rr, rc2 = g.rc2;
+  // In vector registers: the loop has more scalars than there are registers,
+  // and these eight leave it 19 reads of spilled ones instead of 42.  131,072
+  // TIP4P 233 -> 222 us a launch (228 with the spills of two inlined copies),
+  // 65,536 TIP5P 139 -> 133, a build step there 305 -> 275.  (The row pointers
+  // in vector registers as well: 234 and 209.)
+  double Lb = g.L[0], invL = g.invL[0], rr = g.rr, rc2 = g.rc2;
+  asm volatile("" : "+v"(Lb), "+v"(invL), "+v"(rr), "+v"(rc2));
   const double fmax = 33554432.0 / (1.0 + sqrt(rc2));
   const float m2max = (float)(fmax * fmax);
   // each lane's energy and virial over its own pairs (a few per step) in
@@ -514,17 +520,14 @@ __device__ __forceinline__ void tile_body(const Geom &g, const MdBuf &b, const P
 template <int M, bool STAGE>
 __global__ __launch_bounds__(512) void k_md_tile(ModelTable mt, Geom g, MdBuf b, PairK<float> pk,
                                                  int parity, CloseArgs ca, TileLayout lay) {
-  if (ca.mode) {
-    // block 0 closes the previous step while the other blocks run the tiles
-    if (blockIdx.x == 0) {
-      __shared__ double s_close[4][kRed];
-      close_body<false, false>(mt, b, g.n, g.ncell, box_volume(g.L), ca, s_close);
-      return;
-    }
-    tile_body<M, STAGE>(g, b, pk, parity, lay, blockIdx.x - 1, gridDim.x - 1);
-  } else {
-    tile_body<M, STAGE>(g, b, pk, parity, lay, blockIdx.x, gridDim.x);
+  // block 0 closes the previous step while the other blocks run the tiles
+  const int close = ca.mode != 0;
+  if (close && blockIdx.x == 0) {
+    __shared__ double s_close[4][kRed];
+    close_body<false, false>(mt, b, g.n, g.ncell, box_volume(g.L), ca, s_close);
+    return;
   }
+  tile_body<M, STAGE>(g, b, pk, parity, lay, blockIdx.x - close, gridDim.x - close);
 }
 
 // force (lab) and body torque of every molecule from its partials, in the
