@@ -801,7 +801,9 @@ __global__ __launch_bounds__(kMcBlock) void k_mc_trials(McArgs a, StdTable st, i
         aborted = true;
         break;
       }
-      for (int k = tid; k < n; k += kMcBlock) a.b.q6.dq6[k] = q6_of(a.b.q6, k);
+      // (the list's place is free from here on: thread 0's sum in molecule
+      // order reads LDS)
+      for (int k = tid; k < n; k += kMcBlock) l_list[k] = a.b.q6.dq6[k] = q6_of(a.b.q6, k);
       __syncthreads();
     }
     double de = 0.0;
@@ -821,7 +823,8 @@ __global__ __launch_bounds__(kMcBlock) void k_mc_trials(McArgs a, StdTable st, i
         double q6op = 0.0;
         if constexpr (UQ6) {  // sumq6 / nmol (Q6Local.F90:429-440)
           double sq = 0.0;
-          for (int k = 0; k < n; k++) sq = sq + a.b.q6.dq6[k];
+#pragma unroll 8
+          for (int k = 0; k < n; k++) sq = sq + l_list[k];
           q6op = sq / n;
         }
         double dope = 0.0;
