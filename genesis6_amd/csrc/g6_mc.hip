@@ -3,13 +3,14 @@
 // mc2 (mc2.F90:540-862, with DEBUG20050322a as the reference compiles it).
 //
 // The trial loop is sequential by definition, so it runs as one persistent
-// block of 512 threads.  Per trial every thread derives the same proposal
-// from the shared random stream (no broadcast needed), each thread tests the
-// molecules it owns against the moved target (the reference's compressed
-// pair list, radius rc + dt, energies by StdPairPotential), one block
-// reduction forms dE in a fixed order, and every thread takes the same
-// Metropolis decision.  Accepted moves update the target and its PairInfo row
-// and column in place.
+// block of 768 threads.  Per trial eight waves test the molecules they own
+// against the moved target (the reference's compressed pair list, radius
+// rc + dt) and spread the listed molecules' site pairs over their lanes
+// (energies by StdPairPotential), two waves form the switch of the listed
+// molecules and the target's next step sizes, and two prepare the next trial's
+// proposal; one block reduction forms dE in a fixed order, and every thread
+// takes the same Metropolis decision.  Accepted moves update the target and
+// its PairInfo row and column in place.
 //
 // Random numbers: the host generates the Random_GetNext stream (MT19937, the
 // reference's mtrnd) and, for every position k, the Box-Muller factor
@@ -382,7 +383,7 @@ __device__ inline double umbrella_potential(double coeffi, double center, double
 // mc2's trial loop, ntrial trials, one block.  The chain of trials is serial,
 // so the kernel is bound by the latency of one trial, not by a unit of the
 // chip; what a trial does is spread over the block and overlapped:
-// - Eight waves test two to four molecules a thread against the moved target
+// - Eight waves test one to three molecules a thread against the moved target
 //   and append those within the cutoff to one list; the list's site pairs are
 //   then spread densely, a site pair per lane.  (A molecule's site terms in
 //   the thread that owns it kept about five of 64 lanes busy, in every wave:
@@ -441,8 +442,8 @@ __global__ __launch_bounds__(kMcBlock) void k_mc_trials(McArgs a, StdTable st, i
   double *l_q = l_com + 3 * n;                // [4][n]
   double *l_delta = l_q + 4 * n;              // [n]
   double *l_rtr = l_delta + n;                // [n]
-  // the listed molecules: index
-  // and nearest image, then their energies in place; their switch values
+  // the listed molecules: index and nearest image, then their energies in
+  // place; their switch values
   double *l_list = l_rtr + n;                 // [n]
   double *l_er = l_list + n;                  // [n]
   double *l_u = l_er + n;                     // [kMcStage]

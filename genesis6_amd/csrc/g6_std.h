@@ -15,8 +15,9 @@
 namespace g6 {
 
 // The site pairs of StdPairPotential's term list for the MC models, in
-// the order make_std_table produces them (checked at g6_mc_begin), so that
-// the trial kernel indexes sites with constants.
+// the order make_std_table produces them (checked at g6_mc_begin): the trial
+// kernel takes the counts from it, and the NPT kernels index sites with
+// constants.
 template <int M>
 struct StdPattern;
 template <>
@@ -156,42 +157,9 @@ __device__ inline double std_term(const StdTerm &s, double dx, double dy, double
   return s.kind == 2 ? c : (s.kind == 1 ? c + w : w) + s.bb * d6;
 }
 
-// std_energy with the term list of model M: j's sites from memory, the
-// other molecule's sites in registers (constant indices)
-template <int M>
-__device__ inline double std_energy_t(const StdTable &st, const double *xj, const double *yj,
-                                     const double *zj, const double (&xt)[kMaxSite],
-                                     const double (&yt)[kMaxSite], const double (&zt)[kMaxSite],
-                                     double ox, double oy, double oz, double er) {
-  using P = StdPattern<M>;
-  double ep = 0.0;
-#pragma unroll
-  for (int u = 0; u < P::NT; u++) {
-    const StdTerm s = st.t[u];
-    double dx = xj[P::a(u)] - xt[P::b(u)], dy = yj[P::a(u)] - yt[P::b(u)],
-           dz = zj[P::a(u)] - zt[P::b(u)];
-    dx = dx - ox;
-    dy = dy - oy;
-    dz = dz - oz;
-    const double dd = 1.0 / (dx * dx + dy * dy + dz * dz);
-    double e0;
-    if (P::kind(u) == 1) {  // Coulomb + LJ
-      e0 = s.qq * sqrt(dd);
-      const double d6 = dd * dd * dd, d12 = d6 * d6;
-      e0 = e0 + s.aa * d12 + s.bb * d6;
-    } else if (P::kind(u) == 3) {  // LJ only
-      const double d6 = dd * dd * dd, d12 = d6 * d6;
-      e0 = s.aa * d12 + s.bb * d6;
-    } else {
-      e0 = s.qq * sqrt(dd);
-    }
-    ep = ep + e0;
-  }
-  return ep * er;
-}
-
-// std_energy_t with both molecules' sites in registers: a (outer, sites
-// P::a) and b (inner, sites P::b), d = a - b - o
+// std_energy with the term list of model M and both molecules' sites in
+// registers (constant indices): a (outer, sites P::a) and b (inner, sites
+// P::b), d = a - b - o
 template <int M>
 __device__ inline double std_energy_rr(const StdTable &st, const double (&xa)[kMaxSite],
                                       const double (&ya)[kMaxSite], const double (&za)[kMaxSite],
@@ -266,31 +234,6 @@ __device__ inline void place_site(double bx, double by, double bz, double qa, do
   x = cx + (t0 * bx + t1 * by + t2 * bz);
   y = cy + (t3 * bx + t4 * by + t5 * bz);
   z = cz + (t6 * bx + t7 * by + t8 * bz);
-}
-
-// place_sites with a constant site count (the trial kernel's registers)
-template <int NS, class A>
-__device__ inline void place_sites_t(const A &a, double qa, double qb, double qc, double qd,
-                                     double cx, double cy, double cz, double (&x)[kMaxSite],
-                                     double (&y)[kMaxSite], double (&z)[kMaxSite]) {
-  const double t0 = (qa * qa + qb * qb - (qc * qc + qd * qd));
-  const double t1 = -2.0 * (qa * qd + qb * qc);
-  const double t2 = 2.0 * (qb * qd - qa * qc);
-  const double t3 = 2.0 * (qa * qd - qb * qc);
-  const double t4 = qa * qa + qc * qc - (qb * qb + qd * qd);
-  const double t5 = -2.0 * (qa * qb + qc * qd);
-  const double t6 = 2.0 * (qa * qc + qb * qd);
-  const double t7 = 2.0 * (qa * qb - qc * qd);
-  const double t8 = qa * qa + qd * qd - (qb * qb + qc * qc);
-#pragma unroll
-  for (int s = 0; s < NS; s++) {
-    const double r0 = t0 * a.bx[s] + t1 * a.by[s] + t2 * a.bz[s];
-    const double r1 = t3 * a.bx[s] + t4 * a.by[s] + t5 * a.bz[s];
-    const double r2 = t6 * a.bx[s] + t7 * a.by[s] + t8 * a.bz[s];
-    x[s] = cx + r0;
-    y[s] = cy + r1;
-    z[s] = cz + r2;
-  }
 }
 
 }  // namespace g6
