@@ -64,6 +64,27 @@ def test_ladder_steps_equal_single_system_steps_bitwise(prec, mid):
         assert np.array_equal(x, y)
 
 
+@pytest.mark.parametrize("prec", [g6.FP32, g6.FP64])
+def test_two_kernel_ladder_equals_one_kernel_steps_bitwise(prec, monkeypatch):
+    """A ladder past the line of one kernel per step (here none is below it)
+    steps by predictor and force kernels, its systems alone by the step
+    kernel: the same bits."""
+    solo = [make(n, r, sd, T, prec, sk, ns) for n, r, sd, T, sk, ns in SPECS]
+    monkeypatch.setenv("G6_STEP_MAX", "0")
+    lad_sys = [make(n, r, sd, T, prec, sk, ns) for n, r, sd, T, sk, ns in SPECS]
+    lad = g6.Ladder(lad_sys)
+    for k in (1, 2, 37):
+        print("steps", k, flush=True)
+        lad.step(k)
+        th = lad.thermo()
+        for r, (a, b) in enumerate(zip(lad_sys, solo)):
+            b.step(k)
+            for x, y in zip(a.download(), b.download()):
+                assert np.array_equal(x, y), (k, r)
+            assert np.array_equal(th[r], b.thermo()), (k, r)
+            assert np.array_equal(a.nose(), b.nose()), (k, r)
+
+
 def test_set_temperature_matches_oracle():
     n, L = 128, box(128, 1.0)
     com, q = lattice_start(n, L, 21)

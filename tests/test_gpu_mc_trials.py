@@ -24,7 +24,7 @@ def start(n, L, seed):
 
 @pytest.mark.parametrize("model,n,far", [
     ("TIP4P", 2, 0), ("TIP4P", 64, 0), ("SPCE", 65, 0), ("TIP5P", 511, 0), ("NVDE", 513, 0),
-    ("OPLSMEOH", 216, 0), ("TIP4P", 1025, 0), ("TIP4P", 1535, 0), ("TIP4P", 216, 40000),
+    ("OPLSMEOH", 216, 0), ("ST2", 100, 0), ("TIP4P", 1025, 0), ("TIP4P", 1535, 0), ("TIP4P", 216, 40000),
 ])
 def test_trials_equal_the_oracle(model, n, far):
     L = max(20.0, 3.2 * n ** (1 / 3) + 0.1)

@@ -12,7 +12,7 @@ from oracle import pyoracle as O
 pytestmark = pytest.mark.gpu
 
 
-def system(n, L, rc, skin, prec, model=g6.TIP4P, **env):
+def system(n, L, rc, skin, prec, model=g6.TIP4P, grid=None, **env):
     old = {k: os.environ.get(k) for k in env}
     os.environ.update({k: str(v) for k, v in env.items()})
     try:
@@ -25,6 +25,9 @@ def system(n, L, rc, skin, prec, model=g6.TIP4P, **env):
                 os.environ[k] = v
     com, q = g6.lattice_start(n, np.max(L), 31 + n)
     com *= np.asarray(L) / np.max(L)
+    if grid is not None:  # an axis' share of the molecules by its length
+        com = np.stack(np.meshgrid(*[np.arange(k) + 0.5 for k in grid], indexing="ij"), -1)
+        com = com.reshape(-1, 3) * (np.asarray(L) / grid)
     # off the lattice, and some molecules boxes away (unwrapped COMs)
     com += np.random.default_rng(n).normal(0.0, 0.05, com.shape)
     com[::7] += L * np.random.default_rng(n + 1).integers(-3, 4, com[::7].shape)
@@ -57,6 +60,45 @@ def test_scan_and_cell_rows(n, skin, prec):
     for a, b in zip(out[0][1], out[1][1]):
         assert np.array_equal(a, b)
     assert np.array_equal(out[0][2], out[1][2])
+
+
+def brute_pairs(com, L, r):
+    """Minimum-image pairs within r."""
+    d = com[:, None, :] - com[None, :, :]
+    d -= np.asarray(L) * np.round(d / np.asarray(L))
+    return int((np.triu((d * d).sum(-1) < r * r, 1)).sum())
+
+
+# cells of unequal counts per axis: 6 x 9 x 4 (an axis below the five cells of
+# the stencil, two above) and 2 x 5 x 11 (two cells across an axis); under the
+# barostat the box, and with it the stencil's pruning, moves with every step
+@pytest.mark.parametrize("L,rc,skin", [((28.0, 41.0, 17.3), 8.0, 0.5),
+                                       ((13.4, 30.1, 60.5), 4.9, 0.5)])
+@pytest.mark.parametrize("mode", [0, 1, 2])
+@pytest.mark.parametrize("prec", [g6.FP64, g6.FP32])
+def test_scan_and_cell_rows_in_other_boxes(L, rc, skin, mode, prec):
+    grid = [int(e / 3.1) for e in L]
+    n = int(np.prod(grid))
+    out = []
+    for env in (dict(G6_SCAN_MAX=1 << 20), dict(G6_SCAN_MAX=0),
+                dict(G6_SCAN_MAX=0, G6_STEP_MAX=0)):
+        s, com = system(n, np.array(L), rc, skin, prec, grid=grid, **env)
+        print("rows in a box of", L, "mode", mode, env, flush=True)
+        s.set_nose(300.0, 7.5e5)
+        if mode:
+            s.set_andersen(1.0, 1e-3, mode=mode)
+        _, _, th = s.eval_forces()
+        s.step(3)
+        s.step(60)
+        out.append([th, s.thermo(), s.box3(), *s.download()])
+        s.close()
+    for k, r in ((14, rc), (15, rc + skin)):
+        assert out[0][0][k] == brute_pairs(com, L, r)
+    if mode:
+        assert not np.array_equal(out[0][2], L)
+    for other in out[1:]:
+        for a, b in zip(out[0], other):
+            assert np.array_equal(a, b)
 
 
 # blocks of four molecules with one to four of them; a thousand kinetic
