@@ -1285,6 +1285,12 @@ int g6_eval_forces_noalloc(g6_handle h, double *force, double *torque, double *t
   return eval_forces_into(s, static_cast<double *>(p), force, torque, thermo, false);
 }
 
+// the next step builds its rows
+static hipError_t rebuild_rows(System &s) {
+  const int one[3] = {1, 1, 1};
+  return hipMemcpy(s.md.flags + 2, one, sizeof(one), hipMemcpyHostToDevice);
+}
+
 int g6_set_andersen(g6_handle h, int mode, double pex, double mass, const double *v) {
   System *s = get(h);
   if (!s) return G6_EARG;
@@ -1295,6 +1301,7 @@ int g6_set_andersen(g6_handle h, int mode, double pex, double mass, const double
       (void)hipFree(s->md.anders);
       s->md.box = s->md.anders = nullptr;
       s->andersen = false;
+      G6_CHECK(rebuild_rows(*s));  // the rows are of the barostat's box
     }
   } else {
     // orthorhombic (every edge follows the volume) or orz (the z edge alone);
@@ -1343,9 +1350,7 @@ int g6_set_andersen(g6_handle h, int mode, double pex, double mass, const double
     G6_CHECK(hipMemcpy(s->md.box, bx, sizeof(bx), hipMemcpyHostToDevice));
     G6_CHECK(hipMemcpy(s->md.anders, an, sizeof(an), hipMemcpyHostToDevice));
     s->andersen_mode = mode;
-    // rows of the new box
-    int one[3] = {1, 1, 1};
-    G6_CHECK(hipMemcpy(s->md.flags + 2, one, sizeof(one), hipMemcpyHostToDevice));
+    G6_CHECK(rebuild_rows(*s));  // rows of the new box
   }
   drop_graphs(*s);  // the captured launches embed the step sequence
   return 0;

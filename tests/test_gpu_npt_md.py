@@ -193,3 +193,23 @@ def test_the_barostat_after_the_tiles_builds_its_rows():
     same_run(s, f)
     s.close()
     f.close()
+
+
+def test_the_fixed_box_after_the_barostat_builds_its_rows():
+    """Mode 0 gives the handle its first box back: the rows of the barostat's
+    last box are not kept for it."""
+    kw = dict(n=1024, L=31.289, rc=8.5, pex=1.0, mass=1e-5, G6_CELL_CAP=30)
+    print("fixed box after the barostat", flush=True)
+    s = baro_start(**kw)
+    s.step(120)
+    assert s.box() > 31.289 + 0.5
+    s.set_andersen(1.0, 1e-4, mode=0)
+    com, quat, dx, w = s.download()
+    f = baro_start(tiles=True, **kw)
+    f.upload(com, None, dx=dx, w=w, quat=quat)
+    z = s.nose()
+    f.set_nose(z[0], z[1] / 0.001, z[2], z[3:8], z[8])
+    np.testing.assert_array_equal(f.nose(), z)
+    same_run(s, f)
+    s.close()
+    f.close()
