@@ -905,13 +905,33 @@ int g6_upload_state(g6_handle h, const double *com, const double *quat, const do
   return reset_step_state(*s);
 }
 
+// Transfers of g6_download_state into pinned memory.  A kernel writes them:
+// the copy engine is 3 us a transfer faster (407 KB 25 against 28 us, 28 MB 990
+// against 1080), but its first transfer in a process costs 6.3 ms, which took
+// 64 downloads of 960 molecules from 7.1 to 12.5 ms (6.7 with the kernel).
+static __global__ __launch_bounds__(256) void k_stage_copy(double *__restrict__ dst,
+                                                           const double *__restrict__ src,
+                                                           int n) {
+  for (int k = blockIdx.x * 256 + threadIdx.x; k < n; k += gridDim.x * 256) dst[k] = src[k];
+}
+
 int g6_download_state(g6_handle h, double *com, double *quat, double *dx, double *w) {
   System *s = get(h);
   if (!s) return G6_EARG;
   const size_t n = s->n;
   // the state block's rows com, dx, w, quat
   const HostPart part[4] = {{com, 3 * n}, {dx, 15 * n}, {w, 15 * n}, {quat, 20 * n}};
-  G6_CHECK(staged_download(s->device, s->stream, s->md.com, part, 4));
+  int cur = -1;
+  const bool here = hipGetDevice(&cur) == hipSuccess && cur == s->device;
+  auto send = [here](void *to, const void *from, size_t bytes, hipStream_t st) {
+    // (a launch goes to the current device; the engine serves any stream)
+    if (!here) return hipMemcpyAsync(to, from, bytes, hipMemcpyDeviceToHost, st);
+    const int len = (int)(bytes / sizeof(double));
+    k_stage_copy<<<std::min((len + 255) / 256, 256), 256, 0, st>>>((double *)to,
+                                                                   (const double *)from, len);
+    return hipGetLastError();
+  };
+  G6_CHECK(staged_download(s->device, s->stream, s->md.com, part, 4, send));
   return 0;
 }
 

@@ -2,9 +2,12 @@
 // pinned buffers, the copy of one piece to the host arrays beside the transfer
 // of the next.  A copy to pageable memory costs its own staging and
 // synchronization per array: the four state arrays took 82 us for 216
-// molecules, 105 for 4096 and 1530 for 65,536, and take 16, 79 and 990 in
-// pieces of 1 MiB (pieces of 512 KiB and 4 MiB: 102 and 96 us for 4096, 1300 and
-// 1030 for 65,536); the COMs alone 15, 13 and 86 before, 13, 14 and 76 now.
+// molecules, 106 for 4096 and 1500 for 65,536, and take 18, 76 and 1080 in
+// pieces of 1 MiB (pieces of 512 KiB and 4 MiB by the copy engine: 102 and 96 us
+// for 4096, 1300 and 1030 for 65,536, where 1 MiB took 79 and 990); the COMs
+// alone 15, 14 and 86 before, 13, 17 and 78 now.  Into memory that was not
+// touched before, as a fresh array's is, 28 MB take 5.8 ms where a plain copy
+// takes 6.3.
 // Arrays that the caller skips are not moved.
 //
 // An event may be recorded on the streams of its own device alone, so every
@@ -98,8 +101,10 @@ inline hipError_t plain_download(hipStream_t stream, const double *src, const Ho
   return hipStreamSynchronize(stream);
 }
 
+// send(buffer, src, bytes, stream) queues a transfer into a pinned buffer
+template <class Send>
 inline hipError_t staged_download(int dev, hipStream_t stream, const double *src,
-                                  const HostPart *part, int np) {
+                                  const HostPart *part, int np, Send &&send) {
   if (dev < 0 || dev >= kStageDevices || np > kStageParts)
     return plain_download(stream, src, part, np);
   // what the stream has queued ends before the buffers are taken, so that a
@@ -136,21 +141,20 @@ inline hipError_t staged_download(int dev, hipStream_t stream, const double *src
     hipError_t e = hipSuccess;
     // neighbouring arrays are one transfer
     size_t from = 0, into = 0, len = 0;
-    auto send = [&] {
+    auto flush = [&] {
       if (len > 0 && e == hipSuccess)
-        e = hipMemcpyAsync(g.buf[q & 1] + into, (const char *)src + from, len,
-                           hipMemcpyDeviceToHost, stream);
+        e = send(g.buf[q & 1] + into, (const char *)src + from, len, stream);
     };
     ranges(q * kStageBytes, piece_end(q), [&](size_t in, int k, size_t off, size_t bytes) {
       if (start[k] + off != from + len) {
-        send();
+        flush();
         from = start[k] + off;
         into = in;
         len = 0;
       }
       len += bytes;
     });
-    send();
+    flush();
     // (a single piece is waited for with the stream: an event costs 7 us)
     if (e == hipSuccess && pieces > 1) e = hipEventRecord(g.ev[q & 1], stream);
     return e;

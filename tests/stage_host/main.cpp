@@ -29,7 +29,10 @@ static bool download(int dev, hipStream_t s, size_t n, int mask) {
     out[k].assign(len[k], -1.0);
     part[k] = {mask >> k & 1 ? out[k].data() : nullptr, len[k]};
   }
-  if (staged_download(dev, s, src.data(), part, 4) != hipSuccess) return false;
+  auto send = [](void *to, const void *from, size_t bytes, hipStream_t st) {
+    return hipMemcpyAsync(to, from, bytes, hipMemcpyDeviceToHost, st);
+  };
+  if (staged_download(dev, s, src.data(), part, 4, send) != hipSuccess) return false;
   size_t at = 0;
   for (int k = 0; k < 4; k++)
     for (size_t q = 0; q < len[k]; q++, at++)
