@@ -530,12 +530,16 @@ int g6_time_force(g6_handle h, int nlaunch, double *ms);
  * waves per workgroup, info[4] = neighbourhood slots per tile (zeros for the
  * rows), info[5] = the capacity code that moved a tile system to the rows
  * (3 cell residents, 4 neighbourhood slots or row entries, 2 image shift, 6
- * a pair force beyond the fixed-point sums' range; 0 when none did).  FP32 fixed-box systems with at least 256 cells of edge
- * rc + skin take the tiles; G6_TILES=0 in the environment at g6_init keeps
+ * a pair force beyond the fixed-point sums' range; 0 when none did).  FP32
+ * fixed-box systems with at least 256 cells of edge rc + skin take the tiles; G6_TILES=0 in the environment at g6_init keeps
  * the rows and G6_TILE_MIN sets the cell threshold.  A system that a
  * capacity error moved to the rows tries the tiles again at the first
  * g6_step call 1000 steps later (G6_TILE_RETRY), the gap doubling after
- * each failed try; systems in a ladder or under the barostat keep the rows. */
+ * each failed try; systems in a ladder or under the barostat keep the rows.
+ * Two more lines, for tests: G6_SCAN_MAX (at g6_init) is the largest system
+ * whose rows are built from a scan of every molecule, G6_STEP_MAX (at g6_init
+ * and g6_ladder_create) the most molecules of a system or ladder that steps by
+ * one kernel; the results are the same bits on either side of both. */
 int g6_md_kernel(g6_handle h, int32_t *info);
 int g6_model_nsite(int model);
 
