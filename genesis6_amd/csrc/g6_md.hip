@@ -113,7 +113,7 @@ __device__ __forceinline__ void md_pre_body(const ModelTable &mt, const Geom &g,
   // the group of four molecules of lanes 4 l .. 4 l + 3
   const int grp = blk * 16 + (lane >> 2);
   const bool grp_ok = (lane & 3) == 0 && grp * 4 < n;
-  // the block's kinetic partials, stored by lane 63
+  // the block's kinetic partials
   const int nb64 = (n + 63) / 64;
   double *ek = b.stepek + blk;
   double et = 0.0;
@@ -195,16 +195,15 @@ __device__ __forceinline__ void md_pre_body(const ModelTable &mt, const Geom &g,
       const double v[3] = {ok ? S[3] : 0.0, ok ? S[4] : 0.0, ok ? S[5] : 0.0};
       const double vv = v[0] * v[0] + v[1] * v[1] + v[2] * v[2];
       et = quad_sum_d(vv);
-      const double es = wsum63(vv);
-      if (lane == 63) ek[0] = es;
-      int q = 4;
-#pragma unroll
-      for (int l = 0; l < 3; l++)
-#pragma unroll
-        for (int h = l; h < 3; h++, q++) {
-          const double e = wsum63(v[l] * v[h]);
-          if (lane == 63) ek[(size_t)q * nb64] = e;
-        }
+      const double u[8] = {vv,          v[0] * v[0], v[0] * v[1], v[0] * v[2],
+                           v[1] * v[1], v[1] * v[2], v[2] * v[2], 0.0};
+      double e0, e1;
+      wsum_eight(u, lane, e0, e1);
+      if (lane >> 2 == 1) {  // columns 0 and 4..6, then 7..9
+        const int c = lane & 3;
+        ek[(size_t)(c == 0 ? 0 : 3 + c) * nb64] = e0;
+        if (c < 3) ek[(size_t)(7 + c) * nb64] = e1;
+      }
     } else if (role == 1) {
       if (ok) {
         // rigid_collectforce's body-frame torque (RigidModule.F90:301-306)
@@ -229,7 +228,7 @@ __device__ __forceinline__ void md_pre_body(const ModelTable &mt, const Geom &g,
       }
 #pragma unroll
       for (int c = 0; c < 3; c++) {
-        const double w0 = ok ? S[c] : 0.0, e = quad_sum_d(w0 * w0), es = wsum63(w0 * w0);
+        const double w0 = ok ? S[c] : 0.0, e = quad_sum_d(w0 * w0), es = wsum63_quads(e);
         if (lane == 63) ek[(size_t)(1 + c) * nb64] = es;
         if ((lane & 3) == 0) s_ew[c][lane >> 2] = e;
       }

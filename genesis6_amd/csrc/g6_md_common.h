@@ -100,6 +100,35 @@ __device__ inline double wsum_six(const double (&v)[6], int lane) {
   return swap32_add(swap16_add(r));
 }
 
+// wsum63 of a value that is already the sum over its quad (in lane 63)
+__device__ inline double wsum63_quads(double v) {
+  v += dpp_d<0x141>(v);
+  v += dpp_d<0x140>(v);
+  v += dpp_dm<0x142, 0xA>(v);
+  v += dpp_dm<0x143, 0xC>(v);
+  return v;
+}
+
+// wsum63 of eight values, the same bits: lane l of quad 1 returns the sums of
+// v[l mod 4] and v[4 + l mod 4].  The first two steps halve the number of values
+// a lane carries, 74 instructions where eight wsum63 take 144.  (row_ror:4 pairs
+// the quads as wsum63 does in the odd quads alone.)
+__device__ inline void wsum_eight(const double (&v)[8], int lane, double &r0, double &r1) {
+  const bool b0 = lane & 1, b1 = lane & 2;
+  double p[4];
+#pragma unroll
+  for (int k = 0; k < 4; k++)
+    p[k] = (b0 ? v[2 * k + 1] : v[2 * k]) + dpp_d<0xB1>(b0 ? v[2 * k] : v[2 * k + 1]);
+  r0 = (b1 ? p[1] : p[0]) + dpp_d<0x4E>(b1 ? p[0] : p[1]);
+  r1 = (b1 ? p[3] : p[2]) + dpp_d<0x4E>(b1 ? p[2] : p[3]);
+  r0 += dpp_d<0x124>(r0);  // row_ror:4
+  r1 += dpp_d<0x124>(r1);
+  r0 += dpp_d<0x128>(r0);  // row_ror:8
+  r1 += dpp_d<0x128>(r1);
+  r0 = swap32_add(swap16_add(r0));
+  r1 = swap32_add(swap16_add(r1));
+}
+
 // Compensated sums (Knuth's TwoSum): the pair (s, c) holds s + c, the
 // rounding error of every addition carried in c.
 __device__ inline void two_sum_acc(double &s, double &c, double x) {
